@@ -16,6 +16,10 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # contract a*b + c within one source expression only: the arithmetic of a
+    # pass body is then the same in every kernel it is inlined into, so a
+    # field gives the same bits as an ensemble member whatever kernel runs it
+    "-ffp-contract=on",
     "-Wno-unused-value", "-Wno-unused-result",
     "-I" + os.path.join(ROOT, "include"),
 ]

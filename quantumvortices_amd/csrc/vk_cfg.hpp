@@ -68,6 +68,39 @@ template <> struct Cfg<2048> : CfgT<2048, 16, 4, 4, true> {};
 #endif
 template <> struct Cfg<4096> : CfgT<4096, VK4096_S, VK4096_TC, VK4096_TR, VK4096_SPLIT> {};
 
+// Shapes of a single field's passes.  From 2048^2 on they are Cfg<N>.  Up to
+// 1024^2 a pass is a few microseconds of exposed latency (one to four waves
+// per CU), so these shapes spread the field over more workgroups (one wave
+// of rows each, G columns of a panel each; one-wave workgroups need no
+// barrier), exchange real and imaginary parts together, keep the twiddles in
+// registers and load every operand before the first transform (LAT).  Layout
+// and radix plan are Cfg<N>'s, so the results are too, bit for bit.
+// us per RK4 step with Cfg<N>'s workgroups and table-read twiddles, then here:
+// 128^2 107, 66; 256^2 137, 91; 512^2 201, 121; 1024^2 258, 181.  Half as many
+// columns per workgroup: 69, 96, 127, 186; twice as many: 69, 93, 123, 194.
+template <int N> struct CfgS : Cfg<N> {};
+template <> struct CfgS<32> : CfgT<32, 8, 4, 16, false> { static constexpr int G = 4; static constexpr bool LAT = true; };
+template <> struct CfgS<64> : CfgT<64, 8, 8, 8, false> { static constexpr int G = 8; static constexpr bool LAT = true; };
+template <> struct CfgS<128> : CfgT<128, 8, 16, 4, false> { static constexpr int G = 4; static constexpr bool LAT = true; };
+template <> struct CfgS<256> : CfgT<256, 16, 16, 4, false> { static constexpr int G = 4; static constexpr bool LAT = true; };
+template <> struct CfgS<512> : CfgT<512, 16, 8, 2, false> { static constexpr int G = 2; static constexpr bool LAT = true; };
+template <> struct CfgS<1024> : CfgT<1024, 16, 4, 1, false> { static constexpr int G = 2; static constexpr bool LAT = true; };
+
+template <class C, class = void> struct is_lat { static constexpr bool value = false; };
+template <class C> struct is_lat<C, decltype((void)C::LAT)> { static constexpr bool value = C::LAT; };
+
+// twiddles of this thread: in registers for the LAT shapes, else the table
+template <class C> __device__ __forceinline__ auto twiddles(const cplx* __restrict__ tw, int t)
+{
+    if constexpr (is_lat<C>::value) {
+        TwReg<C::N, C::S> w;
+        w.load(tw, t);
+        return w;
+    } else {
+        return tw;
+    }
+}
+
 // Shapes of the ensemble sizes, all with 256-thread workgroups
 // (TC*T = TR*T = 256): variant 0 is Cfg<N>; variant 1 holds 8 points per
 // thread instead of 16 (radix-8 stages, twice the threads per transform,

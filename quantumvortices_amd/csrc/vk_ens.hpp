@@ -87,7 +87,7 @@ __device__ __forceinline__ void ens_tile_p1(const EnsReal* __restrict__ R, const
                                             const int* __restrict__ off, int b)
 {
     VK_ENS_SETUP_B(b)
-    VK_ENS_SWITCH(e.N, (p1_body<C, true>(lb, nb, e.Hpsi, e.Hrho, e.tw, e.g, 1, e.sc, e.Xs)))
+    VK_ENS_SWITCH(e.N, (p1_body<C>(lb, nb, e.Hpsi, e.Hrho, e.tw, e.g, 1, e.sc, e.Xs)))
 }
 
 __device__ __forceinline__ void ens_tile_p2(const EnsReal* __restrict__ R, const int* __restrict__ map,
@@ -102,8 +102,7 @@ __device__ __forceinline__ void ens_tile_p3(const EnsReal* __restrict__ R, const
 {
     VK_ENS_SETUP_B(b)
     const P3Part pa{};
-    VK_ENS_SWITCH(e.N, (p3_body<C, 0, true>(lb, nb, e.Hrho, e.Hrho, nullptr, e.HN, e.tw, e.g, 0, 1, e.gsc, e.sc,
-                                            1.0, 1.0, pa, e.Xs)))
+    VK_ENS_SWITCH(e.N, (p3_body<C, 0>(lb, nb, e.Hrho, e.Hrho, e.Xs, e.HN, e.tw, e.g, 1, e.gsc, e.sc, 1.0, pa)))
 }
 
 __device__ __forceinline__ void ens_tile_p4(const EnsReal* __restrict__ R, const int* __restrict__ map,
@@ -201,7 +200,7 @@ __device__ __forceinline__ void ens_loop_p1(const EnsReal* __restrict__ R, const
 #pragma unroll 1
     for (int b = ens_first(G.base[0]); b < G.nblk[0]; b += gridDim.x) {
         VK_ENS_SETUP_B(b)
-        p1_body<C, true>(lb, nb, e.Hpsi, e.Hrho, e.tw, e.g, 1, e.sc, e.Xs);
+        p1_body<C>(lb, nb, e.Hpsi, e.Hrho, e.tw, e.g, 1, e.sc, e.Xs);
         __syncthreads();
     }
 }
@@ -228,7 +227,7 @@ __device__ __forceinline__ void ens_loop_p3(const EnsReal* __restrict__ R, const
 #pragma unroll 1
     for (int b = ens_first(G.base[0]); b < G.nblk[0]; b += gridDim.x) {
         VK_ENS_SETUP_B(b)
-        p3_body<C, 0, true>(lb, nb, e.Hrho, e.Hrho, nullptr, e.HN, e.tw, e.g, 0, 1, e.gsc, e.sc, 1.0, 1.0, pa, e.Xs);
+        p3_body<C, 0>(lb, nb, e.Hrho, e.Hrho, e.Xs, e.HN, e.tw, e.g, 1, e.gsc, e.sc, 1.0, pa);
         __syncthreads();
     }
 }

@@ -192,17 +192,73 @@ template <int NS, int R> __device__ __forceinline__ int scatter_idx(int idxD, in
     else return lslot(idxD + r * NS);
 }
 
+// Table values a stage needs per butterfly: w^1..w^3 and w^4, w^8, ... (the
+// other factors are one product of two of them)
+constexpr int tw_per(int R) { return R == 2 ? 1 : 3 + (R / 4 - 1); }
+constexpr int tw_mult(int k) { return k < 3 ? k + 1 : 4 * (k - 2); }
+
+// Twiddles read from the table where they are used (few registers: several
+// workgroups per CU hide the loads).
+struct TwMem {
+    const cplx* tw;
+    template <int OFF, int K> __device__ __forceinline__ cplx get(int, int k, int base) const
+    {
+        return tw[tw_mult(k) * base];
+    }
+};
+
+// number of table values of all stages after the first
+template <int N, int S> constexpr int tw_count()
+{
+    int n = 0, ns = 1;
+    for (int st = 0; ns < N; ++st) {
+        const int R = radix_at(N, S, st);
+        if (ns > 1) n += (S / R) * tw_per(R);
+        ns *= R;
+    }
+    return n;
+}
+
+// Twiddles in registers, all loaded before the first transform (their
+// latency then overlaps the data's) and kept for the later ones: for passes
+// whose few waves leave registers idle and every load exposed.
+template <int N, int S> struct TwReg {
+    cplx w[tw_count<N, S>() > 0 ? tw_count<N, S>() : 1];
+    template <int OFF, int K> __device__ __forceinline__ cplx get(int a, int k, int) const { return w[OFF + a * K + k]; }
+
+    template <int ST, int NS, int OFF> __device__ __forceinline__ void load_stage(const cplx* __restrict__ tw, int t)
+    {
+        if constexpr (NS < N) {
+            constexpr int R = radix_at(N, S, ST), T = N / S;
+            if constexpr (NS > 1) {
+                constexpr int STEP = N / (NS * R), K = tw_per(R);
+#pragma unroll
+                for (int a = 0; a < S / R; ++a)
+#pragma unroll
+                    for (int k = 0; k < K; ++k) w[OFF + a * K + k] = tw[tw_mult(k) * (((t + T * a) % NS) * STEP)];
+                load_stage<ST + 1, NS * R, OFF + (S / R) * K>(tw, t);
+            } else {
+                load_stage<ST + 1, NS * R, OFF>(tw, t);
+            }
+        }
+    }
+    __device__ __forceinline__ void load(const cplx* __restrict__ tw, int t) { load_stage<0, 1, 0>(tw, t); }
+};
+
 // One Stockham stage, then recurse.  v: registers; re/im: this transform's
 // LDS arrays (split storage: real parts and imaginary parts exchanged in
 // turn through a single array of Lds<N>::words doubles when re == im).
-template <int N, int S, int ST, int NS, bool SPLIT>
+// OFF: index of the stage's first table value in TwReg.
+template <int N, int S, int ST, int NS, bool SPLIT, int OFF = 0>
 struct Stage {
     static constexpr int R = radix_at(N, S, ST);
     static constexpr int T = N / S;
     static constexpr bool LAST = (NS * R == N);
 
-    __device__ __forceinline__ static void run(cplx (&v)[S], double* re, double* im, int t,
-                                               const cplx* __restrict__ tw)
+    static constexpr int K = tw_per(R);
+
+    template <class W>
+    __device__ __forceinline__ static void run(cplx (&v)[S], double* re, double* im, int t, const W& tw)
     {
         static_assert(S % R == 0, "radix must divide S");
 #pragma unroll
@@ -217,17 +273,17 @@ struct Stage {
                 // (one product at most per factor)
                 constexpr int STEP = N / (NS * R);
                 const int base = jm * STEP;
-                const cplx w1 = tw[base];
+                const cplx w1 = tw.template get<OFF, K>(a, 0, base);
                 if constexpr (R == 2) {
                     x[1] = cmul(x[1], w1);
                 } else {
-                    const cplx w2 = tw[2 * base], w3 = tw[3 * base];
+                    const cplx w2 = tw.template get<OFF, K>(a, 1, base), w3 = tw.template get<OFF, K>(a, 2, base);
                     x[1] = cmul(x[1], w1);
                     x[2] = cmul(x[2], w2);
                     x[3] = cmul(x[3], w3);
 #pragma unroll
                     for (int a4 = 1; a4 < R / 4; ++a4) {
-                        const cplx wa = tw[4 * a4 * base];
+                        const cplx wa = tw.template get<OFF, K>(a, 2 + a4, base);
                         x[4 * a4] = cmul(x[4 * a4], wa);
                         x[4 * a4 + 1] = cmul(x[4 * a4 + 1], cmul(wa, w1));
                         x[4 * a4 + 2] = cmul(x[4 * a4 + 2], cmul(wa, w2));
@@ -280,14 +336,14 @@ struct Stage {
                 for (int s = 0; s < S; ++s) v[s] = mk(re[gather_idx<T>(t, s)], im[gather_idx<T>(t, s)]);
                 lds_barrier();
             }
-            Stage<N, S, ST + 1, NS * R, SPLIT>::run(v, re, im, t, tw);
+            Stage<N, S, ST + 1, NS * R, SPLIT, OFF + (NS > 1 ? (S / R) * K : 0)>::run(v, re, im, t, tw);
         }
     }
 };
 
 // Terminator for unused recursion depth (never instantiated at run time).
-template <int N, int S, int ST, bool SPLIT> struct Stage<N, S, ST, N, SPLIT> {
-    __device__ __forceinline__ static void run(cplx (&)[S], double*, double*, int, const cplx*) {}
+template <int N, int S, int ST, bool SPLIT, int OFF> struct Stage<N, S, ST, N, SPLIT, OFF> {
+    template <class W> __device__ __forceinline__ static void run(cplx (&)[S], double*, double*, int, const W&) {}
 };
 
 // Forward transform of the points held by this thread group.
@@ -302,7 +358,14 @@ __device__ __forceinline__ void fft_fwd(cplx (&v)[S], double* lds, int t, const 
     // transform's values live across the pointwise work in between.
     const cplx* twb = tw;
     asm volatile("" : "+s"(twb));
-    Stage<N, S, 0, 1, SPLIT>::run(v, lds, SPLIT ? lds : lds + Lds<N>::words, t, twb);
+    Stage<N, S, 0, 1, SPLIT>::run(v, lds, SPLIT ? lds : lds + Lds<N>::words, t, TwMem{twb});
+}
+
+// the same with twiddles in registers
+template <int N, int S, bool SPLIT>
+__device__ __forceinline__ void fft_fwd(cplx (&v)[S], double* lds, int t, const TwReg<N, S>& w)
+{
+    Stage<N, S, 0, 1, SPLIT>::run(v, lds, SPLIT ? lds : lds + Lds<N>::words, t, w);
 }
 
 }  // namespace vk

@@ -27,12 +27,6 @@
 using vk::cplx;
 using vk::Geo;
 
-// single-field handles of at least this size keep x-space psi rows between
-// P1 and P3 (one N^2 field more; P3 then runs two transforms instead of three)
-#ifndef VK_XPSI_MIN_N
-#define VK_XPSI_MIN_N 2048
-#endif
-
 namespace {
 thread_local std::string g_err;
 }
@@ -116,8 +110,7 @@ struct vk_gpe {
     cplx* tw = nullptr;
     // state and RK4/ARGLE work fields
     cplx *K0 = nullptr, *K1 = nullptr, *K2 = nullptr, *Hpsi = nullptr, *Hrho = nullptr, *HN = nullptr;
-    cplx* Xs = nullptr;   // x-space psi rows written by P1 and read by P3 (xpsi)
-    int xpsi = 0;
+    cplx* Xs = nullptr;   // x-space psi rows written by P1 and read by P3
     int dev = 0;        // device the handle was created on
     int ncu = 0;        // compute units of the device
     int p1pf = 0;       // RK4 P1 as the persistent prefetching kernel (4096^2)
@@ -158,9 +151,9 @@ struct vk_gpe {
     // ensemble's preparation and the member's next single-field access
     int ens_var = 0;
     Geo geo_v{};
-    // one-member ensemble table: N <= 1024 runs the same kernels as a
-    // batched ensemble member, so both give bit-identical results; svar is
-    // its transform shape (0 as a default ensemble member, 1: CfgE<N, 1>)
+    // transform shape of the single field: 0 (CfgS<N>; bit for bit a default
+    // ensemble member), 1 (CfgE<N, 1>, stepped as an ensemble of one with the
+    // member table below)
     int svar = 0;
     Geo geo_s{};
     vk::EnsReal* e1R = nullptr;
@@ -179,7 +172,7 @@ namespace {
 
 size_t f2(const vk_gpe* h) { return (size_t)h->N * h->N; }
 
-template <int N> using CfgN = vk::Cfg<N>;
+template <int N> using CfgN = vk::CfgS<N>;
 // The same panel layout with one row per row-pass workgroup (256 threads)
 // instead of TR rows: more, smaller workgroups per CU at the cost of half
 // as long row pieces of the panels.
@@ -253,25 +246,8 @@ void row_launch(vk_gpe* h, int kind, Kern k, A... args)
     row_launch_x<C>(h, kind, 0, k, args...);
 }
 
-// P3 keeps S doubles per thread in LDS besides the transform regions (in
-// registers instead with xpsi and no real-space particles), then the
-// particle positions and a one-bit-per-particle hit mask
-template <class C> size_t p3_extra(const vk_gpe* h)
-{
-    const bool park = !h->xpsi || (h->have_part && h->p.np > 0 && h->rs_part && !vk::kP3FregPart);
-    const size_t np = (size_t)std::max(h->p.np, 1);
-    return (park ? (size_t)C::S * C::ROWT * sizeof(double) : 0) + 2 * np * sizeof(double);
-}
-
-template <class C, class Kern, class... A>
-void col_launch(vk_gpe* h, int kind, int nblocks, Kern k, A... args)
-{
-    const size_t lds = (size_t)C::TC * C::COLRS * sizeof(double);
-    set_lds(k, lds);
-    ev_begin(h);
-    hipLaunchKernelGGL(k, dim3(nblocks), dim3(C::COLT), lds, h->stream, args...);
-    ev_end(h, kind);
-}
+// P3 stages the particle positions after its transform regions
+size_t p3_extra(const vk_gpe* h) { return 2 * (size_t)std::max(h->p.np, 1) * sizeof(double); }
 
 // P2 columns per workgroup.  P2 covers only the kx >= 0 panels.  At
 // 4096^2 one column per workgroup (1366 workgroups) is the fastest: with
@@ -281,14 +257,23 @@ void col_launch(vk_gpe* h, int kind, int nblocks, Kern k, A... args)
 #ifndef VK_P2_COLS_4096
 #define VK_P2_COLS_4096 1
 #endif
-template <class C> constexpr int p2_cols() { return C::N == 4096 ? VK_P2_COLS_4096 : C::TC; }
+// The LAT shapes have their own.
+template <class C> constexpr int p2_cols()
+{
+    if constexpr (vk::is_lat<C>::value) return C::G;
+    else return C::N == 4096 ? VK_P2_COLS_4096 : C::TC;
+}
 // P4 columns per workgroup at 4096^2 (0: whole panels).  Two of the four
 // columns of a panel in a 512-thread workgroup: 0.170 ms against 0.189 for
 // whole panels (1024 threads, one workgroup per CU) and 0.193 for one.
 #ifndef VK_P4_COLS_4096
 #define VK_P4_COLS_4096 2
 #endif
-template <class C> constexpr int p4_cols() { return C::N == 4096 && VK_P4_COLS_4096 > 0 ? VK_P4_COLS_4096 : C::TC; }
+template <class C> constexpr int p4_cols()
+{
+    if constexpr (vk::is_lat<C>::value) return C::G;
+    else return C::N == 4096 && VK_P4_COLS_4096 > 0 ? VK_P4_COLS_4096 : C::TC;
+}
 
 // column pass with G columns per workgroup over npan panels
 template <class C, int G, class Kern, class... A>
@@ -325,7 +310,7 @@ void p2_launch(vk_gpe* h, cplx* Hrho, cplx* HV, const cplx* KV, cplx* Krho, cons
 // count whose row blocks divide evenly over the XCDs)
 int p1_prefetch_fits(const vk_gpe* h)
 {
-    if (!VK_P1_PREFETCH || h->N != 4096 || !h->xpsi) return 0;
+    if (!VK_P1_PREFETCH || h->N != 4096) return 0;
     using C = CfgN<4096>;
     static_assert(vk::p1p_lds<C>() <= 160 * 1024, "prefetch buffer exceeds LDS");
     const int g8 = h->ncu / 8, r8 = (C::N / C::TR) / 8;
@@ -589,13 +574,12 @@ void join_particles(vk_gpe* h)
 // ---- RK4 / ARGLE -----------------------------------------------------------------
 
 int ens1_step(vk_gpe* h);
-int make_single_table(vk_gpe* h);
-vk::EnsReal ens_entry(const vk_gpe* h);
+vk::EnsReal single_entry(const vk_gpe* h);
 int prep_rk4(vk_gpe* h);
 
 int rk4_step(vk_gpe* h)
 {
-    if (h->e1R && !(h->have_part && h->p.np > 0)) return ens1_step(h);
+    if (h->svar) return ens1_step(h);
     return dispatch(h->N, [&](auto n) {
         using C = CfgN<decltype(n)::value>;
         const double sc = scale_of(h);
@@ -610,36 +594,31 @@ int rk4_step(vk_gpe* h)
         a.omega = h->p.omega;
         for (int stage = 1; stage <= 4; ++stage) {
             if (parts && !rs) particle_kv(h, Kp);
+            constexpr bool VAR = C::N >= 2048;   // sizes with row-pass variants
+            using C1 = std::conditional_t<VAR, CfgTR1<C>, C>;
             if (h->p1pf)
                 p1p_launch<C>(h, sc);
-            else if (h->xpsi && h->tr1_p1)
-                row_launch<CfgTR1<C>>(h, PK_P1, vk::k_p1x<CfgTR1<C>>, (const cplx*)h->Hpsi, h->Hrho, (const cplx*)h->tw,
-                                      h->geo, 1, sc, h->Xs);
-            else if (h->xpsi)
+            else if (VAR && h->tr1_p1)
+                row_launch<C1>(h, PK_P1, vk::k_p1x<C1>, (const cplx*)h->Hpsi, h->Hrho, (const cplx*)h->tw, h->geo, 1,
+                               sc, h->Xs);
+            else
                 row_launch<C>(h, PK_P1, vk::k_p1x<C>, (const cplx*)h->Hpsi, h->Hrho, (const cplx*)h->tw, h->geo, 1, sc,
                               h->Xs);
-            else
-                row_launch<C>(h, PK_P1, vk::k_p1<C>, (const cplx*)h->Hpsi, h->Hrho, (const cplx*)h->tw, h->geo, 1, sc);
             p2_launch<C>(h, h->Hrho, h->HV, (const cplx*)h->KV, h->Krho,
                           (const cplx*)h->tw, h->geo, (parts && !rs) ? 3 : 0);
             if (parts && !rs) particle_forces(h, h->Krho, Kp, 1, stage);
             if (rs) join_particles(h);   // positions from the previous stage
-            if (h->xpsi && h->tr1_p3) {
-                using C1 = CfgTR1<C>;
+            if (VAR && h->tr1_p3) {
                 auto k3 = !parts ? vk::k_p3x<C1, 0> : (rs ? vk::k_p3x<C1, 6> : vk::k_p3x<C1, 1>);
-                row_launch_x<C1>(h, PK_P3, p3_extra<C1>(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV,
+                row_launch_x<C1>(h, PK_P3, p3_extra(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV,
                                  (const cplx*)h->Xs, h->HN, (const cplx*)h->tw, h->geo, 1, h->p.g * sc, sc, 1.0, pa);
-            } else if (h->xpsi) {
-                auto k3 = !parts ? vk::k_p3x<C, 0> : (rs ? vk::k_p3x<C, 6> : vk::k_p3x<C, 1>);
-                row_launch_x<C>(h, PK_P3, p3_extra<C>(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV,
-                                (const cplx*)h->Xs, h->HN, (const cplx*)h->tw, h->geo, 1, h->p.g * sc, sc, 1.0, pa);
             } else {
-                auto k3 = !parts ? vk::k_p3<C, 0> : (rs ? vk::k_p3<C, 6> : vk::k_p3<C, 1>);
-                row_launch_x<C>(h, PK_P3, p3_extra<C>(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV, (const cplx*)h->Hpsi,
-                              h->HN, (const cplx*)h->tw, h->geo, 1, 1, h->p.g * sc, sc, sc, 1.0, pa);
+                auto k3 = !parts ? vk::k_p3x<C, 0> : (rs ? vk::k_p3x<C, 6> : vk::k_p3x<C, 1>);
+                row_launch_x<C>(h, PK_P3, p3_extra(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV,
+                                (const cplx*)h->Xs, h->HN, (const cplx*)h->tw, h->geo, 1, h->p.g * sc, sc, 1.0, pa);
             }
             if (rs) {
-                if (h->xpsi && h->tr1_p3) particle_step_rs(h, C::N, (CfgTR1<C>::ROWT + 63) / 64, stage);
+                if (VAR && h->tr1_p3) particle_step_rs(h, C::N, (C1::ROWT + 63) / 64, stage);
                 else particle_step_rs(h, C::N / C::TR, (C::ROWT + 63) / 64, stage);
             }
             a.stage = stage;
@@ -703,33 +682,21 @@ int argle_step(vk_gpe* h, int want_res, const double* noise = nullptr)
         if (adv)   // i ky kpsi -> Hdy (all columns)
             colg_launch<C, GC>(h, PK_OTHER, h->NP, vk::k_col_inv<C, GC>, (const cplx*)h->K0, h->Hdy,
                                (const cplx*)h->tw, h->geo, 0, 2);
-        if (h->xpsi)
-            row_launch<C>(h, PK_P1, vk::k_p1x<C>, (const cplx*)h->Hpsi, h->Hrho, (const cplx*)h->tw, h->geo, 0, sc,
-                          h->Xs);
-        else
-            row_launch<C>(h, PK_P1, vk::k_p1<C>, (const cplx*)h->Hpsi, h->Hrho, (const cplx*)h->tw, h->geo, 0, sc);
+        row_launch<C>(h, PK_P1, vk::k_p1x<C>, (const cplx*)h->Hpsi, h->Hrho, (const cplx*)h->tw, h->geo, 0, sc, h->Xs);
         p2_launch<C>(h, h->Hrho, h->HV, (const cplx*)h->KV, h->Krho,
                       (const cplx*)h->tw, h->geo, (parts && !rs) ? 1 : 0);
         if (adv) {
             const vk::AdvArgs aa{h->adv_tg, h->adv_vx, h->adv_vy, 0.25 / h->p.alpha, sc,
                                  h->adv_field ? (const double*)h->Ux : nullptr,
                                  h->adv_field ? (const double*)h->Uy : nullptr};
-            const cplx* xs = h->xpsi ? (const cplx*)h->Xs : nullptr;
-            auto launch = [&](auto k3) {
-                row_launch_x<C>(h, PK_P3, p3_extra<C>(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV,
-                                (const cplx*)h->Hpsi, xs, (const cplx*)h->Hdy, h->HN, (const cplx*)h->tw, h->geo,
-                                -h->p.g * sc, -sc, sc, -1.0, pa, aa);
-            };
-            if (h->xpsi) launch(!parts ? vk::k_p3a<C, 0, true> : (rs ? vk::k_p3a<C, 2, true> : vk::k_p3a<C, 1, true>));
-            else launch(!parts ? vk::k_p3a<C, 0, false> : (rs ? vk::k_p3a<C, 2, false> : vk::k_p3a<C, 1, false>));
-        } else if (h->xpsi) {
-            auto k3 = !parts ? vk::k_p3x<C, 0> : (rs ? vk::k_p3x<C, 2> : vk::k_p3x<C, 1>);
-            row_launch_x<C>(h, PK_P3, p3_extra<C>(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV, (const cplx*)h->Xs,
-                            h->HN, (const cplx*)h->tw, h->geo, 0, -h->p.g * sc, -sc, -1.0, pa);
+            row_launch_x<C>(h, PK_P3, p3_extra(h),
+                            !parts ? vk::k_p3a<C, 0> : (rs ? vk::k_p3a<C, 2> : vk::k_p3a<C, 1>), (const cplx*)h->Hrho,
+                            (const cplx*)h->HV, (const cplx*)h->Hpsi, (const cplx*)h->Xs, (const cplx*)h->Hdy, h->HN,
+                            (const cplx*)h->tw, h->geo, -h->p.g * sc, -sc, -1.0, pa, aa);
         } else {
-            auto k3 = !parts ? vk::k_p3<C, 0> : (rs ? vk::k_p3<C, 2> : vk::k_p3<C, 1>);
-            row_launch_x<C>(h, PK_P3, p3_extra<C>(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV, (const cplx*)h->Hpsi, h->HN,
-                          (const cplx*)h->tw, h->geo, 0, 0, -h->p.g * sc, -sc, sc, -1.0, pa);
+            auto k3 = !parts ? vk::k_p3x<C, 0> : (rs ? vk::k_p3x<C, 2> : vk::k_p3x<C, 1>);
+            row_launch_x<C>(h, PK_P3, p3_extra(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV, (const cplx*)h->Xs,
+                            h->HN, (const cplx*)h->tw, h->geo, 0, -h->p.g * sc, -sc, -1.0, pa);
         }
         vk::ArgleArgs a{h->p.alpha, h->p.omega, h->p.dt, want_res};
         if (h->sgle) {
@@ -958,7 +925,6 @@ int vk_gpe_create(vk_gpe** out, const vk_gpe_params* p)
         if (hipMalloc(b, fb) != hipSuccess || hipMemset(*b, 0, fb) != hipSuccess)
             return cleanup(fail(VK_ERR_HIP, "hipMalloc failed (fields)"));
     }
-    h->xpsi = N >= VK_XPSI_MIN_N;
     {
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -977,10 +943,7 @@ int vk_gpe_create(vk_gpe** out, const vk_gpe_params* p)
         h->tr1_p1 = t1 ? t1[0] == '1' : (N == 4096 || N == 2048);
         h->tr1_p3 = t3 ? t3[0] == '1' : (N == 4096 || N == 2048);
     }
-    // psi rows: the single-field RK4/ARGLE path at N >= VK_XPSI_MIN_N and the
-    // ensemble kernels (which also step single fields of N <= 1024)
-    const bool rows = h->xpsi || (N >= 128 && N <= 1024);
-    if (rows && hipMalloc(&h->Xs, fb) != hipSuccess) return cleanup(fail(VK_ERR_HIP, "hipMalloc failed (psi rows)"));
+    if (hipMalloc(&h->Xs, fb) != hipSuccess) return cleanup(fail(VK_ERR_HIP, "hipMalloc failed (psi rows)"));
     if (hipMalloc(&h->tw, sizeof(cplx) * N) != hipSuccess) return cleanup(fail(VK_ERR_HIP, "hipMalloc tw"));
     // twiddles w_k = exp(-2 pi i k/N): long-double sin/cos on the first
     // octant, exact quadrant/octant symmetries elsewhere
@@ -1037,10 +1000,6 @@ int vk_gpe_create(vk_gpe** out, const vk_gpe_params* p)
         h->HV = h->Hrho;
         h->KV = h->K1;
         h->Krho = h->K1;
-    }
-    if (p->np == 0) {
-        int rc = make_single_table(h);
-        if (rc) return cleanup(rc);
     }
     if (hipDeviceSynchronize() != hipSuccess) return cleanup(fail(VK_ERR_HIP, "create: device sync"));
     *out = h;
@@ -1377,7 +1336,7 @@ static int sgle_sync_omega(vk_gpe* h)
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipMemcpy(&h->p.omega, h->omega_dev, sizeof(double), hipMemcpyDeviceToHost));
     if (h->e1R) {
-        const vk::EnsReal x = ens_entry(h);
+        const vk::EnsReal x = single_entry(h);
         HIPCHK(hipMemcpy(h->e1R, &x, sizeof(x), hipMemcpyHostToDevice));
     }
     return 0;
@@ -1427,7 +1386,7 @@ int vk_gpe_set_dt(vk_gpe* h, double dt)
     HIPCHK(hipStreamSynchronize(h->stream));
     h->p.dt = dt;
     if (h->e1R) {
-        const vk::EnsReal x = ens_entry(h);
+        const vk::EnsReal x = single_entry(h);
         HIPCHK(hipMemcpy(h->e1R, &x, sizeof(x), hipMemcpyHostToDevice));
     }
     return 0;
@@ -1595,7 +1554,7 @@ int vk_gpe_pass_times(vk_gpe* h, int nsteps, double* ms_out, int nkinds)
 int vk_gpe_set_row_variants(vk_gpe* h, int p1, int p3)
 {
     if (!h || p1 < 0 || p1 > 2 || p3 < 0 || p3 > 1) return fail(VK_ERR_ARG, "set_row_variants: bad arguments");
-    if (!h->xpsi) return fail(VK_ERR_UNSUPPORTED, "set_row_variants: the row-pass variants exist for the psi-row path only");
+    if (h->N < 2048) return fail(VK_ERR_UNSUPPORTED, "set_row_variants: the row-pass variants exist for the psi-row path only");
     if (p1 == 2 && !p1_prefetch_fits(h))
         return fail(VK_ERR_UNSUPPORTED, "set_row_variants: the prefetching P1 does not fit this size or device");
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -1616,7 +1575,7 @@ int vk_gpe_get_row_variants(vk_gpe* h, int* p1, int* p3)
 int vk_gpe_autotune_rows(vk_gpe* h, int nsteps, int* choice, double* ms_out)
 {
     if (!h || nsteps <= 0) return fail(VK_ERR_ARG, "autotune_rows: bad arguments");
-    if (!h->xpsi) return fail(VK_ERR_UNSUPPORTED, "autotune_rows: the row-pass variants exist for the psi-row path only");
+    if (h->N < 2048) return fail(VK_ERR_UNSUPPORTED, "autotune_rows: the row-pass variants exist for the psi-row path only");
     int rc = ensure_rk4(h);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -1700,13 +1659,10 @@ double vk_gpe_pass_bytes(vk_gpe* h, int kind)
         for (int ky = -h->N / 2; ky < h->N / 2; ++ky)
             if (!masked_host(kx, ky, h->N)) ++disk;
     const double D = 16.0 * (double)disk;
-    // the RK4 step of a single field of N <= 1024 without particles runs the
-    // ensemble kernels, which pass psi rows from P1 to P3 as well
-    const bool rows = h->xpsi || (h->e1R && !(h->have_part && h->p.np > 0));
     switch (kind) {
-    case PK_P1: return F * (fr + fp + (rows ? 1.0 : 0.0));   // + psi rows written for P3
+    case PK_P1: return F * (fr + fp + 1.0);   // + psi rows written for P3
     case PK_P2: return F * 2.0 * fp;
-    case PK_P3: return F * (fp + (rows ? 1.0 : fr) + fr);    // psi rows instead of Hpsi
+    case PK_P3: return F * (fp + 1.0 + fr);    // psi rows
     // K accesses per mode, stages 1-4: K0 read + K2 write; K0, K2 read + K1,
     // K2 write; K0, K2 read + K2 write (str2 is not read in stage 3); K0, K1,
     // K2 read + K0 write
@@ -1819,17 +1775,6 @@ int build_maps(const std::vector<vk_gpe*>& hs, const std::vector<int>& ids, int*
     return 0;
 }
 
-// set the LDS limit of the single-field pass kernels of size C before any
-// graph capture
-template <class C> void preconfig_passes()
-{
-    set_lds(vk::k_p1<C>, (size_t)C::TR * C::ROWRS * sizeof(double));
-    set_lds(vk::k_p2<C>, (size_t)C::TC * C::COLRS * sizeof(double));
-    set_lds(vk::k_p3<C, 0>, (size_t)C::TR * C::ROWRS * sizeof(double) + (size_t)C::S * C::ROWT * sizeof(double) + 16);
-    for (auto k : {vk::k_p4<C, 1>, vk::k_p4<C, 2>, vk::k_p4<C, 3>, vk::k_p4<C, 4>})
-        set_lds(k, (size_t)C::TC * C::COLRS * sizeof(double));
-}
-
 vk::EnsReal ens_entry(const vk_gpe* h)
 {
     vk::EnsReal x{};
@@ -1847,16 +1792,24 @@ vk::EnsReal ens_entry(const vk_gpe* h)
     return x;
 }
 
+// the same in the single-field shape svar
+vk::EnsReal single_entry(const vk_gpe* h)
+{
+    vk::EnsReal x = ens_entry(h);
+    x.var = h->svar;
+    x.g = h->svar ? h->geo_s : h->geo;
+    return x;
+}
+
 int make_single_table(vk_gpe* h)
 {
-    if (h->N < 128 || h->N > 1024) return 0;
     // the table and block maps of the single-field shape svar (build_maps
     // and ens_entry read the member shape fields, borrowed here)
     const int keep_var = h->ens_var;
     const Geo keep_geo = h->geo_v;
     h->ens_var = h->svar;
     h->geo_v = h->geo_s;
-    const vk::EnsReal x = ens_entry(h);
+    const vk::EnsReal x = single_entry(h);
     for (int k = 0; k < 3; ++k) {
         if (h->e1map[k]) { hipFree(h->e1map[k]); h->e1map[k] = nullptr; }
         if (h->e1off[k]) { hipFree(h->e1off[k]); h->e1off[k] = nullptr; }
@@ -1885,8 +1838,7 @@ int make_single_table(vk_gpe* h)
 // (hstate 2).
 int prep_rk4(vk_gpe* h)
 {
-    const bool e1 = h->e1R && !(h->have_part && h->p.np > 0);
-    if (!(e1 && h->svar)) return ensure_rk4(h);
+    if (!h->svar) return ensure_rk4(h);
     if (h->hstate == 3) return 0;
     int rc = ensure_rk4(h);
     if (rc) return rc;
@@ -2144,7 +2096,6 @@ int vk_ens_create(vk_ens** out, int nreal, const vk_gpe_params* params)
     set_lds(vk::k_ens_p3, e->lds[2]);
     set_lds(vk::k_ens_p4, e->lds[3]);
     for (auto k : {vk::k_ens_p4s<1>, vk::k_ens_p4s<2>, vk::k_ens_p4s<3>, vk::k_ens_p4s<4>}) set_lds(k, e->lds[3]);
-    for (int N : e->sizes) dispatch(N, [&](auto n) { preconfig_passes<CfgN<decltype(n)::value>>(); return 0; });
     // the persistent step: as many workgroups as the device holds at once
     {
         e->plds = *std::max_element(e->lds, e->lds + 4);
@@ -2439,7 +2390,7 @@ int vk_ens_diagnostics_all(vk_ens* e, double* scal, double* spec)
         char* htab = static_cast<char*>(e->htab) + toff;
         toff += (ens_diag_tab_bytes(hs.size()) + 255) / 256 * 256;
         int rc = dispatch(kv.first.first, [&](auto nn) {
-            using C = CfgN<decltype(nn)::value>;
+            using C = vk::Cfg<decltype(nn)::value>;
             if (kv.first.second == 0) {
                 // Hpsi stale (a member in its second shape): IFFT_y(K0) on
                 // all panels in the single-field layout, as ensure_any does
@@ -2663,7 +2614,7 @@ extern "C" {
 int vk_gpe_set_shape(vk_gpe* h, int var)
 {
     if (!h || (var != 0 && var != 1)) return fail(VK_ERR_ARG, "set_shape: bad arguments");
-    if (!h->e1R || !vk::has_variant(h->N, var) || h->p.np > 0)
+    if (h->np_cap > 0 || h->N < 128 || h->N > 1024 || !vk::has_variant(h->N, var))
         return fail(VK_ERR_UNSUPPORTED, "set_shape: shapes exist for N in {256, 512, 1024} without particles");
     HIPCHK(hipStreamSynchronize(h->stream));
     if (var == h->svar) return 0;

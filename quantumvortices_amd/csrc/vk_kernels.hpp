@@ -24,21 +24,15 @@
 #define VK_P4_WAVES 4
 #endif
 #if VK_P4_WAVES > 0
-#define VK_P4OCC __attribute__((amdgpu_waves_per_eu(VK_P4_WAVES)))
+#define VK_P4OCC(C) __attribute__((amdgpu_waves_per_eu(is_lat<C>::value ? 1 : VK_P4_WAVES)))
 #else
-#define VK_P4OCC VK_COCC
+#define VK_P4OCC(C) VK_COCC
 #endif
 #ifdef VK_P1_WAVES
 #define VK_P1OCC __attribute__((amdgpu_waves_per_eu(VK_P1_WAVES)))
 #else
 #define VK_P1OCC VK_OCC
 #endif
-// P3 with real-space particles keeps its factor f in registers too, not in
-// 64 KB of LDS slots (P3 0.186 -> 0.184 ms; results bitwise the same)
-#ifndef VK_P3_FREG_PART
-#define VK_P3_FREG_PART 1
-#endif
-namespace vk { constexpr bool kP3FregPart = VK_P3_FREG_PART != 0; }
 // P3 on the psi-row path without particles (PM = 0) at 4 waves per SIMD
 // (<= 128 VGPRs): +0.8% pure-GPE steps/s with two rows per workgroup.  With
 // particles the compiler's choice (231 VGPRs with one row per workgroup,
@@ -51,9 +45,9 @@ namespace vk { constexpr bool kP3FregPart = VK_P3_FREG_PART != 0; }
 #ifndef VK_P3_PART_WAVES
 #define VK_P3_PART_WAVES 1
 #endif
-#define VK_P3OCC(PM) __attribute__((amdgpu_waves_per_eu((PM) == 0 ? VK_P3_WAVES : VK_P3_PART_WAVES)))
+#define VK_P3OCC(C, PM) __attribute__((amdgpu_waves_per_eu(!is_lat<C>::value && (PM) == 0 ? VK_P3_WAVES : VK_P3_PART_WAVES)))
 #else
-#define VK_P3OCC(PM) VK_OCC
+#define VK_P3OCC(C, PM) VK_OCC
 #endif
 
 namespace vk {
@@ -134,6 +128,7 @@ __device__ __forceinline__ void row_fwd_body(int blk_, int nblk_, const cplx* __
                                              const cplx* __restrict__ tw, Geo g, int pstore, int op)
 {
     VK_ROW_SETUP(C)
+    const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
     const cplx* xr = X + (size_t)y * N;
 #pragma unroll
@@ -141,7 +136,7 @@ __device__ __forceinline__ void row_fwd_body(int blk_, int nblk_, const cplx* __
         cplx a = xr[t + T * s];
         v[s] = op == 1 ? mk(a.x * a.x + a.y * a.y, 0.0) : a;
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int pp = VK_PANEL(s);
@@ -165,10 +160,11 @@ __device__ __forceinline__ void col_fwd_body(int b, const cplx* __restrict__ H, 
                                              const cplx* __restrict__ tw, Geo g, int pmode, int op)
 {
     VK_COL_SETUP_G(C, G, b, panel_of_block(pb_, C::NP, g, pmode), VK_NPAN(C, g, pmode))
+    const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) v[s] = H[hoff<C>(p, t + T * s, c)];
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
     const int kxs = ksg(kx, N);
     cplx* kr = K + (size_t)kx * N;
 #pragma unroll
@@ -194,6 +190,7 @@ __device__ __forceinline__ void col_inv_body(int b, const cplx* __restrict__ K, 
                                              const cplx* __restrict__ tw, Geo g, int pmode, int op)
 {
     VK_COL_SETUP_G(C, G, b, panel_of_block(pb_, C::NP, g, pmode), VK_NPAN(C, g, pmode))
+    const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
     const int kxs = ksg(kx, N);
     const cplx* kr = K + (size_t)kx * N;
@@ -206,7 +203,7 @@ __device__ __forceinline__ void col_inv_body(int b, const cplx* __restrict__ K, 
         if (op == 2) a = mk(-(double)kys * a.y, (double)kys * a.x);
         v[s] = conjc(a);
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) H[hoff<C>(p, t + T * s, c)] = conjc(v[s]);
 }
@@ -226,6 +223,7 @@ __device__ __forceinline__ void row_inv_body(int blk_, int nblk_, const cplx* __
                                              const cplx* __restrict__ tw, Geo g, int pload, int op, double scale)
 {
     VK_ROW_SETUP(C)
+    const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
     const int Kp = TC * g.Pp;
     const brsrc rH = mkbuf(H, N);
@@ -253,7 +251,7 @@ __device__ __forceinline__ void row_inv_body(int blk_, int nblk_, const cplx* __
         }
         v[s] = conjc(a);
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
     cplx* xr = X + (size_t)y * N;
 #pragma unroll
     for (int s = 0; s < S; ++s) xr[t + T * s] = rmul(scale, conjc(v[s]));
@@ -282,24 +280,22 @@ __global__ void k_dealias(cplx* __restrict__ K, int N)
 // ----------------------------------------------------------------------------
 
 // P1 after its loads: v holds the conjugated Hpsi row points of this thread
-template <class C, bool XPSI>
+template <class C, class W>
 __device__ __forceinline__ void p1_core(cplx (&v)[C::S], double* lg, int t, int y, int pidx0, int c,
-                                        cplx* __restrict__ Hrho, const cplx* __restrict__ tw, const Geo& g,
+                                        cplx* __restrict__ Hrho, const W& w_, const Geo& g,
                                         double scale, cplx* __restrict__ Xpsi)
 {
     constexpr int N = C::N, S = C::S, T = C::T, TC = C::TC;
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
-    if constexpr (XPSI) {
-        cplx* xr = Xpsi + (size_t)y * N;
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    cplx* xr = Xpsi + (size_t)y * N;
 #pragma unroll
-        for (int s = 0; s < S; ++s) xr[t + T * s] = rmul(scale, conjc(v[s]));
-    }
+    for (int s = 0; s < S; ++s) xr[t + T * s] = rmul(scale, conjc(v[s]));
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const double a = scale * v[s].x, b = scale * v[s].y;   // conj does not change |.|
         v[s] = mk(a * a + b * b, 0.0);
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int pp = VK_PANEL(s);
@@ -308,13 +304,13 @@ __device__ __forceinline__ void p1_core(cplx (&v)[C::S], double* lg, int t, int 
 }
 
 // P1 (row): psi row from Hpsi (inverse along x, times 1/N^2), rho = |psi|^2,
-// forward along x, keep kx >= 0 retained panels (rho is real).  XPSI: also
-// store the psi row in x-space (Xpsi[y*N + x]) for P3, which then needs no
-// transform of its own for psi.
-template <class C, bool XPSI = false>
+// forward along x, keep kx >= 0 retained panels (rho is real).  The psi row
+// is stored in x-space (Xpsi[y*N + x]) for P3, which then needs no transform
+// of its own for psi.
+template <class C>
 __device__ __forceinline__ void p1_body(int blk_, int nblk_, const cplx* __restrict__ Hpsi, cplx* __restrict__ Hrho,
                                                 const cplx* __restrict__ tw, Geo g, int psi_pmode,
-                                                double scale, cplx* __restrict__ Xpsi = nullptr)
+                                                double scale, cplx* __restrict__ Xpsi)
 {
     VK_ROW_SETUP(C)
     cplx v[S];
@@ -324,17 +320,10 @@ __device__ __forceinline__ void p1_body(int blk_, int nblk_, const cplx* __restr
         const int pp = VK_PANEL(s);
         v[s] = bld(rH, boff(hoff<C>(pp, y, c), panel_stored(pp, NP, g, psi_pmode)));
     }
+    const auto w_ = twiddles<C>(tw, t);
 #pragma unroll
     for (int s = 0; s < S; ++s) v[s] = panel_stored(VK_PANEL(s), NP, g, psi_pmode) ? conjc(v[s]) : czero();
-    p1_core<C, XPSI>(v, lg, t, y, pidx0, c, Hrho, tw, g, scale, Xpsi);
-}
-
-template <class C>
-__global__ void __launch_bounds__(C::ROWT) VK_OCC k_p1(const cplx* __restrict__ Hpsi, cplx* __restrict__ Hrho,
-                                                const cplx* __restrict__ tw, Geo g, int psi_pmode,
-                                                double scale)
-{
-    p1_body<C>(blockIdx.x, gridDim.x, Hpsi, Hrho, tw, g, psi_pmode, scale);
+    p1_core<C>(v, lg, t, y, pidx0, c, Hrho, w_, g, scale, Xpsi);
 }
 
 template <class C>
@@ -342,7 +331,7 @@ __global__ void __launch_bounds__(C::ROWT) VK_P1OCC k_p1x(const cplx* __restrict
                                                  const cplx* __restrict__ tw, Geo g, int psi_pmode,
                                                  double scale, cplx* __restrict__ Xpsi)
 {
-    p1_body<C, true>(blockIdx.x, gridDim.x, Hpsi, Hrho, tw, g, psi_pmode, scale, Xpsi);
+    p1_body<C>(blockIdx.x, gridDim.x, Hpsi, Hrho, tw, g, psi_pmode, scale, Xpsi);
 }
 
 // Retained-panel geometry of a size, at compile time (as the host computes
@@ -453,7 +442,7 @@ __global__ void __launch_bounds__(C::ROWT) k_p1xp(const cplx* __restrict__ Hpsi,
         // all reads are done before the next copies overwrite the slots
         __syncthreads();
         if (k + 1 < K) prefetch(xcd * R8 + j + (k + 1) * G8);
-        p1_core<C, true>(v, lg, t, y, pidx0, c, Hrho, tw, g, scale, Xpsi);
+        p1_core<C>(v, lg, t, y, pidx0, c, Hrho, tw, g, scale, Xpsi);
     }
 }
 
@@ -469,10 +458,11 @@ __device__ __forceinline__ void p2_body(int blk_, int nblk_, cplx* __restrict__ 
 {
     const int flags = FL >= 0 ? FL : flags_;
     VK_COL_SETUP_G(C, G, blk_, pb_, g.Pp)
+    const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) v[s] = Hrho[hoff<C>(p, t + T * s, c)];
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int ky = t + T * s;
@@ -481,7 +471,7 @@ __device__ __forceinline__ void p2_body(int blk_, int nblk_, cplx* __restrict__ 
         else if (flags & 2) Krho[(size_t)kx * N + ky] = v[s];
         v[s] = conjc(v[s]);
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) Hrho[hoff<C>(p, t + T * s, c)] = conjc(v[s]);
     if (flags & 1) {
@@ -490,7 +480,7 @@ __device__ __forceinline__ void p2_body(int blk_, int nblk_, cplx* __restrict__ 
             const int ky = t + T * s;
             v[s] = kmasked(kx, ksg(ky, N), N) ? czero() : conjc(KV[(size_t)kx * N + ky]);
         }
-        fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+        fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
         for (int s = 0; s < S; ++s) HV[hoff<C>(p, t + T * s, c)] = conjc(v[s]);
     }
@@ -594,39 +584,40 @@ struct AdvArgs {
 };
 
 // P3 (row): rho_d (+ i V) row from the kx >= 0 halves (Hermitian), psi row
-// from Hpsi, N = (gs*rho_d + V) * psi, forward along x -> HN.
-// gs = +-g/N^2, vs = +-1/N^2 (RK4 +, ARGLE -); psi scaled by 1/N^2.
+// as P1 stored it (x-space, scaled), N = (gs*rho_d + V) * psi, forward along
+// x -> HN.  gs = +-g/N^2, vs = +-1/N^2 (RK4 +, ARGLE -).
 // PM (particle mode, compile time): 0 none; 1 spectral potential (HV);
 // 2 real-space potential; 6 real-space potential + force partial sums.
 // vsign: +1 RK4, -1 ARGLE.
-// XPSI: psi comes from the x-space rows P1 stored (already scaled), so the
-// factor f stays in registers and no transform of Hpsi runs here.
 // ADV: advective ARGLE; grad psi from the rows of i kx Hpsi and of Hdy =
 // IFFT_y(i ky kpsi), two more transforms.
-template <class C, int PM, bool XPSI = false, bool ADV = false>
+template <class C, int PM, bool ADV = false>
 __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restrict__ Hrhod, const cplx* __restrict__ HV,
-                                                const cplx* __restrict__ Hpsi, cplx* __restrict__ HN,
-                                                const cplx* __restrict__ tw, Geo g, int psi_pmode,
-                                                int store_pmode, double gs, double vs, double scale,
-                                                double vsign, P3Part pa, const cplx* __restrict__ Xpsi = nullptr,
+                                                const cplx* __restrict__ Xpsi, cplx* __restrict__ HN,
+                                                const cplx* __restrict__ tw, Geo g, int store_pmode, double gs,
+                                                double vs, double vsign, P3Part pa,
+                                                const cplx* __restrict__ Hpsi = nullptr,
                                                 const cplx* __restrict__ Hdy = nullptr, AdvArgs aa = AdvArgs{})
 {
     constexpr int flags = PM;
     VK_ROW_SETUP(C)
+    const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
     const int Kp = TC * g.Pp;
-    // f in registers on the psi-row path (with real-space particles too,
-    // unless VK_P3_FREG_PART=0), else parked in LDS slots after the
-    // transform regions; particle positions staged after those during the
-    // first transform, read back as broadcasts
-    constexpr bool FREG = XPSI && ((flags & 2) == 0 || kP3FregPart);
-    double* qlds = lds + TR * C::ROWRS + (FREG ? 0 : S * C::ROWT);
+    // particle positions staged after the transform regions during the first
+    // transform, read back as broadcasts
+    double* qlds = lds + TR * C::ROWRS;
     if constexpr ((flags & 2) != 0) {
         for (int i = threadIdx.x; i < 2 * pa.np; i += blockDim.x) qlds[i] = pa.pos[i];
     }
     // kx >= 0 columns are stored; kx < 0 ones are the conjugates of N - kx
     const brsrc rR = mkbuf(Hrhod, N);
     cplx bv[(flags & 1) ? S : 1];
+    cplx xv[is_lat<C>::value ? S : 1];
+    if constexpr (is_lat<C>::value) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) xv[s] = (Xpsi + (size_t)y * N)[t + T * s];
+    }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int kxi = t + T * s;
@@ -647,19 +638,13 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
         }
         v[s] = conjc(mk(a.x - b.y, a.y + b.x));   // a + i b, conj for the inverse
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
     // v[s].x = rho_d (unnormalised); v[s].y = -V (unnormalised, flags & 1).
-    // The real factor f = g rho_d + V goes to thread-private LDS slots (after
-    // the transform regions) and waits there while psi is transformed.
-    double* fl = lds + TR * C::ROWRS;
-    double fr_[FREG ? S : 1];
-#define VK_F(s) (FREG ? fr_[FREG ? (s) : 0] : fl[(s) * C::ROWT + threadIdx.x])
+    double f[S];   // the real factor g rho_d + V
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-        double fv;
-        if constexpr ((flags & 1) != 0) fv = gs * v[s].x + vs * (-v[s].y);
-        else fv = gs * v[s].x;
-        VK_F(s) = fv;
+        if constexpr ((flags & 1) != 0) f[s] = gs * v[s].x + vs * (-v[s].y);
+        else f[s] = gs * v[s].x;
     }
     if constexpr ((flags & 2) != 0) {
         // real-space particle potential added into the slots; force partials
@@ -724,13 +709,9 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
                         double X, dX;
                         pcoord(pwrap((t + T * sw) * pa.dx - qx), X, dX);
                         const double e = pa.V0 * exp(-(X * X + Y * Y) * inv2d2);
-                        if constexpr (FREG) {
 #pragma unroll
-                            for (int s = 0; s < S; ++s)
-                                if (s == sw) fr_[FREG ? s : 0] += vsign * e;
-                        } else {
-                            fl[sw * C::ROWT + threadIdx.x] += vsign * e;
-                        }
+                        for (int s = 0; s < S; ++s)
+                            if (s == sw) f[s] += vsign * e;
                         fr[0] += rs * (-e * X * dX * invd2);
                         fr[1] += rs * (-e * Y * dY * invd2);
                     }
@@ -758,35 +739,20 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
             for (int s = 0; s < S; ++s) {
                 const size_t i = (size_t)y * N + t + T * s;
                 const double ux = aa.ux[i], uy = aa.uy[i];
-                VK_F(s) -= aa.c4 * (ux * ux + uy * uy);
+                f[s] -= aa.c4 * (ux * ux + uy * uy);
             }
         } else if (aa.tg) {
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 const cplx e = tw[t + T * s];
                 const double ux = -e.y * cy_, uy = -e.x * sy_;
-                VK_F(s) -= aa.c4 * (ux * ux + uy * uy);
+                f[s] -= aa.c4 * (ux * ux + uy * uy);
             }
         }
     }
-    if constexpr (XPSI) {
-        const cplx* xr = Xpsi + (size_t)y * N;
+    const cplx* xr = Xpsi + (size_t)y * N;
 #pragma unroll
-        for (int s = 0; s < S; ++s) v[s] = rmul(VK_F(s), xr[t + T * s]);
-    } else {
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const int pp = VK_PANEL(s);
-            v[s] = panel_stored(pp, NP, g, psi_pmode) ? conjc(Hpsi[hoff<C>(pp, y, c)]) : czero();
-        }
-        fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const cplx ps = rmul(scale, conjc(v[s]));
-            v[s] = rmul(VK_F(s), ps);
-        }
-    }
-#undef VK_F
+    for (int s = 0; s < S; ++s) v[s] = rmul(f[s], is_lat<C>::value ? xv[is_lat<C>::value ? s : 0] : xr[t + T * s]);
     if constexpr (ADV) {
         // -i (u + v).grad psi, one gradient component at a time
         cplx w[S];
@@ -796,7 +762,7 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
             for (int s = 0; s < S; ++s) {
                 const int pp = VK_PANEL(s);
                 cplx a = czero();
-                if (panel_stored(pp, NP, g, psi_pmode)) {
+                if (panel_stored(pp, NP, g, 0)) {
                     if (comp == 0) {
                         a = Hpsi[hoff<C>(pp, y, c)];
                         const double kk = (double)ksg(t + T * s, N);
@@ -807,7 +773,7 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
                 }
                 w[s] = conjc(a);
             }
-            fft_fwd<N, S, C::SPLIT>(w, lg, t, tw);
+            fft_fwd<N, S, C::SPLIT>(w, lg, t, w_);
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 const cplx e = tw[t + T * s];
@@ -820,7 +786,7 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
             }
         }
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
     // branch-free buffer stores (an unstored panel gets the out-of-range
     // offset and is dropped): conditional stores made the compiler sink the
     // last butterfly into one branch per store (P3 0.191 -> 0.187 ms)
@@ -833,34 +799,22 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
 }
 
 template <class C, int PM>
-__global__ void __launch_bounds__(C::ROWT) VK_OCC k_p3(const cplx* __restrict__ Hrhod, const cplx* __restrict__ HV,
-                                                const cplx* __restrict__ Hpsi, cplx* __restrict__ HN,
-                                                const cplx* __restrict__ tw, Geo g, int psi_pmode,
-                                                int store_pmode, double gs, double vs, double scale,
-                                                double vsign, P3Part pa)
-{
-    p3_body<C, PM>(blockIdx.x, gridDim.x, Hrhod, HV, Hpsi, HN, tw, g, psi_pmode, store_pmode, gs, vs, scale, vsign, pa);
-}
-
-template <class C, int PM, bool XPSI>
 __global__ void __launch_bounds__(C::ROWT) VK_OCC k_p3a(const cplx* __restrict__ Hrhod, const cplx* __restrict__ HV,
                                                  const cplx* __restrict__ Hpsi, const cplx* __restrict__ Xpsi,
                                                  const cplx* __restrict__ Hdy, cplx* __restrict__ HN,
                                                  const cplx* __restrict__ tw, Geo g, double gs, double vs,
-                                                 double scale, double vsign, P3Part pa, AdvArgs aa)
+                                                 double vsign, P3Part pa, AdvArgs aa)
 {
-    p3_body<C, PM, XPSI, true>(blockIdx.x, gridDim.x, Hrhod, HV, Hpsi, HN, tw, g, 0, 0, gs, vs, XPSI ? 1.0 : scale,
-                               vsign, pa, Xpsi, Hdy, aa);
+    p3_body<C, PM, true>(blockIdx.x, gridDim.x, Hrhod, HV, Xpsi, HN, tw, g, 0, gs, vs, vsign, pa, Hpsi, Hdy, aa);
 }
 
 template <class C, int PM>
-__global__ void __launch_bounds__(C::ROWT) VK_P3OCC(PM) k_p3x(const cplx* __restrict__ Hrhod, const cplx* __restrict__ HV,
+__global__ void __launch_bounds__(C::ROWT) VK_P3OCC(C, PM) k_p3x(const cplx* __restrict__ Hrhod, const cplx* __restrict__ HV,
                                                  const cplx* __restrict__ Xpsi, cplx* __restrict__ HN,
                                                  const cplx* __restrict__ tw, Geo g, int store_pmode, double gs,
                                                  double vs, double vsign, P3Part pa)
 {
-    p3_body<C, PM, true>(blockIdx.x, gridDim.x, Hrhod, HV, nullptr, HN, tw, g, 0, store_pmode, gs, vs, 1.0, vsign,
-                         pa, Xpsi);
+    p3_body<C, PM>(blockIdx.x, gridDim.x, Hrhod, HV, Xpsi, HN, tw, g, store_pmode, gs, vs, vsign, pa);
 }
 
 struct RKArgs {
@@ -894,13 +848,27 @@ __device__ __forceinline__ void p4_body(int blk_, int nblk_, const cplx* __restr
                                                 Geo g, RKArgs a)
 {
     VK_COL_SETUP_G(C, G, blk_, panel_of_block(pb_, C::NP, g, 1), g.Pp + g.Pn)
+    const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) v[s] = HN[hoff<C>(p, t + T * s, c)];
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
     const int kxs = ksg(kx, N);
     const size_t rowo = (size_t)kx * N;
     const brsrc r0 = mkbuf(K0, N), r1 = mkbuf(K1, N), r2 = mkbuf(K2, N);
+    // LAT: the K operands before the transform (their latency overlaps it)
+    constexpr bool LAT = is_lat<C>::value;
+    cplx k0v[LAT ? S : 1], k1v[LAT && STAGE >= 3 ? S : 1], k2v[LAT && STAGE >= 2 ? S : 1];
+    if constexpr (LAT) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int ky = t + T * s;
+            const unsigned o = boff(rowo + ky, !kmasked(kxs, ksg(ky, N), N));
+            k0v[s] = bld(r0, o);
+            if constexpr (STAGE >= 2) k2v[s] = bld(r2, o);
+            if constexpr (STAGE >= 3) k1v[s] = bld(r1, o);
+        }
+    }
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int ky = t + T * s;
@@ -908,15 +876,15 @@ __device__ __forceinline__ void p4_body(int blk_, int nblk_, const cplx* __restr
         const bool keep = !kmasked(kxs, kys, N);
         const unsigned o = boff(rowo + ky, keep);
         const double kr2 = (double)(kxs * kxs + kys * kys);
-        const cplx s1 = bld(r0, o);
-        const cplx ps = STAGE == 1 ? s1 : bld(r2, o);
+        const cplx s1 = LAT ? k0v[LAT ? s : 0] : bld(r0, o);
+        const cplx ps = STAGE == 1 ? s1 : LAT ? k2v[LAT ? s : 0] : bld(r2, o);
         const cplx lin = rmul(a.alpha * kr2 - a.omega, ps);
         const cplx rhs = cmul(a.pref, cadd(lin, v[s]));
         const cplx inc = rmul(a.wacc, rhs);
         cplx acc = inc, kn;
         if constexpr (STAGE == 2) acc = cadd(rmul(a.r1, csub(ps, s1)), inc);
-        else if constexpr (STAGE == 3) acc = cadd(bld(r1, o), inc);
-        else if constexpr (STAGE == 4) acc = cadd(cadd(bld(r1, o), rmul(a.r3, csub(ps, s1))), inc);
+        else if constexpr (STAGE == 3) acc = cadd(LAT ? k1v[LAT ? s : 0] : bld(r1, o), inc);
+        else if constexpr (STAGE == 4) acc = cadd(cadd(LAT ? k1v[LAT ? s : 0] : bld(r1, o), rmul(a.r3, csub(ps, s1))), inc);
         if constexpr (STAGE < 4) {
             if constexpr (STAGE == 2) bst(r1, o, acc);
             kn = cadd(s1, rmul(a.cstep, rhs));
@@ -927,13 +895,13 @@ __device__ __forceinline__ void p4_body(int blk_, int nblk_, const cplx* __restr
         }
         v[s] = conjc(keep ? kn : czero());
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) Hpsi[hoff<C>(p, t + T * s, c)] = conjc(v[s]);
 }
 
 template <class C, int STAGE, int G = C::TC>
-__global__ void __launch_bounds__(G * C::T) VK_P4OCC k_p4(const cplx* __restrict__ HN, cplx* __restrict__ Hpsi,
+__global__ void __launch_bounds__(G * C::T) VK_P4OCC(C) k_p4(const cplx* __restrict__ HN, cplx* __restrict__ Hpsi,
                                                 cplx* __restrict__ K0, cplx* __restrict__ K1,
                                                 cplx* __restrict__ K2, const cplx* __restrict__ tw,
                                                 Geo g, RKArgs a)
@@ -965,12 +933,19 @@ __device__ __forceinline__ void a4_body(int blk_, int nblk_, const cplx* __restr
                                                 ArgleArgs a, double* __restrict__ part)
 {
     VK_COL_SETUP_G(C, G, blk_, pb_, C::NP)
+    const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) v[s] = HN[hoff<C>(p, t + T * s, c)];
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
     const int kxs = ksg(kx, N);
     const size_t rowo = (size_t)kx * N;
+    constexpr bool LAT = is_lat<C>::value;
+    cplx k0v[LAT ? S : 1];
+    if constexpr (LAT) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) k0v[s] = K0[rowo + t + T * s];
+    }
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
     double r[2] = {0.0, 0.0};
     const double omega = a.omega_dev ? *a.omega_dev : a.omega;
 #pragma unroll
@@ -978,7 +953,7 @@ __device__ __forceinline__ void a4_body(int blk_, int nblk_, const cplx* __restr
         const int ky = t + T * s;
         const int kys = ksg(ky, N);
         const size_t o = rowo + ky;
-        const cplx old = K0[o];
+        const cplx old = LAT ? k0v[LAT ? s : 0] : K0[o];
         const double kr2 = (double)(kxs * kxs + kys * kys);
         const cplx t1 = cadd(v[s], rmul(omega, old));
         const double t2 = 1.0 + a.alpha * kr2 * a.dt;
@@ -997,7 +972,7 @@ __device__ __forceinline__ void a4_body(int blk_, int nblk_, const cplx* __restr
         }
         v[s] = conjc(nw);
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, tw);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) Hpsi[hoff<C>(p, t + T * s, c)] = conjc(v[s]);
     if (a.want_res) {
