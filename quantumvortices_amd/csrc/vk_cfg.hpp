@@ -185,10 +185,11 @@ __device__ __forceinline__ size_t hoff(int p, int y, int c)
 // offsets fit in 32 bits and kOOB is beyond every field.
 typedef __amdgpu_buffer_rsrc_t brsrc;
 constexpr unsigned kOOB = 0x80000000u;
-__device__ __forceinline__ brsrc mkbuf(const void* p, int N)
+__device__ __forceinline__ brsrc mkbuf_bytes(const void* p, int bytes)
 {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, N * N * 16, 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, bytes, 0x00020000);
 }
+__device__ __forceinline__ brsrc mkbuf(const void* p, int N) { return mkbuf_bytes(p, N * N * 16); }
 __device__ __forceinline__ cplx bld(brsrc r, unsigned off)
 {
     const auto w = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);

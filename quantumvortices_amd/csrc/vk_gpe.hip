@@ -131,8 +131,14 @@ struct vk_gpe {
     cplx *Xn = nullptr, *Kn = nullptr;
     double *omega_dev = nullptr, *npart = nullptr;
     cplx *HV = nullptr, *KV = nullptr, *Krho = nullptr, *Vhat = nullptr, *EX = nullptr, *EY = nullptr;
+    double* pst2 = nullptr;   // real-space path: positions and velocities after RK4 stages 1 and 3
+    int side_busy = 0;        // a particle update is queued on pstream
     double *fpart = nullptr, *pst = nullptr, *part = nullptr, *dsum = nullptr;
     unsigned char* phit = nullptr;   // real-space path: window flags per row block and particle
+    int4* pwin = nullptr;            // real-space path: windows and factor tables of the positions,
+    double2 *ptx = nullptr, *pty = nullptr;
+    double* Vx = nullptr;            // and the potential on the grid for ARGLE
+    int tab_valid = 0, vx_valid = 0; // they belong to the current positions
     int hstate = 0;   // 0: Hpsi stale, 1: Hpsi = IFFT_y K0 on all panels, 2: K0 dealiased, Hpsi on retained panels,
                       // 3: K0 dealiased, Hpsi on the retained panels of the single-field shape svar (layout CfgE<N, svar>)
     int kv_valid = 0;
@@ -246,8 +252,8 @@ void row_launch(vk_gpe* h, int kind, Kern k, A... args)
     row_launch_x<C>(h, kind, 0, k, args...);
 }
 
-// P3 stages the particle positions after its transform regions
-size_t p3_extra(const vk_gpe* h) { return 2 * (size_t)std::max(h->p.np, 1) * sizeof(double); }
+// P3 stages the particle windows after its transform regions
+size_t p3_extra(const vk_gpe* h) { return (size_t)std::max(h->p.np, 1) * sizeof(int4); }
 
 // P2 columns per workgroup.  P2 covers only the kx >= 0 panels.  At
 // 4096^2 one column per workgroup (1366 workgroups) is the fastest: with
@@ -446,7 +452,7 @@ double ipow(double x, int n)
     return r;
 }
 
-vk::PartArgs part_args(const vk_gpe* h, int nrows, int half, int stage, int src = 0, int nblk = 0)
+vk::PartArgs part_args(const vk_gpe* h, int nrows, int half, int stage, int nblk = 0, int nw = 0)
 {
     const double pi = 4.0 * std::atan(1.0);
     const double L = 2.0 * pi;
@@ -464,9 +470,8 @@ vk::PartArgs part_args(const vk_gpe* h, int nrows, int half, int stage, int src 
     a.dt = h->p.dt;
     a.mass = h->p.mass;
     a.stage = stage;
-    a.src = src;
     a.nblk = nblk;
-    a.coef_rs = 2.0 * h->p.alpha * (dx * dx) / ((double)h->N * (double)h->N);
+    a.nw = nw;
     return a;
 }
 
@@ -492,17 +497,40 @@ vk::P3Part p3part(const vk_gpe* h)
 {
     vk::P3Part q{};
     if (h->p.np > 0 && h->have_part) {
-        const double pi = 4.0 * std::atan(1.0);
-        q.pos = h->pst;
+        q.win = h->pwin;
+        q.tx = h->ptx;
+        q.ty = h->pty;
         q.ppart = h->fpart;
         q.phit = h->phit;
         q.np = h->p.np;
-        q.V0 = h->p.V0;
-        q.d = h->p.d;
-        q.W = real_space_window(h->p.d);
-        q.dx = 2.0 * pi / h->N;
+        q.vx = h->Vx;
     }
     return q;
+}
+
+vk::WTab wtab(const vk_gpe* h)
+{
+    return vk::WTab{h->p.V0, h->p.d, real_space_window(h->p.d), h->pwin, h->ptx, h->pty};
+}
+
+// windows and tables of the current positions
+void particle_tables(vk_gpe* h)
+{
+    hipLaunchKernelGGL(vk::k_wtab, dim3(h->p.np, 2), dim3(128), 0, h->stream, (const double*)h->pst, h->N, wtab(h));
+    h->tab_valid = 1;
+}
+
+// ARGLE never moves the particles: their potential on the grid, once per set
+// of positions
+int particle_field(vk_gpe* h)
+{
+    if (h->vx_valid) return 0;
+    if (!h->Vx) HIPCHK(hipMalloc(&h->Vx, f2(h) * sizeof(double)));
+    if (!h->tab_valid) particle_tables(h);
+    hipLaunchKernelGGL(vk::k_potfield, dim3(std::min((int)(f2(h) / 256), 4096)), dim3(256), 0, h->stream,
+                       (const int4*)h->pwin, (const double2*)h->ptx, (const double2*)h->pty, h->p.np, h->N, h->Vx);
+    h->vx_valid = 1;
+    return 0;
 }
 
 // Real-space particle path in P3: valid when the Gaussian's spectrum beyond
@@ -542,33 +570,37 @@ int particle_forces(vk_gpe* h, const cplx* Krho, int nrows, int half, int stage)
     return 0;
 }
 
-// particle stage update from the real-space block partials written by P3
-// The update depends on P3 (force partials) and is needed by the next
-// P3 (positions); it runs on a side stream while P4, P1, P2 proceed.
+// Particle stage update from the real-space block partials written by P3; the
+// next P3 needs its window tables.  From 2048^2 on it runs on a side stream
+// while P4, P1, P2 proceed (0.1 ms of passes hide it); below, the two event
+// waits would cost more than the update itself (6 us).
 int particle_step_rs(vk_gpe* h, int nblk, int nw, int stage)
 {
-    const bool side = !h->timing && h->pstream;
+    const bool side = !h->timing && h->pstream && h->N >= 2048;
     hipStream_t st = side ? h->pstream : h->stream;
     if (side) {
         hipEventRecord(h->ev_p3, h->stream);
         hipStreamWaitEvent(h->pstream, h->ev_p3, 0);
     }
     ev_begin(h);
-    const double dx = 2.0 * (4.0 * std::atan(1.0)) / h->N;
-    const double coef = 2.0 * h->p.alpha * (dx * dx) / ((double)h->N * (double)h->N);
-    hipLaunchKernelGGL(vk::k_pforce_rs, dim3(h->p.np), dim3(256), 0, st, (const double*)h->fpart,
-                       (const unsigned char*)h->phit, nblk, nw, h->p.np, coef, h->pst + 28 * h->p.np + 8);
-    hipLaunchKernelGGL(vk::k_pstep, dim3(1), dim3(vk::PSTEP_T), 0, st, (const double*)h->fpart, (const cplx*)h->EX,
-                       h->pst, part_args(h, 0, 0, stage, 1, nblk));
+    double *cur = stage % 2 ? h->pst : h->pst2, *nxt = stage % 2 ? h->pst2 : h->pst;
+    hipLaunchKernelGGL(vk::k_pstage, dim3(h->p.np), dim3(256), 0, st, (const double*)h->fpart,
+                       (const unsigned char*)h->phit, (const double*)cur, nxt, h->pst,
+                       part_args(h, 0, 0, stage, nblk, nw), wtab(h));
     ev_end(h, PK_PART);
-    if (side) hipEventRecord(h->ev_ps, h->pstream);
+    if (side) {
+        hipEventRecord(h->ev_ps, h->pstream);
+        h->side_busy = 1;
+    }
     return 0;
 }
 
 // order the main stream after the last side-stream particle update
 void join_particles(vk_gpe* h)
 {
-    if (h->pstream && h->ev_ps) hipStreamWaitEvent(h->stream, h->ev_ps, 0);
+    if (!h->side_busy) return;
+    hipStreamWaitEvent(h->stream, h->ev_ps, 0);
+    h->side_busy = 0;
 }
 
 // ---- RK4 / ARGLE -----------------------------------------------------------------
@@ -587,6 +619,8 @@ int rk4_step(vk_gpe* h)
         const int parts = h->have_part && h->p.np > 0;
         const int rs = parts && h->rs_part;
         const int Kp = C::TC * h->geo.Pp;
+        if (rs && !h->tab_valid) particle_tables(h);
+        h->vx_valid = 0;
         const vk::P3Part pa = p3part(h);
         vk::RKArgs a{};
         a.pref = make_double2(-h->p.disp, -1.0);   // (1 - i disp)/i
@@ -609,11 +643,11 @@ int rk4_step(vk_gpe* h)
             if (parts && !rs) particle_forces(h, h->Krho, Kp, 1, stage);
             if (rs) join_particles(h);   // positions from the previous stage
             if (VAR && h->tr1_p3) {
-                auto k3 = !parts ? vk::k_p3x<C1, 0> : (rs ? vk::k_p3x<C1, 6> : vk::k_p3x<C1, 1>);
+                auto k3 = !parts ? vk::k_p3x<C1, 0> : (rs ? vk::k_p3x<C1, 4> : vk::k_p3x<C1, 1>);
                 row_launch_x<C1>(h, PK_P3, p3_extra(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV,
                                  (const cplx*)h->Xs, h->HN, (const cplx*)h->tw, h->geo, 1, h->p.g * sc, sc, 1.0, pa);
             } else {
-                auto k3 = !parts ? vk::k_p3x<C, 0> : (rs ? vk::k_p3x<C, 6> : vk::k_p3x<C, 1>);
+                auto k3 = !parts ? vk::k_p3x<C, 0> : (rs ? vk::k_p3x<C, 4> : vk::k_p3x<C, 1>);
                 row_launch_x<C>(h, PK_P3, p3_extra(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV,
                                 (const cplx*)h->Xs, h->HN, (const cplx*)h->tw, h->geo, 1, h->p.g * sc, sc, 1.0, pa);
             }
@@ -672,6 +706,10 @@ int argle_step(vk_gpe* h, int want_res, const double* noise = nullptr)
         const double sc = scale_of(h);
         const int parts = h->have_part && h->p.np > 0;
         const int rs = parts && h->rs_part;
+        if (rs) {
+            int rc = particle_field(h);
+            if (rc) return rc;
+        }
         const vk::P3Part pa = p3part(h);
         if (parts && !rs && !h->kv_valid) {
             particle_kv(h, C::TC * h->geo.Pp);
@@ -690,11 +728,11 @@ int argle_step(vk_gpe* h, int want_res, const double* noise = nullptr)
                                  h->adv_field ? (const double*)h->Ux : nullptr,
                                  h->adv_field ? (const double*)h->Uy : nullptr};
             row_launch_x<C>(h, PK_P3, p3_extra(h),
-                            !parts ? vk::k_p3a<C, 0> : (rs ? vk::k_p3a<C, 2> : vk::k_p3a<C, 1>), (const cplx*)h->Hrho,
+                            !parts ? vk::k_p3a<C, 0> : (rs ? vk::k_p3a<C, 8> : vk::k_p3a<C, 1>), (const cplx*)h->Hrho,
                             (const cplx*)h->HV, (const cplx*)h->Hpsi, (const cplx*)h->Xs, (const cplx*)h->Hdy, h->HN,
                             (const cplx*)h->tw, h->geo, -h->p.g * sc, -sc, -1.0, pa, aa);
         } else {
-            auto k3 = !parts ? vk::k_p3x<C, 0> : (rs ? vk::k_p3x<C, 2> : vk::k_p3x<C, 1>);
+            auto k3 = !parts ? vk::k_p3x<C, 0> : (rs ? vk::k_p3x<C, 8> : vk::k_p3x<C, 1>);
             row_launch_x<C>(h, PK_P3, p3_extra(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV, (const cplx*)h->Xs,
                             h->HN, (const cplx*)h->tw, h->geo, 0, -h->p.g * sc, -sc, -1.0, pa);
         }
@@ -987,6 +1025,10 @@ int vk_gpe_create(vk_gpe** out, const vk_gpe_params* p)
             hipMalloc(&h->EY, sizeof(cplx) * np * N) != hipSuccess ||
             hipMalloc(&h->fpart, sizeof(double) * nfp) != hipSuccess ||
             hipMalloc(&h->phit, rows * np) != hipSuccess ||
+            hipMalloc(&h->pst2, sizeof(double) * 4 * np) != hipSuccess ||
+            hipMalloc(&h->pwin, sizeof(int4) * np) != hipSuccess ||
+            hipMalloc(&h->ptx, sizeof(double2) * np * N) != hipSuccess ||
+            hipMalloc(&h->pty, sizeof(double2) * np * N) != hipSuccess ||
             hipMalloc(&h->pst, sizeof(double) * (30 * np + 8)) != hipSuccess)
             return cleanup(fail(VK_ERR_HIP, "hipMalloc failed (particle tables)"));
         if (hipMemset(h->pst, 0, sizeof(double) * (30 * np + 8)) != hipSuccess)
@@ -1018,6 +1060,11 @@ void vk_gpe_destroy(vk_gpe* h)
         for (auto f : pf) if (f) hipFree(f);
         if (h->fpart) hipFree(h->fpart);
         if (h->phit) hipFree(h->phit);
+        if (h->pst2) hipFree(h->pst2);
+        if (h->pwin) hipFree(h->pwin);
+        if (h->ptx) hipFree(h->ptx);
+        if (h->pty) hipFree(h->pty);
+        if (h->Vx) hipFree(h->Vx);
         if (h->pst) hipFree(h->pst);
     }
     for (auto x : h->X) if (x) hipFree(x);
@@ -1201,7 +1248,7 @@ int vk_gpe_particles_set(vk_gpe* h, const double* pos, const double* vel, const 
     if (fext) HIPCHK(hipMemcpyAsync(h->pst + 4 * np, fext, sizeof(double) * 2 * np, hipMemcpyDefault, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
     if (!h->have_part && (rc = particle_potential(h))) return rc;
-    h->kv_valid = 0;
+    h->kv_valid = h->tab_valid = h->vx_valid = 0;
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipGetLastError());
     return 0;
@@ -1407,7 +1454,7 @@ int vk_gpe_set_obstacles(vk_gpe* h, int np, const double* pos, double V0, double
     h->p.d = d;
     h->rs_part = use_real_space(h->p);
     h->have_part = 0;
-    h->kv_valid = 0;
+    h->kv_valid = h->tab_valid = h->vx_valid = 0;
     if (np == 0) return 0;
     std::vector<double> st(30 * (size_t)np + 8, 0.0);
     std::copy(pos, pos + 2 * np, st.begin());
@@ -1642,7 +1689,7 @@ int vk_gpe_autotune_rows(vk_gpe* h, int nsteps, int* choice, double* ms_out)
     release();
     if (rc) return rc;
     h->hstate = 2;
-    h->kv_valid = 0;
+    h->kv_valid = h->tab_valid = h->vx_valid = 0;
     if (choice) { choice[0] = b1; choice[1] = b3; }
     return 0;
 }

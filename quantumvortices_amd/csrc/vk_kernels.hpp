@@ -33,22 +33,12 @@
 #else
 #define VK_P1OCC VK_OCC
 #endif
-// P3 on the psi-row path without particles (PM = 0) at 4 waves per SIMD
-// (<= 128 VGPRs): +0.8% pure-GPE steps/s with two rows per workgroup.  With
-// particles the compiler's choice (231 VGPRs with one row per workgroup,
-// two workgroups per CU) is kept: at 3 waves per SIMD (168 VGPRs, 188 B of
-// spills) P3 takes 0.243 instead of 0.163 ms.
+// P3 without particles or with real-space ones (PM 0, 4) at 4 waves per SIMD
+// (<= 128 VGPRs; LAT shapes, one wave per SIMD, as they come)
 #ifndef VK_P3_WAVES
 #define VK_P3_WAVES 4
 #endif
-#if VK_P3_WAVES > 0
-#ifndef VK_P3_PART_WAVES
-#define VK_P3_PART_WAVES 1
-#endif
-#define VK_P3OCC(C, PM) __attribute__((amdgpu_waves_per_eu(!is_lat<C>::value && (PM) == 0 ? VK_P3_WAVES : VK_P3_PART_WAVES)))
-#else
-#define VK_P3OCC(C, PM) VK_OCC
-#endif
+#define VK_P3OCC(C, PM) __attribute__((amdgpu_waves_per_eu(!is_lat<C>::value && ((PM) == 0 || (PM) == 4) ? VK_P3_WAVES : 1)))
 
 namespace vk {
 
@@ -544,12 +534,19 @@ __device__ __forceinline__ void block_sum(double (&x)[NV], double* sh)
 // spectrum is negligible beyond the dealias radius, so that the reference's
 // spectral translation IFFT(exp(-i k.q) Vhat) equals V(x - q) to far below
 // FP64 roundoff; see the host-side selection).
+// V and its gradient factor into one function of x and one of y per particle,
+// tabulated over the window by k_wtab whenever the positions change.  P3 with
+// the sines and exponentials in its point loop took 17.5 us at 512^2 with 8
+// particles (229 VGPRs and 162 us at 4096^2 with 32); from the tables 10.9 us
+// (128 VGPRs, 137 us: the time without particles).
 struct P3Part {
-    const double* pos;   // (x, y) per particle
+    const int4* win;     // per particle: first column and count of its window, first row and count
+    const double2* tx;   // [particle][k < N]: ex, -ex X dX/dx / d^2, ex = exp(-X^2 / (2 d^2))
+    const double2* ty;   // the same in y, times V0
     double* ppart;       // per row block, wave and particle: sum rho_raw * dV/dx, dV/dy
     unsigned char* phit; // per row block and particle: 1 if the window reaches the block
     int np;
-    double V0, d, W, dx; // potential height, width, window radius, grid spacing
+    const double* vx;    // static potential on the grid (PM 8)
 };
 
 // minimum-image displacement in [-pi, pi)
@@ -586,8 +583,9 @@ struct AdvArgs {
 // P3 (row): rho_d (+ i V) row from the kx >= 0 halves (Hermitian), psi row
 // as P1 stored it (x-space, scaled), N = (gs*rho_d + V) * psi, forward along
 // x -> HN.  gs = +-g/N^2, vs = +-1/N^2 (RK4 +, ARGLE -).
-// PM (particle mode, compile time): 0 none; 1 spectral potential (HV);
-// 2 real-space potential; 6 real-space potential + force partial sums.
+// PM (particle mode, compile time): 0 none; 1 spectral potential (HV); 4
+// real-space potential of moving particles + force partial sums; 8 static
+// potential from the grid array.
 // vsign: +1 RK4, -1 ARGLE.
 // ADV: advective ARGLE; grad psi from the rows of i kx Hpsi and of Hdy =
 // IFFT_y(i ky kpsi), two more transforms.
@@ -604,19 +602,26 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
     const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
     const int Kp = TC * g.Pp;
-    // particle positions staged after the transform regions during the first
+    // particle windows staged after the transform regions during the first
     // transform, read back as broadcasts
-    double* qlds = lds + TR * C::ROWRS;
-    if constexpr ((flags & 2) != 0) {
-        for (int i = threadIdx.x; i < 2 * pa.np; i += blockDim.x) qlds[i] = pa.pos[i];
+    int4* ql = reinterpret_cast<int4*>(lds + TR * C::ROWRS);
+    if constexpr ((flags & 4) != 0) {
+        for (int i = threadIdx.x; i < pa.np; i += blockDim.x) ql[i] = pa.win[i];
+        // a one-wave workgroup's transform has no barrier
+        if constexpr (C::ROWT <= 64) lds_barrier();
     }
     // kx >= 0 columns are stored; kx < 0 ones are the conjugates of N - kx
     const brsrc rR = mkbuf(Hrhod, N);
     cplx bv[(flags & 1) ? S : 1];
     cplx xv[is_lat<C>::value ? S : 1];
+    double sv[(flags & 8) ? S : 1];
     if constexpr (is_lat<C>::value) {
 #pragma unroll
         for (int s = 0; s < S; ++s) xv[s] = (Xpsi + (size_t)y * N)[t + T * s];
+    }
+    if constexpr ((flags & 8) != 0) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) sv[(flags & 8) ? s : 0] = pa.vx[(size_t)y * N + t + T * s];
     }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
@@ -646,15 +651,14 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
         if constexpr ((flags & 1) != 0) f[s] = gs * v[s].x + vs * (-v[s].y);
         else f[s] = gs * v[s].x;
     }
-    if constexpr ((flags & 2) != 0) {
-        // real-space particle potential added into the slots; force partials
-        double rho[S];
+    if constexpr ((flags & 8) != 0) {
 #pragma unroll
-        for (int s = 0; s < S; ++s) rho[s] = v[s].x;
+        for (int s = 0; s < S; ++s) f[s] += vsign * sv[(flags & 8) ? s : 0];
+    }
+    if constexpr ((flags & 4) != 0) {
+        // real-space particle potential added into f; force partials
         const int blk = xcd_remap(blk_, nblk_);
         const int yb = blk * TR;
-        const double inv2d2 = 1.0 / (2.0 * (pa.d * pa.d)), invd2 = 1.0 / (pa.d * pa.d);
-        const double idx = 1.0 / pa.dx, Wg = pa.W * idx, invN = 1.0 / N;
         // The particle loop has no workgroup barrier: every wave tests the
         // windows itself (one lane per particle, a ballot gives the hit set,
         // the same in every wave), reduces its force partials with lane
@@ -663,70 +667,53 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
         constexpr int WV = C::ROWT < 64 ? C::ROWT : 64;   // lanes of a wave in use
         constexpr int NW = (C::ROWT + 63) / 64;            // waves per workgroup
         const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
+        const brsrc rX = mkbuf_bytes(pa.tx, pa.np * N * 16);
         for (int base = 0; base < pa.np; base += WV) {
-            // window test in grid units (multiplications only): minimum-image
-            // row distance of the workgroup's rows to the particle
             const int pq = base + lane;
             bool hit = false;
             if (lane < WV && pq < pa.np) {
-                const double cyq = qlds[2 * pq + 1] * idx;
-                for (int r2 = 0; r2 < TR; ++r2) {
-                    double dr = (yb + r2) - cyq;
-                    dr -= N * rint(dr * invN);
-                    hit |= fabs(dr) <= Wg;
-                }
-                if constexpr ((flags & 4) != 0)
-                    if (wv == 0) pa.phit[(size_t)blk * pa.np + pq] = hit ? 1 : 0;
+                const int4 w = ql[pq];
+                for (int r2 = 0; r2 < TR; ++r2) hit |= ((yb + r2 - w.z) & (N - 1)) < w.w;
+                if (wv == 0) pa.phit[(size_t)blk * pa.np + pq] = hit ? 1 : 0;
             }
             // hit particles in increasing order (uniform over the wave)
             for (unsigned long long m = __ballot(hit); m != 0ull; m &= m - 1ull) {
                 const int pp = base + __builtin_ctzll(m);
-                const double qx = qlds[2 * pp], qy = qlds[2 * pp + 1];
-                const double cx = qx * idx, cy = qy * idx;   // centre in grid units
+                const int4 w = ql[pp];
                 double fr[2] = {0.0, 0.0};
-                double dr = y - cy;
-                dr -= N * rint(dr * invN);
-                if (fabs(dr) <= Wg) {
-                    double Y, dY;
-                    pcoord(pwrap(y * pa.dx - qy), Y, dY);
-                    // points of this thread inside the window (cheap test for
-                    // all S), then the transcendental work once per such point,
-                    // in increasing s (a single point when the window is
-                    // narrower than the thread stride T)
-                    unsigned mask = 0;
+                const int ky = (y - w.z) & (N - 1);
+                const bool row = ky < w.w;
+                const double2 wy = pa.ty[(size_t)pp * N + (row ? ky : 0)];
+                // LAT shapes: a window spans several of a thread's points, all
+                // its loads at once; else (window narrower than the thread
+                // stride T) mostly one, skipped by the waves outside
+                cplx wx[is_lat<C>::value ? S : 1];
+                if constexpr (is_lat<C>::value) {
 #pragma unroll
                     for (int s = 0; s < S; ++s) {
-                        double dc = (t + T * s) - cx;
-                        dc -= N * rint(dc * invN);
-                        if (fabs(dc) <= Wg) mask |= 1u << s;
-                    }
-                    while (mask) {
-                        const int sw = __builtin_ctz(mask);
-                        mask &= mask - 1;
-                        double rs = 0.0;
-#pragma unroll
-                        for (int s = 0; s < S; ++s) rs = (s == sw) ? rho[s] : rs;
-                        double X, dX;
-                        pcoord(pwrap((t + T * sw) * pa.dx - qx), X, dX);
-                        const double e = pa.V0 * exp(-(X * X + Y * Y) * inv2d2);
-#pragma unroll
-                        for (int s = 0; s < S; ++s)
-                            if (s == sw) f[s] += vsign * e;
-                        fr[0] += rs * (-e * X * dX * invd2);
-                        fr[1] += rs * (-e * Y * dY * invd2);
+                        const int k = (t + T * s - w.x) & (N - 1);
+                        wx[s] = bld(rX, boff((size_t)pp * N + k, row && k < w.y));
                     }
                 }
-                if constexpr ((flags & 4) != 0) {
 #pragma unroll
-                    for (int o = WV / 2; o > 0; o >>= 1) {
-                        fr[0] += __shfl_xor(fr[0], o, WV);
-                        fr[1] += __shfl_xor(fr[1], o, WV);
+                for (int s = 0; s < S; ++s) {
+                    const int k = (t + T * s - w.x) & (N - 1);
+                    if (is_lat<C>::value || (row && k < w.y)) {
+                        const cplx a = is_lat<C>::value ? wx[is_lat<C>::value ? s : 0] : bld(rX, boff((size_t)pp * N + k, true));
+                        f[s] += vsign * (a.x * wy.x);
+                        fr[0] += v[s].x * (a.y * wy.x);
+                        fr[1] += v[s].x * (a.x * wy.y);
                     }
-                    if (lane == 0) {
-                        double* q = pa.ppart + (((size_t)blk * NW + wv) * pa.np + pp) * 2;
-                        q[0] = fr[0];
-                        q[1] = fr[1];
-                    }
+                }
+#pragma unroll
+                for (int o = WV / 2; o > 0; o >>= 1) {
+                    fr[0] += __shfl_xor(fr[0], o, WV);
+                    fr[1] += __shfl_xor(fr[1], o, WV);
+                }
+                if (lane == 0) {
+                    double* q = pa.ppart + (((size_t)blk * NW + wv) * pa.np + pp) * 2;
+                    q[0] = fr[0];
+                    q[1] = fr[1];
                 }
             }
         }
@@ -1222,6 +1209,65 @@ __global__ void k_pot_x(cplx* __restrict__ X, int N, double dx, double c1, doubl
     }
 }
 
+struct WTab {
+    double V0, d, W;     // potential height, width, window radius
+    int4* win;
+    double2 *tx, *ty;
+};
+
+// Windows and factor tables of the real-space particle potential (P3Part):
+// particle p covers the columns x with |x dx - qx| <= W (minimum image, all N
+// when the window spans the period), from column win.x on; V(x, y) =
+// tx.x ty.x, dV/dx = tx.y ty.x, dV/dy = tx.x ty.y.  Positions that are not
+// finite get empty windows.  One direction of one particle at coordinate q,
+// by nt threads.
+__device__ __forceinline__ void window_table(const WTab& w, int p, int dir, double q, int N, int tid, int nt)
+{
+    const double dx = 6.283185307179586476925 / N;
+    const double c = q / dx, r = w.W / dx;
+    int n = 0, first = 0;
+    if (fabs(c) < 1e15) {
+        const double lo = ceil(c - r), hi = floor(c + r);
+        n = (int)fmin(fmax(hi - lo + 1.0, 0.0), (double)N);
+        first = (int)(lo - N * floor(lo / N)) & (N - 1);
+    }
+    if (tid == 0) {
+        int* o = reinterpret_cast<int*>(w.win + p) + 2 * dir;
+        o[0] = first;
+        o[1] = n;
+    }
+    const double inv2d2 = 1.0 / (2.0 * (w.d * w.d)), invd2 = 1.0 / (w.d * w.d), a = dir ? w.V0 : 1.0;
+    double2* tab = (dir ? w.ty : w.tx) + (size_t)p * N;
+    for (int k = tid; k < n; k += nt) {
+        double X, dX;
+        pcoord(pwrap(((first + k) & (N - 1)) * dx - q), X, dX);
+        const double e = a * exp(-(X * X) * inv2d2);
+        tab[k] = make_double2(e, -e * X * dX * invd2);
+    }
+}
+
+__global__ void k_wtab(const double* __restrict__ pos, int N, WTab w)
+{
+    window_table(w, blockIdx.x, blockIdx.y, pos[2 * blockIdx.x + blockIdx.y], N, threadIdx.x, blockDim.x);
+}
+
+// V on the grid from the tables (particles in increasing order)
+__global__ void k_potfield(const int4* __restrict__ win, const double2* __restrict__ tx, const double2* __restrict__ ty,
+                           int np, int N, double* __restrict__ V)
+{
+    const size_t n2 = (size_t)N * N;
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n2; i += (size_t)gridDim.x * blockDim.x) {
+        const int x = (int)(i & (N - 1)), y = (int)(i / N);
+        double v = 0.0;
+        for (int p = 0; p < np; ++p) {
+            const int4 w = win[p];
+            const int kx = (x - w.x) & (N - 1), ky = (y - w.z) & (N - 1);
+            if (kx < w.y && ky < w.w) v += tx[(size_t)p * N + kx].x * ty[(size_t)p * N + ky].x;
+        }
+        V[i] = v;
+    }
+}
+
 // EX[p*N + i] = exp(-i kx(i) qx_p), EY[p*N + i] = exp(-i ky(i) qy_p)
 __global__ void k_ptab(const double* __restrict__ pos, cplx* __restrict__ EX, cplx* __restrict__ EY,
                        int np, int N)
@@ -1298,33 +1344,8 @@ __global__ void k_force_rows(const cplx* __restrict__ Krho, const cplx* __restri
                 for (int k = 0; k < 4; ++k) fpart[((size_t)kx * np + p0 + j) * 4 + k] = acc[4 * j + k];
 }
 
-// fl[p] = coef * sum over the row blocks b whose window flag is set, in a
-// fixed order, of the nw wave partials ppart[b][w][p] (x, y); one workgroup
-// per particle
-__global__ void k_pforce_rs(const double* __restrict__ ppart, const unsigned char* __restrict__ phit, int nblk,
-                            int nw, int np, double coef, double* __restrict__ fl)
-{
-    __shared__ double sh[2 * 16];
-    const int pp = blockIdx.x;
-    double acc[2] = {0.0, 0.0};
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-        if (!phit[(size_t)b * np + pp]) continue;
-        for (int w = 0; w < nw; ++w) {
-            acc[0] += ppart[(((size_t)b * nw + w) * np + pp) * 2];
-            acc[1] += ppart[(((size_t)b * nw + w) * np + pp) * 2 + 1];
-        }
-    }
-    block_sum<2>(acc, sh);
-    if (threadIdx.x == 0) {
-        fl[2 * pp] = coef * acc[0];
-        fl[2 * pp + 1] = coef * acc[1];
-    }
-}
-
 struct PartArgs {
-    int src;                  // 0: spectral row partials (fpart); 1: real-space block partials
-    int nblk;                 // real-space: number of row blocks
-    double coef_rs;           // real-space: 2 alpha dvol / N^2
+    int nblk, nw;             // real space: row blocks and waves per block
     int np, N, nrows, half;   // rows kx in [0,nrows); half: weight 2 for kx>0
     double coef;              // 2 alpha dvol / N^2
     double rf;                // short-range factor 384 dE pi^12 r0^12 / L^12
@@ -1366,13 +1387,8 @@ __global__ void __launch_bounds__(PSTEP_T) k_pstep(const double* __restrict__ fp
     double* dg = st + 28 * np;
     const int tid = threadIdx.x, lane = tid % 64, wv = tid / 64;
     constexpr int NW = PSTEP_T / 64;
-    // fluid forces, fixed order over rows (spectral) or row blocks (real space)
-    for (int pp = tid; pp < np && a.src == 1; pp += PSTEP_T) {
-        // reduced by k_pforce_rs into st[28 np + 8 ...]
-        fl[2 * pp] = st[28 * np + 8 + 2 * pp];
-        fl[2 * pp + 1] = st[28 * np + 8 + 2 * pp + 1];
-    }
-    for (int pp = tid; pp < np && a.src == 0; pp += PSTEP_T) {
+    // fluid forces, fixed order over rows
+    for (int pp = tid; pp < np; pp += PSTEP_T) {
         double bx = 0.0, by = 0.0;
         for (int kx = 0; kx < a.nrows; ++kx) {
             const double* f = fpart + ((size_t)kx * np + pp) * 4;
@@ -1476,6 +1492,87 @@ __global__ void __launch_bounds__(PSTEP_T) k_pstep(const double* __restrict__ fp
             dg[3] = my;
         }
     }
+}
+
+// One RK4 stage of the particles on the real-space path, one workgroup per
+// particle: its fluid force (coef times the sum over the row blocks whose
+// window flag is set, in a fixed order, of the wave partials of P3), its
+// short-range force, its update, and the window tables of its new position.
+// Another particle's new position depends only on the state at the start of
+// the stage (see k_pstep), so every workgroup forms the ones it needs itself:
+// the stage reads positions and velocities from `cur` and writes them to
+// `nxt` (pos(2np) vel(2np) each; four stages end where they began).
+// Separate force, update and table kernels took 12 us of a 512^2 stage; this
+// one 6.
+__global__ void __launch_bounds__(256) k_pstage(const double* __restrict__ ppart, const unsigned char* __restrict__ phit,
+                                                const double* __restrict__ cur, double* __restrict__ nxt,
+                                                double* __restrict__ st, PartArgs a, WTab w)
+{
+    __shared__ double sh[4 * 4];
+    __shared__ double pnew[2];
+    const int np = a.np, p = blockIdx.x, tid = threadIdx.x;
+    const double *pos = cur, *vel = cur + 2 * np;
+    double* fext = st + 4 * np;
+    double* tpos = st + 6 * np;
+    double* tvel = st + 8 * np;
+    double* ku = st + 10 * np;   // [4][2np]
+    double* kq = st + 18 * np;   // [4][2np]
+    double* frc = st + 26 * np;
+    auto newpos = [&](int i) {
+        const double q = pos[i], kqv = a.dt * vel[i], tp = a.stage == 1 ? q : tpos[i];
+        if (a.stage <= 2) return tp + 0.5 * kqv;
+        if (a.stage == 3) return tp + kqv;
+        return tp + (1.0 / 6.0) * (kq[i] + 2.0 * kq[2 * np + i] + 2.0 * kq[4 * np + i] + kqv);
+    };
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    if (tid < 64) {
+        const double px = pos[2 * p], py = pos[2 * p + 1];
+        for (int q = tid; q < np; q += 64) {
+            if (q == p) continue;
+            const double x = px - (q < p ? newpos(2 * q) : pos[2 * q]);
+            const double y = py - (q < p ? newpos(2 * q + 1) : pos[2 * q + 1]);
+            const double b = -3.0 + cos(x) + cos(y);
+            const double b2 = b * b, b4 = b2 * b2;
+            const double den = b4 * b2 * b;
+            acc[2] += -a.rf * sin(x) / den;
+            acc[3] += -a.rf * sin(y) / den;
+        }
+    }
+    for (int b = tid; b < a.nblk; b += 256) {
+        if (!phit[(size_t)b * np + p]) continue;
+        for (int v = 0; v < a.nw; ++v) {
+            acc[0] += ppart[(((size_t)b * a.nw + v) * np + p) * 2];
+            acc[1] += ppart[(((size_t)b * a.nw + v) * np + p) * 2 + 1];
+        }
+    }
+    block_sum<4>(acc, sh);
+    if (tid == 0) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int i = 2 * p + c;
+            const double F = a.coef * acc[c] + acc[2 + c] + fext[i];
+            frc[i] = F;
+            const double u = vel[i], kuv = a.dt * F / a.mass;
+            const double qn = newpos(i);
+            if (a.stage == 1) {
+                tpos[i] = pos[i];
+                tvel[i] = u;
+            }
+            const int sidx = a.stage - 1;
+            const double tv = a.stage == 1 ? u : tvel[i];
+            ku[sidx * 2 * np + i] = kuv;
+            kq[sidx * 2 * np + i] = a.dt * u;
+            double un;
+            if (a.stage <= 2) un = tv + 0.5 * kuv;
+            else if (a.stage == 3) un = tv + kuv;
+            else un = tv + (1.0 / 6.0) * (ku[i] + 2.0 * ku[2 * np + i] + 2.0 * ku[4 * np + i] + kuv);
+            nxt[i] = qn;
+            nxt[2 * np + i] = un;
+            pnew[c] = qn;
+        }
+    }
+    __syncthreads();
+    window_table(w, p, tid / 128, pnew[tid / 128], a.N, tid % 128, 128);
 }
 
 // ----------------------------------------------------------------------------
