@@ -63,18 +63,6 @@ enum PassKind { PK_P1 = 0, PK_P2, PK_P3, PK_P4, PK_PART, PK_ARG4, PK_OTHER, PK_C
 const char* kPassNames[PK_COUNT] = {"p1_rho_row", "p2_dealias_col", "p3_nonlin_row", "p4_rk4_col",
                                     "particles", "argle_update_col", "other"};
 
-int shell_of(int kx, int ky)
-{
-    // nint(sqrt(kx^2+ky^2)) (src/diagnostics.f90:341-343) by the integer
-    // identity  m(m-1) < s <= m(m+1)
-    const long long s = (long long)kx * kx + (long long)ky * ky;
-    if (s == 0) return 0;
-    long long m = (long long)std::sqrt((double)s);
-    while (m * (m + 1) < s) ++m;
-    while (m > 0 && (m - 1) * m >= s) --m;
-    return (int)m;
-}
-
 bool masked_host(int kx, int ky, int N) { return 9LL * ((long long)kx * kx + (long long)ky * ky) >= (long long)N * N; }
 
 std::mutex g_scratch_mu;
@@ -94,7 +82,6 @@ int scratch_setup(int dev)
     g_scratch_ptr[dev] = static_cast<cplx*>(ptr);
     return 0;
 }
-int ksg_host(int i, int N) { return i < N / 2 ? i : i - N; }
 
 }  // namespace
 
@@ -146,11 +133,9 @@ struct vk_gpe {
     int np_cap = 0;     // particle buffers are sized for this many particles
     int rs_part = 0;   // particle potential and force evaluated in real space inside P3
     // diagnostics
-    cplx* X[7] = {};
-    cplx* Kd[5] = {};
+    cplx *X0 = nullptr, *Kd0 = nullptr;
     cplx* Hd = nullptr;
-    int *modes = nullptr, *offs = nullptr;
-    double *dspec = nullptr, *dpart = nullptr;
+    double* hres = nullptr;   // pinned: sums and spectra of the last call
     int diag_ready = 0;
     // ensemble shape variant of this member (CfgE<N, ens_var>) and its
     // panel geometry; Hpsi holds that variant's layout only between the
@@ -294,7 +279,7 @@ void colg_launch(vk_gpe* h, int kind, int npan, Kern k, A... args)
     ev_end(h, kind);
 }
 
-// the flags (last argument: 0, 1 or 3) select a compile-time instantiation
+// the flags (last argument, 0..3) select a compile-time instantiation
 template <class C>
 void p2_launch(vk_gpe* h, cplx* Hrho, cplx* HV, const cplx* KV, cplx* Krho, const cplx* tw, Geo g, int flags)
 {
@@ -302,8 +287,8 @@ void p2_launch(vk_gpe* h, cplx* Hrho, cplx* HV, const cplx* KV, cplx* Krho, cons
     auto go = [&](auto k) { colg_launch<C, G>(h, PK_P2, h->geo.Pp, k, Hrho, HV, KV, Krho, tw, g, flags); };
     if (flags == 0) go(vk::k_p2<C, G, 0>);
     else if (flags == 1) go(vk::k_p2<C, G, 1>);
-    else if (flags == 3) go(vk::k_p2<C, G, 3>);
-    else go(vk::k_p2<C, G>);
+    else if (flags == 2) go(vk::k_p2<C, G, 2>);
+    else go(vk::k_p2<C, G, 3>);
 }
 
 // The persistent prefetching P1 (vk::k_p1xp) runs at 4096^2 when the
@@ -364,21 +349,6 @@ int fwd2d(vk_gpe* h, const cplx* X, cplx* Hs, cplx* K, int op_row, int op_col)
         row_launch<C>(h, PK_OTHER, vk::k_row_fwd<C>, X, Hs, (const cplx*)h->tw, h->geo, 0, op_row);
         constexpr int G = p4_cols<C>();
         colg_launch<C, G>(h, PK_OTHER, h->NP, vk::k_col_fwd<C, G>, (const cplx*)Hs, K, (const cplx*)h->tw, h->geo, 0,
-                          op_col);
-        return 0;
-    });
-}
-
-// forward 2D transform of a real field: only the kx >= 0 panels are stored
-// by the row pass and transformed by the column pass (the rest follows from
-// Hermitian symmetry)
-int fwd2d_half(vk_gpe* h, const cplx* X, cplx* Hs, cplx* K, int op_row, int op_col)
-{
-    return dispatch(h->N, [&](auto n) {
-        using C = CfgN<decltype(n)::value>;
-        row_launch<C>(h, PK_OTHER, vk::k_row_fwd<C>, X, Hs, (const cplx*)h->tw, h->geo, 2, op_row);
-        constexpr int G = p4_cols<C>();
-        colg_launch<C, G>(h, PK_OTHER, h->geo.Pp, vk::k_col_fwd<C, G>, (const cplx*)Hs, K, (const cplx*)h->tw, h->geo, 2,
                           op_col);
         return 0;
     });
@@ -760,84 +730,71 @@ int argle_step(vk_gpe* h, int want_res, const double* noise = nullptr)
 int diag_setup(vk_gpe* h)
 {
     if (h->diag_ready) return 0;
-    const size_t fb = f2(h) * sizeof(cplx);
-    for (auto& x : h->X) HIPCHK(hipMalloc(&x, fb));
-    for (auto& k : h->Kd) HIPCHK(hipMalloc(&k, fb));
-    HIPCHK(hipMalloc(&h->Hd, fb));
-    HIPCHK(hipMemset(h->Hd, 0, fb));
-    // retained modes grouped by shell, in the reference's loop order
-    // (kx index outer, ky index inner; src/diagnostics.f90:332-402)
-    const int N = h->N, ns = h->nshell;
-    std::vector<int> cnt(ns + 2, 0);
-    for (int i1 = 0; i1 < N; ++i1)
-        for (int i2 = 0; i2 < N; ++i2) {
-            const int kx = ksg_host(i1, N), ky = ksg_host(i2, N);
-            if (masked_host(kx, ky, N)) continue;
-            cnt[shell_of(kx, ky) + 1]++;
-        }
-    for (int m = 0; m <= ns; ++m) cnt[m + 1] += cnt[m];
-    std::vector<int> modes(cnt[ns + 1]);
-    std::vector<int> pos(cnt.begin(), cnt.end());
-    for (int i1 = 0; i1 < N; ++i1)
-        for (int i2 = 0; i2 < N; ++i2) {
-            const int kx = ksg_host(i1, N), ky = ksg_host(i2, N);
-            if (masked_host(kx, ky, N)) continue;
-            modes[pos[shell_of(kx, ky)]++] = i1 * N + i2;
-        }
-    HIPCHK(hipMalloc(&h->modes, sizeof(int) * std::max<size_t>(1, modes.size())));
-    HIPCHK(hipMalloc(&h->offs, sizeof(int) * (ns + 2)));
-    HIPCHK(hipMemcpy(h->modes, modes.data(), sizeof(int) * modes.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(h->offs, cnt.data(), sizeof(int) * (ns + 2), hipMemcpyHostToDevice));
-    HIPCHK(hipMalloc(&h->dspec, sizeof(double) * 6 * (ns + 1)));
-    HIPCHK(hipMalloc(&h->dpart, sizeof(double) * 8 * 1024));
+    if (!h->Hd) {
+        HIPCHK(hipMalloc(&h->Hd, f2(h) * sizeof(cplx)));
+        HIPCHK(hipMemset(h->Hd, 0, f2(h) * sizeof(cplx)));
+    }
     h->diag_ready = 1;
     return 0;
 }
 
-// the diagnostics' device work on h->stream: energy sums in h->dsum, the six
-// spectra in h->dspec, particle diagnostics in the particle state
-int diag_launch(vk_gpe* h)
+// Scratch of the diagnostics: fields that hold nothing between steps.  K2
+// (2 N^2 doubles) takes the spectra's column partials and the row sums.
+double* diag_part(const vk_gpe* h) { return reinterpret_cast<double*>(h->K2); }
+double* diag_rsum(const vk_gpe* h)
+{
+    return diag_part(h) + (size_t)(h->N / 3 + 1) * 6 * vk::spec_shells(h->N);
+}
+size_t diag_results(const vk_gpe* h) { return 8 + 6 * (size_t)(h->nshell + 1); }
+vk::SpecArgs spec_args(const vk_gpe* h)
+{
+    const double en = 1.0 / ((double)h->N * (double)h->N);
+    return vk::SpecArgs{h->p.alpha, h->p.g, en * en, h->N, h->nshell};
+}
+vk::DiagArgs diag_args(const vk_gpe* h, int has_v)
+{
+    return vk::DiagArgs{h->p.alpha, h->p.omega, h->p.g, (double)1e-30f, h->N, has_v};
+}
+
+// columns per workgroup of the spectra pass: workgroups of 256 threads
+template <class C> constexpr int diag_cols()
+{
+    if constexpr (vk::is_lat<C>::value) return C::G;
+    else return C::T >= 256 ? 1 : 256 / C::T;
+}
+
+// the diagnostics' device work on h->stream: the energy sums and the six
+// spectra to out (8 + 6 (nshell + 1) doubles the device can write), particle
+// diagnostics in the particle state
+int diag_launch(vk_gpe* h, double* out)
 {
     int rc = diag_setup(h);
     if (rc) return rc;
     if ((rc = ensure_any(h))) return rc;
     const double sc = scale_of(h);
     const int pl = h->hstate == 2 ? 1 : 0;
-    cplx **X = h->X, **Kd = h->Kd;
-    // psi, d_x psi, d_y psi
-    if ((rc = row_inv(h, h->Hpsi, X[0], pl, 0, sc))) return rc;
-    if ((rc = row_inv(h, h->Hpsi, X[1], pl, 1, sc))) return rc;
-    if ((rc = col_inv(h, h->K0, h->Hd, pl, 2))) return rc;
-    if ((rc = row_inv(h, h->Hd, X[2], pl, 0, sc))) return rc;
-    // rho-hat (dealiased) -> Kd[4]; P_G rho -> X[3].  rho, P_G rho, V and
-    // the w and q fields are real: only their kx >= 0 columns are
-    // transformed, the rest is their Hermitian mirror.
-    const int Kp = h->TC * h->geo.Pp;
-    if ((rc = fwd2d_half(h, X[0], h->Hd, Kd[4], 1, 1))) return rc;
-    if ((rc = col_inv(h, Kd[4], h->Hd, 2, 0))) return rc;
-    if ((rc = row_inv(h, h->Hd, X[3], 2, 0, sc))) return rc;
     const int parts = h->have_part && h->p.np > 0;
-    if (parts) {
-        particle_kv(h, Kp);
-        if ((rc = col_inv(h, h->KV, h->Hd, 2, 0))) return rc;
-        if ((rc = row_inv(h, h->Hd, X[4], 2, 0, sc))) return rc;
-    }
-    vk::DiagArgs da{h->p.alpha, h->p.omega, h->p.g, (double)1e-30f, h->N, parts};
-    const int nb = 1024;
-    hipLaunchKernelGGL(vk::k_diag_x, dim3(nb), dim3(256), 0, h->stream, (const cplx*)X[0], (const cplx*)X[1],
-                       (const cplx*)X[2], (const cplx*)X[3], (const cplx*)X[4], X[1], X[2], X[5], X[6], da, h->dpart);
-    hipLaunchKernelGGL(vk::k_reduce_fixed, dim3(1), dim3(256), 0, h->stream, (const double*)h->dpart, nb, 8, h->dsum);
-    // spectra: FFT of w_x, w_y, q_x, q_y (kx >= 0 halves)
-    if ((rc = fwd2d_half(h, X[1], h->Hd, Kd[0], 0, 0))) return rc;
-    if ((rc = fwd2d_half(h, X[2], h->Hd, Kd[1], 0, 0))) return rc;
-    if ((rc = fwd2d_half(h, X[5], h->Hd, Kd[2], 0, 0))) return rc;
-    if ((rc = fwd2d_half(h, X[6], h->Hd, Kd[3], 0, 0))) return rc;
-    const double en = 1.0 / ((double)h->N * (double)h->N);
-    vk::SpecArgs sa{h->p.alpha, h->p.g, en * en, h->N, h->nshell};
-    hipLaunchKernelGGL(vk::k_spectra, dim3(h->nshell + 1), dim3(256), 0, h->stream, (const int*)h->modes,
-                       (const int*)h->offs, (const cplx*)Kd[0], (const cplx*)Kd[1], (const cplx*)Kd[2],
-                       (const cplx*)Kd[3], (const cplx*)Kd[4], (const cplx*)h->K0, sa, h->dspec);
-    if (parts) particle_forces(h, Kd[4], Kp, 1, 0);
+    const int Kp = h->TC * h->geo.Pp;
+    cplx *H1 = h->HN, *H2 = h->Xs;
+    if ((rc = col_inv(h, h->K0, h->Hd, pl, 2))) return rc;   // i ky kpsi
+    if (parts) particle_kv(h, Kp);
+    rc = dispatch(h->N, [&](auto n) {
+        using C = CfgN<decltype(n)::value>;
+        using C1 = std::conditional_t<(C::N >= 2048), CfgTR1<C>, C>;
+        const cplx* tw = h->tw;
+        row_launch<C1>(h, PK_OTHER, vk::k_p1d<C1>, (const cplx*)h->Hpsi, h->Hrho, tw, h->geo, pl, sc);
+        p2_launch<C>(h, h->Hrho, h->HV, (const cplx*)h->KV, h->Krho, tw, h->geo, parts ? 3 : 2);
+        row_launch<C1>(h, PK_OTHER, vk::k_diag_row<C1>, (const cplx*)h->Hpsi, (const cplx*)h->Hd, (const cplx*)h->Hrho,
+                       (const cplx*)h->HV, H1, H2, tw, h->geo, pl, sc, diag_args(h, parts), diag_rsum(h));
+        constexpr int G = diag_cols<C>();
+        colg_launch<C, G>(h, PK_OTHER, h->geo.Pp, vk::k_diag_col<C, G>, H1, (const cplx*)H2,
+                          (const cplx*)h->K0, (const cplx*)h->Krho, tw, h->geo, diag_part(h));
+        return 0;
+    });
+    if (rc) return rc;
+    hipLaunchKernelGGL(vk::k_spec_reduce, dim3(h->nshell / 64 + 1, 7), dim3(64 * vk::SPEC_G), 0, h->stream,
+                       (const double*)diag_part(h), (const double*)diag_rsum(h), spec_args(h), out);
+    if (parts) particle_forces(h, h->Krho, Kp, 1, 0);
     return 0;
 }
 
@@ -878,17 +835,16 @@ void diag_final(const vk_gpe* h, const double* s, const double* sp, const double
 
 int diagnostics(vk_gpe* h, double* scal, double* spec, double* pscal)
 {
-    int rc = diag_launch(h);
+    // results in pinned memory, which the last kernel writes
+    if (!h->hres) HIPCHK(hipHostMalloc((void**)&h->hres, diag_results(h) * sizeof(double)));
+    int rc = diag_launch(h, h->hres);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipGetLastError());
-    double s[8], dg[4] = {};
-    HIPCHK(hipMemcpy(s, h->dsum, sizeof(s), hipMemcpyDeviceToHost));
-    std::vector<double> sp(6 * (h->nshell + 1));
-    HIPCHK(hipMemcpy(sp.data(), h->dspec, sizeof(double) * sp.size(), hipMemcpyDeviceToHost));
+    double dg[4] = {};
     if (h->have_part && h->p.np > 0)
         HIPCHK(hipMemcpy(dg, h->pst + 28 * h->p.np, sizeof(dg), hipMemcpyDeviceToHost));
-    diag_final(h, s, sp.data(), dg, scal, spec, pscal);
+    diag_final(h, h->hres, h->hres + 8, dg, scal, spec, pscal);
     return 0;
 }
 
@@ -1067,12 +1023,9 @@ void vk_gpe_destroy(vk_gpe* h)
         if (h->Vx) hipFree(h->Vx);
         if (h->pst) hipFree(h->pst);
     }
-    for (auto x : h->X) if (x) hipFree(x);
-    for (auto k : h->Kd) if (k) hipFree(k);
-    if (h->modes) hipFree(h->modes);
-    if (h->offs) hipFree(h->offs);
-    if (h->dspec) hipFree(h->dspec);
-    if (h->dpart) hipFree(h->dpart);
+    if (h->X0) hipFree(h->X0);
+    if (h->Kd0) hipFree(h->Kd0);
+    if (h->hres) hipHostFree(h->hres);
     if (h->part) hipFree(h->part);
     if (h->dsum) hipFree(h->dsum);
     if (h->e1R) hipFree(h->e1R);
@@ -1090,7 +1043,7 @@ static int ensure_hdy(vk_gpe* h);
 
 static int need_x0(vk_gpe* h)
 {
-    if (!h->X[0]) HIPCHK(hipMalloc(&h->X[0], f2(h) * sizeof(cplx)));
+    if (!h->X0) HIPCHK(hipMalloc(&h->X0, f2(h) * sizeof(cplx)));
     if (!h->Hd) {
         HIPCHK(hipMalloc(&h->Hd, f2(h) * sizeof(cplx)));
         HIPCHK(hipMemset(h->Hd, 0, f2(h) * sizeof(cplx)));
@@ -1100,7 +1053,7 @@ static int need_x0(vk_gpe* h)
 
 static int set_from_x0(vk_gpe* h, int flags)
 {
-    int rc = fwd2d(h, h->X[0], h->Hd, h->K0, 0, 0);
+    int rc = fwd2d(h, h->X0, h->Hd, h->K0, 0, 0);
     if (rc) return rc;
     h->hstate = 0;
     if (flags & VK_SYNC_DEALIAS) {
@@ -1118,7 +1071,7 @@ int vk_gpe_set_psi(vk_gpe* h, const double* psi, int flags)
     if (rc) return rc;
     // stream-ordered: a device-to-device hipMemcpy does not block the host and
     // is not ordered against this non-blocking stream
-    HIPCHK(hipMemcpyAsync(h->X[0], psi, f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
+    HIPCHK(hipMemcpyAsync(h->X0, psi, f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
     return set_from_x0(h, flags);
 }
 
@@ -1138,10 +1091,10 @@ int vk_gpe_get_psi(vk_gpe* h, double* psi, double* kpsi)
     if (psi) {
         if ((rc = need_x0(h))) return rc;
         if ((rc = ensure_any(h))) return rc;
-        if ((rc = row_inv(h, h->Hpsi, h->X[0], h->hstate == 2 ? 1 : 0, 0, scale_of(h)))) return rc;
+        if ((rc = row_inv(h, h->Hpsi, h->X0, h->hstate == 2 ? 1 : 0, 0, scale_of(h)))) return rc;
         HIPCHK(hipStreamSynchronize(h->stream));
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(psi, h->X[0], f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
+        HIPCHK(hipMemcpyAsync(psi, h->X0, f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
     }
     if (kpsi) {
@@ -1226,8 +1179,8 @@ static int particle_potential(vk_gpe* h)
 {
     const double pi = 4.0 * std::atan(1.0);
     const double L = 2.0 * pi, dx = L / h->N, c1 = 2 * pi / (2.0 * L);
-    hipLaunchKernelGGL(vk::k_pot_x, dim3(1024), dim3(256), 0, h->stream, h->X[0], h->N, dx, c1, h->p.V0, h->p.d);
-    int rc = fwd2d(h, h->X[0], h->Hd, h->Vhat, 0, 1);
+    hipLaunchKernelGGL(vk::k_pot_x, dim3(1024), dim3(256), 0, h->stream, h->X0, h->N, dx, c1, h->p.V0, h->p.d);
+    int rc = fwd2d(h, h->X0, h->Hd, h->Vhat, 0, 1);
     if (rc) return rc;
     h->have_part = 1;
     return 0;
@@ -1482,21 +1435,21 @@ int vk_fft2d(vk_gpe* h, int dir, const double* in, double* out)
     if (!h || !in || !out || (dir != -1 && dir != 1)) return fail(VK_ERR_ARG, "fft2d: bad arguments");
     int rc = need_x0(h);
     if (rc) return rc;
-    if (!h->Kd[0]) HIPCHK(hipMalloc(&h->Kd[0], f2(h) * sizeof(cplx)));
+    if (!h->Kd0) HIPCHK(hipMalloc(&h->Kd0, f2(h) * sizeof(cplx)));
     const size_t fb = f2(h) * sizeof(cplx);
     if (dir < 0) {
-        HIPCHK(hipMemcpy(h->X[0], in, fb, hipMemcpyHostToDevice));
-        if ((rc = fwd2d(h, h->X[0], h->Hd, h->Kd[0], 0, 0))) return rc;
+        HIPCHK(hipMemcpy(h->X0, in, fb, hipMemcpyHostToDevice));
+        if ((rc = fwd2d(h, h->X0, h->Hd, h->Kd0, 0, 0))) return rc;
         HIPCHK(hipStreamSynchronize(h->stream));
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpy(out, h->Kd[0], fb, hipMemcpyDeviceToHost));
+        HIPCHK(hipMemcpy(out, h->Kd0, fb, hipMemcpyDeviceToHost));
     } else {
-        HIPCHK(hipMemcpy(h->Kd[0], in, fb, hipMemcpyHostToDevice));
-        if ((rc = col_inv(h, h->Kd[0], h->Hd, 0, 0))) return rc;
-        if ((rc = row_inv(h, h->Hd, h->X[0], 0, 0, scale_of(h)))) return rc;
+        HIPCHK(hipMemcpy(h->Kd0, in, fb, hipMemcpyHostToDevice));
+        if ((rc = col_inv(h, h->Kd0, h->Hd, 0, 0))) return rc;
+        if ((rc = row_inv(h, h->Hd, h->X0, 0, 0, scale_of(h)))) return rc;
         HIPCHK(hipStreamSynchronize(h->stream));
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpy(out, h->X[0], fb, hipMemcpyDeviceToHost));
+        HIPCHK(hipMemcpy(out, h->X0, fb, hipMemcpyDeviceToHost));
     }
     return 0;
 }
@@ -1557,7 +1510,7 @@ int vk_gpe_set_ic_vortices(vk_gpe* h, int nv, const double* xs, const double* ys
         HIPCHK(hipMemcpy(dy, ys, sizeof(double) * nv, hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(dq, qs, sizeof(int) * nv, hipMemcpyHostToDevice));
     }
-    hipLaunchKernelGGL(vk::k_ic, dim3(2048), dim3(256), 0, h->stream, h->X[0], h->N, nv, (const double*)dx,
+    hipLaunchKernelGGL(vk::k_ic, dim3(2048), dim3(256), 0, h->stream, h->X0, h->N, nv, (const double*)dx,
                        (const double*)dy, (const int*)dq, h->p.xi, nimg);
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipGetLastError());
@@ -2031,80 +1984,44 @@ int col_inv_var(vk_gpe* h, int var)
 // Diagnostics of the members hs (all of size C::N, all with Hpsi in layout
 // pl: 1 retained panels, 0 all panels) as batched launches on stream st:
 // the single-field pipeline (diag_launch) with blockIdx.y selecting the
-// member, so each member gets bit for bit its single-field result.  Member
-// i's sums go to sums[i] (8 doubles) and its spectra to spec[i].
-// tab: device memory for the operand tables, ens_diag_tab_bytes(hs.size());
+// member.  Its sums run per row, column and shell, whatever the workgroup
+// shape, so each member gets bit for bit its single-field result.  Member
+// i's sums and spectra go to out[i].
+// tab: device memory for the operand table, ens_diag_tab_bytes(hs.size());
 // htab: pinned host memory of the same size, not rewritten before the
 // stream has passed the copy.
-constexpr int kDiagPairSteps = 16;
-size_t ens_diag_tab_bytes(size_t n)
-{
-    return ((kDiagPairSteps * n * sizeof(vk::BPair) + 255) / 256) * 256 + n * sizeof(vk::DiagB);
-}
+size_t ens_diag_tab_bytes(size_t n) { return n * sizeof(vk::DiagB); }
 
 template <class C>
 int ens_diag_group(const std::vector<vk_gpe*>& hs, int pl, hipStream_t st, void* tab, void* htab,
-                   const std::vector<double*>& sums, const std::vector<double*>& spec)
+                   const std::vector<double*>& out)
 {
     const int n = (int)hs.size();
     const vk_gpe* h0 = hs[0];
     const Geo g = h0->geo;
     const cplx* tw = h0->tw;   // the same table in every member of this size
     const double sc = scale_of(h0);
-    const size_t dd_off = ((kDiagPairSteps * n * sizeof(vk::BPair) + 255) / 256) * 256;
-    vk::BPair* pairs = static_cast<vk::BPair*>(htab);
-    vk::DiagB* db = reinterpret_cast<vk::DiagB*>(static_cast<char*>(htab) + dd_off);
+    vk::DiagB* db = static_cast<vk::DiagB*>(htab);
     for (int i = 0; i < n; ++i) {
-        vk_gpe* h = hs[i];
-        cplx** X = h->X;
-        cplx** Kd = h->Kd;
-        const vk::BPair row[kDiagPairSteps] = {
-            {h->Hpsi, X[0]}, {h->Hpsi, X[1]}, {h->K0, h->Hd}, {h->Hd, X[2]},   // psi, d_x psi, d_y psi
-            {X[0], h->Hd}, {h->Hd, Kd[4]},                                     // rho-hat, dealiased
-            {Kd[4], h->Hd}, {h->Hd, X[3]},                                     // P_G rho
-            {X[1], h->Hd}, {h->Hd, Kd[0]}, {X[2], h->Hd}, {h->Hd, Kd[1]},       // w, q transforms
-            {X[5], h->Hd}, {h->Hd, Kd[2]}, {X[6], h->Hd}, {h->Hd, Kd[3]}};
-        for (int k = 0; k < kDiagPairSteps; ++k) pairs[(size_t)k * n + i] = row[k];
-        vk::DiagB& d = db[i];
-        d.psi = X[0]; d.D1 = X[1]; d.D2 = X[2]; d.PR = X[3];
-        d.W1 = X[1]; d.W2 = X[2]; d.Q1 = X[5]; d.Q2 = X[6];
-        d.part = h->dpart;
-        d.sums = sums[i];
-        d.spec = spec[i];
-        d.KW1 = Kd[0]; d.KW2 = Kd[1]; d.KQ1 = Kd[2]; d.KQ2 = Kd[3]; d.KR = Kd[4]; d.KP = h->K0;
-        d.da = vk::DiagArgs{h->p.alpha, h->p.omega, h->p.g, (double)1e-30f, h->N, 0};
-        const double en = 1.0 / ((double)h->N * (double)h->N);
-        d.sa = vk::SpecArgs{h->p.alpha, h->p.g, en * en, h->N, h->nshell};
+        const vk_gpe* h = hs[i];
+        db[i] = vk::DiagB{h->Hpsi, h->K0, h->Hd, h->Hrho, h->Krho, h->HN, h->Xs, diag_rsum(h), diag_part(h), out[i],
+                          diag_args(h, 0), spec_args(h)};
     }
-    char* base = static_cast<char*>(tab);
-    vk::BPair* dp = reinterpret_cast<vk::BPair*>(base);
-    vk::DiagB* dd = reinterpret_cast<vk::DiagB*>(base + dd_off);
+    const vk::DiagB* dd = static_cast<const vk::DiagB*>(tab);
     HIPCHK(hipMemcpyAsync(tab, htab, ens_diag_tab_bytes(n), hipMemcpyHostToDevice, st));
     const size_t rl = (size_t)C::TR * C::ROWRS * sizeof(double), cl = (size_t)C::TC * C::COLRS * sizeof(double);
-    set_lds(vk::k_row_inv_b<C>, rl);
-    set_lds(vk::k_row_fwd_b<C>, rl);
-    set_lds(vk::k_col_inv_b<C>, cl);
-    set_lds(vk::k_col_fwd_b<C>, cl);
+    set_lds(vk::k_p1d_b<C>, rl);
+    set_lds(vk::k_diag_row_b<C>, rl);
+    set_lds(vk::k_diag_dy_b<C>, cl);
+    set_lds(vk::k_p2d_b<C>, cl);
+    set_lds(vk::k_diag_col_b<C>, cl);
     const dim3 rg(C::N / C::TR, n), rb(C::ROWT), cb(C::COLT);
-    const int ncl = pl == 1 ? g.Pp + g.Pn : C::NP;
-    auto P = [&](int k) { return (const vk::BPair*)(dp + (size_t)k * n); };
-    hipLaunchKernelGGL(vk::k_row_inv_b<C>, rg, rb, rl, st, P(0), tw, g, pl, 0, sc);
-    hipLaunchKernelGGL(vk::k_row_inv_b<C>, rg, rb, rl, st, P(1), tw, g, pl, 1, sc);
-    hipLaunchKernelGGL(vk::k_col_inv_b<C>, dim3(ncl, n), cb, cl, st, P(2), tw, g, pl, 2);
-    hipLaunchKernelGGL(vk::k_row_inv_b<C>, rg, rb, rl, st, P(3), tw, g, pl, 0, sc);
-    hipLaunchKernelGGL(vk::k_row_fwd_b<C>, rg, rb, rl, st, P(4), tw, g, 2, 1);
-    hipLaunchKernelGGL(vk::k_col_fwd_b<C>, dim3(g.Pp, n), cb, cl, st, P(5), tw, g, 2, 1);
-    hipLaunchKernelGGL(vk::k_col_inv_b<C>, dim3(g.Pp, n), cb, cl, st, P(6), tw, g, 2, 0);
-    hipLaunchKernelGGL(vk::k_row_inv_b<C>, rg, rb, rl, st, P(7), tw, g, 2, 0, sc);
-    const int nb = 1024;   // as the single-field pass: the same partial sums
-    hipLaunchKernelGGL(vk::k_diag_x_b, dim3(nb, n), dim3(256), 0, st, (const vk::DiagB*)dd);
-    hipLaunchKernelGGL(vk::k_reduce_fixed_b, dim3(n), dim3(256), 0, st, (const vk::DiagB*)dd, nb);
-    for (int k = 8; k < kDiagPairSteps; k += 2) {
-        hipLaunchKernelGGL(vk::k_row_fwd_b<C>, rg, rb, rl, st, P(k), tw, g, 2, 0);
-        hipLaunchKernelGGL(vk::k_col_fwd_b<C>, dim3(g.Pp, n), cb, cl, st, P(k + 1), tw, g, 2, 0);
-    }
-    hipLaunchKernelGGL(vk::k_spectra_b, dim3(h0->nshell + 1, n), dim3(256), 0, st, (const int*)h0->modes,
-                       (const int*)h0->offs, (const vk::DiagB*)dd);
+    hipLaunchKernelGGL(vk::k_diag_dy_b<C>, dim3(pl == 1 ? g.Pp + g.Pn : C::NP, n), cb, cl, st, dd, tw, g, pl);
+    hipLaunchKernelGGL(vk::k_p1d_b<C>, rg, rb, rl, st, dd, tw, g, pl, sc);
+    hipLaunchKernelGGL(vk::k_p2d_b<C>, dim3(g.Pp, n), cb, cl, st, dd, tw, g);
+    hipLaunchKernelGGL(vk::k_diag_row_b<C>, rg, rb, rl, st, dd, tw, g, pl, sc);
+    hipLaunchKernelGGL(vk::k_diag_col_b<C>, dim3(g.Pp, n), cb, cl, st, dd, tw, g);
+    hipLaunchKernelGGL(vk::k_spec_reduce_b, dim3(h0->nshell / 64 + 1, 7, n), dim3(64 * vk::SPEC_G), 0, st, dd);
     return 0;
 }
 
@@ -2385,7 +2302,7 @@ int vk_ens_diagnostics_all(vk_ens* e, double* scal, double* spec)
     HIPCHK(hipStreamSynchronize(e->stream));
     const size_t nreal = e->h.size();
     std::vector<size_t> offs(nreal + 1, 0);
-    for (size_t r = 0; r < nreal; ++r) offs[r + 1] = offs[r] + 8 + 6 * (size_t)(e->h[r]->nshell + 1);
+    for (size_t r = 0; r < nreal; ++r) offs[r + 1] = offs[r] + diag_results(e->h[r]);
     const size_t need = offs[nreal];
     if (need > e->nstage) {
         if (e->hstage) hipHostFree(e->hstage);
@@ -2424,11 +2341,10 @@ int vk_ens_diagnostics_all(vk_ens* e, double* scal, double* spec)
     size_t toff = 0;
     for (auto& kv : groups) {
         std::vector<vk_gpe*> hs;
-        std::vector<double*> su, sp;
+        std::vector<double*> res;
         for (int r : kv.second) {
             hs.push_back(e->h[r]);
-            su.push_back(e->dstage + offs[r]);
-            sp.push_back(e->dstage + offs[r] + 8);
+            res.push_back(e->dstage + offs[r]);
         }
         char* etab = static_cast<char*>(e->dtab) + toff;
         char* ehtab = static_cast<char*>(e->htab) + toff;
@@ -2436,8 +2352,8 @@ int vk_ens_diagnostics_all(vk_ens* e, double* scal, double* spec)
         char* tab = static_cast<char*>(e->dtab) + toff;
         char* htab = static_cast<char*>(e->htab) + toff;
         toff += (ens_diag_tab_bytes(hs.size()) + 255) / 256 * 256;
-        int rc = dispatch(kv.first.first, [&](auto nn) {
-            using C = vk::Cfg<decltype(nn)::value>;
+        int rc = dispatch_var(kv.first.first, 0, [&](auto shape) {
+            using C = decltype(shape);
             if (kv.first.second == 0) {
                 // Hpsi stale (a member in its second shape): IFFT_y(K0) on
                 // all panels in the single-field layout, as ensure_any does
@@ -2450,7 +2366,7 @@ int vk_ens_diagnostics_all(vk_ens* e, double* scal, double* spec)
                                    (const vk::BPair*)etab, (const cplx*)hs[0]->tw, hs[0]->geo, 0, 0);
                 for (auto h : hs) h->hstate = 1;
             }
-            return ens_diag_group<C>(hs, hs[0]->hstate == 2 ? 1 : 0, e->stream, tab, htab, su, sp);
+            return ens_diag_group<C>(hs, hs[0]->hstate == 2 ? 1 : 0, e->stream, tab, htab, res);
         });
         if (rc) return rc;
         for (auto h : hs)

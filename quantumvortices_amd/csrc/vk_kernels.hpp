@@ -270,16 +270,18 @@ __global__ void k_dealias(cplx* __restrict__ K, int N)
 // ----------------------------------------------------------------------------
 
 // P1 after its loads: v holds the conjugated Hpsi row points of this thread
-template <class C, class W>
+template <class C, bool XS, class W>
 __device__ __forceinline__ void p1_core(cplx (&v)[C::S], double* lg, int t, int y, int pidx0, int c,
                                         cplx* __restrict__ Hrho, const W& w_, const Geo& g,
                                         double scale, cplx* __restrict__ Xpsi)
 {
     constexpr int N = C::N, S = C::S, T = C::T, TC = C::TC;
     fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
-    cplx* xr = Xpsi + (size_t)y * N;
+    if constexpr (XS) {
+        cplx* xr = Xpsi + (size_t)y * N;
 #pragma unroll
-    for (int s = 0; s < S; ++s) xr[t + T * s] = rmul(scale, conjc(v[s]));
+        for (int s = 0; s < S; ++s) xr[t + T * s] = rmul(scale, conjc(v[s]));
+    }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const double a = scale * v[s].x, b = scale * v[s].y;   // conj does not change |.|
@@ -296,8 +298,8 @@ __device__ __forceinline__ void p1_core(cplx (&v)[C::S], double* lg, int t, int 
 // P1 (row): psi row from Hpsi (inverse along x, times 1/N^2), rho = |psi|^2,
 // forward along x, keep kx >= 0 retained panels (rho is real).  The psi row
 // is stored in x-space (Xpsi[y*N + x]) for P3, which then needs no transform
-// of its own for psi.
-template <class C>
+// of its own for psi; the diagnostics do without (XS false).
+template <class C, bool XS = true>
 __device__ __forceinline__ void p1_body(int blk_, int nblk_, const cplx* __restrict__ Hpsi, cplx* __restrict__ Hrho,
                                                 const cplx* __restrict__ tw, Geo g, int psi_pmode,
                                                 double scale, cplx* __restrict__ Xpsi)
@@ -313,7 +315,7 @@ __device__ __forceinline__ void p1_body(int blk_, int nblk_, const cplx* __restr
     const auto w_ = twiddles<C>(tw, t);
 #pragma unroll
     for (int s = 0; s < S; ++s) v[s] = panel_stored(VK_PANEL(s), NP, g, psi_pmode) ? conjc(v[s]) : czero();
-    p1_core<C>(v, lg, t, y, pidx0, c, Hrho, w_, g, scale, Xpsi);
+    p1_core<C, XS>(v, lg, t, y, pidx0, c, Hrho, w_, g, scale, Xpsi);
 }
 
 template <class C>
@@ -432,7 +434,7 @@ __global__ void __launch_bounds__(C::ROWT) k_p1xp(const cplx* __restrict__ Hpsi,
         // all reads are done before the next copies overwrite the slots
         __syncthreads();
         if (k + 1 < K) prefetch(xcd * R8 + j + (k + 1) * G8);
-        p1_core<C>(v, lg, t, y, pidx0, c, Hrho, tw, g, scale, Xpsi);
+        p1_core<C, true>(v, lg, t, y, pidx0, c, Hrho, tw, g, scale, Xpsi);
     }
 }
 
@@ -1009,51 +1011,135 @@ struct DiagArgs {
     int has_v;
 };
 
-// x-space pass: momentum, energies, norm partial sums (in the reference's
-// :84-207 quantities before the final factors) and the fields
-//   w = 2 alpha Im(psi* grad psi)/(|psi|+smlnum) -> W1, W2
-//   q = Re(psi* grad psi)/(|psi|+smlnum)          -> Q1, Q2   (:263-317)
-// sums: 0 momx 1 momy 2 egrad 3 echem 4 eintr 5 eppot 6 norm 7 unused
-__device__ __forceinline__ void diag_x_body(int blk, int nblk, const cplx* __restrict__ psi,
-                                            const cplx* __restrict__ D1, const cplx* __restrict__ D2,
-                                            const cplx* __restrict__ PR, const cplx* __restrict__ V,
-                                            cplx* __restrict__ W1, cplx* __restrict__ W2, cplx* __restrict__ Q1,
-                                            cplx* __restrict__ Q2, DiagArgs a, double* __restrict__ part)
+// Sums over a row of nv <= 8 values per point group: thread t of the row's T
+// holds x[]; out[i] = the sum over t in a fixed tree (neighbour pairs, then
+// pairs of pairs, ...), the same in every workgroup shape.  sh: nv * T
+// doubles of LDS of this row.  Every thread of the workgroup calls it.
+template <int NV, int T>
+__device__ __forceinline__ void row_sum(const double (&x)[NV], double* sh, int t, double* __restrict__ out)
 {
-    __shared__ double sh[8 * 16];
-    double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    const size_t n2 = (size_t)a.N * a.N;
-    for (size_t i = blk * (size_t)blockDim.x + threadIdx.x; i < n2; i += (size_t)nblk * blockDim.x) {
-        const cplx ps = psi[i], d1 = D1[i], d2 = D2[i], pr = PR[i];
-        const cplx cp = conjc(ps);
-        const cplx a1 = cmul(cp, d1), a2 = cmul(cp, d2);
-        const double apsi = hypot(ps.x, ps.y);
-        const double ap2 = apsi * apsi;
-        acc[0] += a1.y;
-        acc[1] += a2.y;
-        const double h1 = hypot(d1.x, d1.y), h2 = hypot(d2.x, d2.y);
-        acc[2] += a.alpha * (h1 * h1 + h2 * h2);
-        acc[3] += a.omega * ap2;
-        acc[4] += 0.5 * a.g * hypot(pr.x, pr.y) * ap2;
-        if (a.has_v) acc[5] += V[i].x * pr.x;
-        acc[6] += ap2;
-        const double rl = apsi + a.smlnum;
-        W1[i] = mk(2.0 * a.alpha * (a1.y / rl), 0.0);
-        W2[i] = mk(2.0 * a.alpha * (a2.y / rl), 0.0);
-        Q1[i] = mk(a1.x / rl, 0.0);
-        Q2[i] = mk(a2.x / rl, 0.0);
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) sh[i * T + t] = x[i];
+#pragma unroll
+    for (int h = 1; h < T; h *= 2) {
+        lds_barrier();
+        if (t % (2 * h) == 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) sh[i * T + t] += sh[i * T + t + h];
+        }
     }
-    block_sum<8>(acc, sh);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < 8; ++k) part[(size_t)blk * 8 + k] = acc[k];
+    lds_barrier();
+    if (t == 0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) out[i] = sh[i * T];
+    }
 }
 
-__global__ void k_diag_x(const cplx* __restrict__ psi, const cplx* __restrict__ D1,
-                         const cplx* __restrict__ D2, const cplx* __restrict__ PR,
-                         const cplx* __restrict__ V, cplx* __restrict__ W1, cplx* __restrict__ W2,
-                         cplx* __restrict__ Q1, cplx* __restrict__ Q2, DiagArgs a, double* __restrict__ part)
+// Row pass of the diagnostics (src/diagnostics.f90:54-317): from the rows of
+// Hpsi, Hdy = IFFT_y(i ky kpsi), Hrhod (and HV) the x-space psi, d_x psi,
+// d_y psi, P_G rho (and V), never stored; per row the sums
+//   0 momx 1 momy 2 egrad 3 echem 4 eintr 5 eppot 6 norm   (rsum[y][8])
+// and the transforms along x of two pairs of real fields, packed as complex
+// ones, on the retained panels: H1: w_x + i q_x, H2: w_y + i q_y with
+//   w = 2 alpha Im(psi* grad psi)/(|psi| + smlnum),
+//   q = Re(psi* grad psi)/(|psi| + smlnum)
+// (this pairing lets each direction's pair go before the next one's gradient
+// is formed; w_x with w_y would hold 64 registers more and spill 240).
+// Six transforms per row.  4096^2: 0.8 GB against the 5.4 GB of separate
+// transforms and a pointwise pass over x-space arrays (1.5 ms).
+template <class C>
+__device__ __forceinline__ void diag_row_body(int blk_, int nblk_, const cplx* __restrict__ Hpsi,
+                                              const cplx* __restrict__ Hdy, const cplx* __restrict__ Hrhod,
+                                              const cplx* __restrict__ HV, cplx* __restrict__ H1,
+                                              cplx* __restrict__ H2, const cplx* __restrict__ tw, Geo g, int pl,
+                                              double scale, const DiagArgs& a, double* __restrict__ rsum)
 {
-    diag_x_body(blockIdx.x, gridDim.x, psi, D1, D2, PR, V, W1, W2, Q1, Q2, a, part);
+    VK_ROW_SETUP(C)
+    const auto w_ = twiddles<C>(tw, t);
+    cplx v[S], ps[S];
+    const brsrc rH = mkbuf(Hpsi, N), rD = mkbuf(Hdy, N), rR = mkbuf(Hrhod, N);
+    // Offsets are formed anew for each load and store phase (from an opaque
+    // copy of the panel index), not kept across the transforms.
+    auto again = [&](int q) {
+        if constexpr (!is_lat<C>::value) asm volatile("" : "+v"(q));
+        return q;
+    };
+    double acc[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    // a row of a field stored on the panels of mode pl, conjugated for the
+    // inverse; dx: times i kx
+    auto load = [&](brsrc rb, bool dx) {
+        const int p0 = again(pidx0);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int pp = p0 + (T / TC) * s;
+            v[s] = bld(rb, boff(hoff<C>(pp, y, c), panel_stored(pp, NP, g, pl)));
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            cplx z = v[s];
+            if (dx) {
+                const double kk = (double)ksg(t + T * s, N);
+                z = mk(-kk * z.y, kk * z.x);
+            }
+            v[s] = conjc(z);
+        }
+    };
+    load(rH, false);
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+#pragma unroll
+    for (int s = 0; s < S; ++s) ps[s] = rmul(scale, conjc(v[s]));
+    // P_G rho + i V from the kx >= 0 halves
+    const int Kp = TC * g.Pp, t0 = again(t);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int kxi = t0 + T * s;
+        const int km = kxi >= Kp ? N - kxi : kxi;
+        const unsigned o = boff(hoff<C>(km / TC, y, km % TC), kxi < Kp || kxi > N - Kp);
+        cplx z = bld(rR, o);
+        cplx zv = a.has_v ? bld(mkbuf(HV, N), o) : czero();
+        if (kxi > N - Kp) {
+            z = conjc(z);
+            zv = conjc(zv);
+        }
+        v[s] = conjc(mk(z.x - zv.y, z.y + zv.x));
+    }
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const double pr = scale * v[s].x, ap2 = ps[s].x * ps[s].x + ps[s].y * ps[s].y;
+        acc[3] += a.omega * ap2;
+        acc[4] += 0.5 * a.g * fabs(pr) * ap2;
+        if (a.has_v) acc[5] += (-scale * v[s].y) * pr;
+        acc[6] += ap2;
+    }
+#pragma unroll
+    for (int dir = 0; dir < 2; ++dir) {
+        load(dir == 0 ? rH : rD, dir == 0);
+        fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const cplx d = rmul(scale, conjc(v[s]));
+            const cplx z = cmul(conjc(ps[s]), d);
+            acc[dir] += z.y;
+            acc[2] += a.alpha * (d.x * d.x + d.y * d.y);
+            double px = ps[s].x;
+            if constexpr (!is_lat<C>::value) asm volatile("" : "+v"(px));   // formed twice, not kept
+            const double inv = 1.0 / (sqrt(px * px + ps[s].y * ps[s].y) + a.smlnum);
+            v[s] = mk(2.0 * a.alpha * (z.y * inv), z.x * inv);
+            // one point's square root and division at a time
+            if constexpr (!is_lat<C>::value) __builtin_amdgcn_sched_barrier(0);
+        }
+        fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+        const brsrc ro = mkbuf(dir == 0 ? H1 : H2, N);
+        const int p0 = again(pidx0);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int pp = p0 + (T / TC) * s;
+            bst(ro, boff(hoff<C>(pp, y, c), panel_stored(pp, NP, g, 1)), v[s]);
+        }
+    }
+    row_sum<7, T>(acc, lg, t, rsum + 8 * (size_t)y);
 }
 
 struct SpecArgs {
@@ -1061,58 +1147,210 @@ struct SpecArgs {
     int N, nshell;
 };
 
-// Shell binning: one workgroup per shell m over the list of retained modes
-// in that shell (idx = kx*N + ky), fixed-order reduction.
-// spec[(i)*(nshell+1) + m], i = 0..5 = spec_gp(m, i+1) (:394-399).
-__device__ __forceinline__ void spectra_body(int m, const int* __restrict__ modes, const int* __restrict__ offs,
-                                             const cplx* __restrict__ KW1, const cplx* __restrict__ KW2,
-                                             const cplx* __restrict__ KQ1, const cplx* __restrict__ KQ2,
-                                             const cplx* __restrict__ KR, const cplx* __restrict__ KP, SpecArgs a,
-                                             double* __restrict__ spec)
+// shells that hold retained modes: 0 .. spec_shells - 1, nint(|k|) of the
+// dealias radius N/3
+__host__ __device__ constexpr int spec_shells(int N) { return (N + 1) / 3 + 1; }
+
+// largest ky >= 0 of column kx in a shell <= m: kx^2 + ky^2 <= m (m + 1)
+// (src/diagnostics.f90:341-343 by the integer identity m(m-1) < k^2 <=
+// m(m+1)); -1 if there is none
+__device__ __forceinline__ int shell_end(int m, int kx)
 {
-    __shared__ double sh[6 * 16];
-    double acc[6] = {0, 0, 0, 0, 0, 0};
-    for (int j = offs[m] + threadIdx.x; j < offs[m + 1]; j += blockDim.x) {
-        const int idx = modes[j];
-        const int kx = ksg(idx / a.N, a.N), ky = ksg(idx % a.N, a.N);
-        // the real fields' transforms hold the kx >= 0 columns: a mode with
-        // kx < 0 takes the values of its mirror -k, whose terms are the same
-        // (every term is a squared modulus, invariant under k -> -k with
-        // the conjugated amplitudes)
-        const int kxm = kx < 0 ? -kx : kx, kym = kx < 0 ? -ky : ky;
-        const int idh = kxm * a.N + (kym < 0 ? kym + a.N : kym);
-        const double kxd = kxm, kyd = kym, kr2 = kxd * kxd + kyd * kyd;
-        const cplx aa1 = KW1[idh], aa2 = KW2[idh];
-        cplx bb = czero();
-        if (!(kx == 0 && ky == 0)) {
-            // bb = -i (kx/k^2) aa1 - i (ky/k^2) aa2
-            const double f1 = kxd / kr2, f2 = kyd / kr2;
-            const cplx b1 = mk(f1 * aa1.y, -f1 * aa1.x), b2 = mk(f2 * aa2.y, -f2 * aa2.x);
-            bb = cadd(b1, b2);
-        }
-        const cplx cc1 = mk(-kxd * bb.y, kxd * bb.x), cc2 = mk(-kyd * bb.y, kyd * bb.x);
-        const cplx dd1 = csub(aa1, cc1), dd2 = csub(aa2, cc2);
-        const cplx e1 = KQ1[idh], e2 = KQ2[idh], ff = KR[idh], gg = KP[idx];
-        auto ab2 = [](cplx z) { const double h = hypot(z.x, z.y); return h * h; };
-        acc[0] += a.enorm * (ab2(aa1) + ab2(aa2)) * 0.5;
-        acc[1] += a.enorm * (ab2(dd1) + ab2(dd2)) * 0.5;
-        acc[2] += a.enorm * (ab2(cc1) + ab2(cc2)) * 0.5;
-        acc[3] += a.enorm * (ab2(e1) + ab2(e2)) * 2.0 * (a.alpha * a.alpha);
-        acc[4] += a.enorm * ab2(ff) * 0.5 * a.g * 2.0 * a.alpha;
-        acc[5] += a.enorm * ab2(gg);
-    }
-    block_sum<6>(acc, sh);
-    if (threadIdx.x == 0)
-        for (int i = 0; i < 6; ++i) spec[(size_t)i * (a.nshell + 1) + m] = acc[i];
+    const int r = m * (m + 1) - kx * kx;
+    return r < 0 ? -1 : (int)sqrt((double)r);
 }
 
-__global__ void k_spectra(const int* __restrict__ modes, const int* __restrict__ offs,
-                          const cplx* __restrict__ KW1, const cplx* __restrict__ KW2,
-                          const cplx* __restrict__ KQ1, const cplx* __restrict__ KQ2,
-                          const cplx* __restrict__ KR, const cplx* __restrict__ KP, SpecArgs a,
-                          double* __restrict__ spec)
+// Column pass of the spectra (src/diagnostics.f90:320-402): the columns kx
+// and -kx of H1 and H2 (kx >= 0 panels), transformed along y and separated
+// into the transforms of the real fields by their symmetry, with rho-hat and
+// kpsi give the terms of every mode of the two columns; a mode and its mirror
+// share the first five.  The shells of a column are runs of ky, so each
+// shell's sum is one thread's, in order of |ky|; part[kx][6][spec_shells],
+// entries m >= kx, summed over the columns by spec_reduce_body.
+// 4096^2: 0.6 GB in order, against a gather of 16-byte values by shell lists
+// (0.42 ms) after eight transforms.
+template <class C, int G = C::TC>
+__device__ __forceinline__ void diag_col_body(int b, cplx* __restrict__ H1, const cplx* __restrict__ H2,
+                                              const cplx* __restrict__ K0, const cplx* __restrict__ Krho,
+                                              const cplx* __restrict__ tw, Geo g, double* __restrict__ part)
 {
-    spectra_body(blockIdx.x, modes, offs, KW1, KW2, KQ1, KQ2, KR, KP, a, spec);
+    VK_COL_SETUP_G(C, G, b, pb_, g.Pp)
+    const auto w_ = twiddles<C>(tw, t);
+    const bool live = kx <= g.M;
+    const int km = (N - kx) & (N - 1);
+    constexpr int MS = spec_shells(N);
+    const double mult = kx > 0 ? 2.0 : 1.0;
+    double* pk = part + (size_t)kx * 6 * MS;
+    // val of every ky of this column into its shells of spectrum q
+    auto bin = [&](const double (&val)[S], int q) {
+        lds_barrier();
+#pragma unroll
+        for (int s = 0; s < S; ++s) lg[t + T * s] = val[s];
+        lds_barrier();
+        if (live)
+            for (int m = kx + t; m < MS; m += T) {
+                const int hi = shell_end(m, kx);
+                double x = 0.0;
+                for (int k = m > 0 ? shell_end(m - 1, kx) + 1 : 0; k <= hi; ++k) x += k > 0 ? lg[k] + lg[N - k] : lg[0];
+                pk[q * MS + m] = x;
+            }
+    };
+    cplx v[S], um[S];
+    // the transforms of the two real fields packed in H: v, um
+    auto pair = [&](const cplx* H) {
+        const brsrc rb = mkbuf(H, N);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            v[s] = bld(rb, boff(hoff<C>(p, t + T * s, c), live));
+            um[s] = bld(rb, boff(hoff<C>(km / TC, t + T * s, km % TC), live));
+        }
+        fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+        lds_barrier();
+        fft_fwd<N, S, C::SPLIT>(um, lg, t, w_);
+        lds_barrier();
+        // um at -ky
+#pragma unroll
+        for (int s = 0; s < S; ++s) lg[t + T * s] = um[s].x;
+        lds_barrier();
+#pragma unroll
+        for (int s = 0; s < S; ++s) um[s].x = lg[(N - t - T * s) & (N - 1)];
+        lds_barrier();
+#pragma unroll
+        for (int s = 0; s < S; ++s) lg[t + T * s] = um[s].y;
+        lds_barrier();
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            um[s].y = -lg[(N - t - T * s) & (N - 1)];
+            const cplx z = v[s], m = um[s];
+            v[s] = mk(0.5 * (z.x + m.x), 0.5 * (z.y + m.y));
+            um[s] = mk(0.5 * (z.y - m.y), -0.5 * (z.x - m.x));
+        }
+    };
+    auto sq = [](cplx z) { return z.x * z.x + z.y * z.y; };
+    double e[3][S];
+    // w_x, q_x: w_x waits in its column of H1, this workgroup's alone
+    pair(H1);
+#pragma unroll
+    for (int s = 0; s < S; ++s) e[2][s] = mult * sq(um[s]);
+    const brsrc r1 = mkbuf(H1, N);
+#pragma unroll
+    for (int s = 0; s < S; ++s) bst(r1, boff(hoff<C>(p, t + T * s, c), live), v[s]);
+    lds_barrier();
+    pair(H2);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const bool use = live && !kmasked(kx, ksg(t + T * s, N), N);
+        e[2][s] = use ? e[2][s] + mult * sq(um[s]) : 0.0;
+        um[s] = bld(r1, boff(hoff<C>(p, t + T * s, c), live));
+    }
+    bin(e[2], 3);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int ky = ksg(t + T * s, N);
+        const bool use = live && !kmasked(kx, ky, N);
+        const double kxd = kx, kyd = ky, kr2 = kxd * kxd + kyd * kyd;
+        const double ik2 = kr2 > 0.0 ? 1.0 / kr2 : 0.0;
+        // compressible part k (k.w)/k^2, and the rest
+        const cplx wx = um[s], wy = v[s];
+        const cplx dv = rmul(ik2, mk(kxd * wx.x + kyd * wy.x, kxd * wx.y + kyd * wy.y));
+        const cplx c1 = rmul(kxd, dv), c2 = rmul(kyd, dv);
+        e[0][s] = use ? mult * (sq(wx) + sq(wy)) : 0.0;
+        e[1][s] = use ? mult * (sq(csub(wx, c1)) + sq(csub(wy, c2))) : 0.0;
+        e[2][s] = use ? mult * (sq(c1) + sq(c2)) : 0.0;
+    }
+    bin(e[0], 0);
+    bin(e[1], 1);
+    bin(e[2], 2);
+    const brsrc rk = mkbuf(K0, N), rr = mkbuf(Krho, N);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int k = t + T * s;
+        const bool use = live && !kmasked(kx, ksg(k, N), N);
+        e[1][s] = mult * sq(bld(rr, boff((size_t)kx * N + k, use)));
+        e[2][s] = sq(bld(rk, boff((size_t)kx * N + k, use))) +
+                  sq(bld(rk, boff((size_t)km * N + ((N - k) & (N - 1)), use && kx > 0)));
+    }
+    bin(e[1], 4);
+    bin(e[2], 5);
+}
+
+// The column partials of diag_col_body and the row sums of diag_row_body to
+// the results: block (bx, q < 6): 64 shells of spectrum q over the columns,
+// out[8 + q (nshell + 1) + m]; block (0, 6): the 8 sums over the rows, out[0..7].
+// Fixed order: 16 interleaved partial sums, added in turn.
+constexpr int SPEC_G = 16;
+__device__ __forceinline__ void spec_reduce_body(const double* __restrict__ part, const double* __restrict__ rsum,
+                                                 const SpecArgs& a, double* __restrict__ out)
+{
+    __shared__ double sh[SPEC_G][64];
+    const int l = threadIdx.x % 64, w = threadIdx.x / 64, q = blockIdx.y;
+    const int MS = spec_shells(a.N), M = a.N / 3;
+    double x = 0.0;
+    if (q == 6) {
+        if (blockIdx.x > 0) return;
+        // lane l: value l % 8 of the rows l / 8 + 8 w + 128 i
+        if (l % 8 < 7)
+            for (int y = l / 8 + 8 * w; y < a.N; y += 8 * SPEC_G) x += rsum[8 * (size_t)y + l % 8];
+        sh[w][l] = x;
+        __syncthreads();
+        if (threadIdx.x < 8) {
+            double s = 0.0;
+            for (int k = 0; k < SPEC_G; ++k)
+                for (int j = 0; j < 8; ++j) s += sh[k][8 * j + threadIdx.x];
+            out[threadIdx.x] = threadIdx.x < 7 ? s : 0.0;
+        }
+        return;
+    }
+    const int m = blockIdx.x * 64 + l;
+    if (m < MS) {
+        const int last = m < M ? m : M;
+#pragma unroll 4
+        for (int kx = w; kx <= last; kx += SPEC_G) x += part[((size_t)kx * 6 + q) * MS + m];
+    }
+    sh[w][l] = x;
+    __syncthreads();
+    if (w == 0 && m <= a.nshell) {
+        double s = sh[0][l];
+#pragma unroll
+        for (int k = 1; k < SPEC_G; ++k) s += sh[k][l];
+        // factors of spec_gp (:394-399)
+        const double f = q < 3 ? 0.5 : q == 3 ? 2.0 * (a.alpha * a.alpha) : q == 4 ? 0.5 * a.g * 2.0 * a.alpha : 1.0;
+        out[8 + q * (a.nshell + 1) + m] = a.enorm * s * f;
+    }
+}
+
+template <class C>
+__global__ void __launch_bounds__(C::ROWT) k_p1d(const cplx* __restrict__ Hpsi, cplx* __restrict__ Hrho,
+                                                 const cplx* __restrict__ tw, Geo g, int psi_pmode, double scale)
+{
+    p1_body<C, false>(blockIdx.x, gridDim.x, Hpsi, Hrho, tw, g, psi_pmode, scale, nullptr);
+}
+
+// two waves per SIMD (<= 256 VGPRs); the LAT shapes one
+#define VK_DIAGOCC(C) __attribute__((amdgpu_waves_per_eu(is_lat<C>::value ? 1 : 2)))
+
+template <class C>
+__global__ void __launch_bounds__(C::ROWT) VK_DIAGOCC(C)
+k_diag_row(const cplx* __restrict__ Hpsi, const cplx* __restrict__ Hdy, const cplx* __restrict__ Hrhod,
+           const cplx* __restrict__ HV, cplx* __restrict__ H1, cplx* __restrict__ H2, const cplx* __restrict__ tw,
+           Geo g, int pl, double scale, DiagArgs a, double* __restrict__ rsum)
+{
+    diag_row_body<C>(blockIdx.x, gridDim.x, Hpsi, Hdy, Hrhod, HV, H1, H2, tw, g, pl, scale, a, rsum);
+}
+
+template <class C, int G>
+__global__ void __launch_bounds__(G * C::T) VK_DIAGOCC(C)
+k_diag_col(cplx* __restrict__ H1, const cplx* __restrict__ H2, const cplx* __restrict__ K0,
+           const cplx* __restrict__ Krho, const cplx* __restrict__ tw, Geo g, double* __restrict__ part)
+{
+    diag_col_body<C, G>(blockIdx.x, H1, H2, K0, Krho, tw, g, part);
+}
+
+__global__ void __launch_bounds__(64 * SPEC_G) k_spec_reduce(const double* __restrict__ part,
+                                                             const double* __restrict__ rsum, SpecArgs a,
+                                                             double* __restrict__ out)
+{
+    spec_reduce_body(part, rsum, a, out);
 }
 
 // ----------------------------------------------------------------------------
@@ -1127,22 +1365,6 @@ struct BPair {
 };
 
 template <class C>
-__global__ void __launch_bounds__(C::ROWT) VK_OCC k_row_fwd_b(const BPair* __restrict__ P, const cplx* __restrict__ tw,
-                                                       Geo g, int pstore, int op)
-{
-    const BPair q = P[blockIdx.y];
-    row_fwd_body<C>(blockIdx.x, gridDim.x, q.src, q.dst, tw, g, pstore, op);
-}
-
-template <class C>
-__global__ void __launch_bounds__(C::COLT) VK_OCC k_col_fwd_b(const BPair* __restrict__ P, const cplx* __restrict__ tw,
-                                                       Geo g, int pmode, int op)
-{
-    const BPair q = P[blockIdx.y];
-    col_fwd_body<C>(blockIdx.x, q.src, q.dst, tw, g, pmode, op);
-}
-
-template <class C>
 __global__ void __launch_bounds__(C::COLT) VK_OCC k_col_inv_b(const BPair* __restrict__ P, const cplx* __restrict__ tw,
                                                        Geo g, int pmode, int op)
 {
@@ -1150,42 +1372,59 @@ __global__ void __launch_bounds__(C::COLT) VK_OCC k_col_inv_b(const BPair* __res
     col_inv_body<C>(blockIdx.x, q.src, q.dst, tw, g, pmode, op);
 }
 
-template <class C>
-__global__ void __launch_bounds__(C::ROWT) VK_OCC k_row_inv_b(const BPair* __restrict__ P, const cplx* __restrict__ tw,
-                                                       Geo g, int pload, int op, double scale)
-{
-    const BPair q = P[blockIdx.y];
-    row_inv_body<C>(blockIdx.x, gridDim.x, q.src, q.dst, tw, g, pload, op, scale);
-}
-
 // one field's diagnostics operands
 struct DiagB {
-    const cplx *psi, *D1, *D2, *PR;
-    cplx *W1, *W2, *Q1, *Q2;
-    double* part;     // 8 partial sums per block
-    double* sums;     // 8 sums
-    double* spec;     // 6 (nshell + 1) spectra
-    const cplx *KW1, *KW2, *KQ1, *KQ2, *KR, *KP;
+    const cplx *Hpsi, *K0;
+    cplx *Hd, *Hrho, *Krho, *H1, *H2;
+    double *rsum, *part, *out;
     DiagArgs da;
     SpecArgs sa;
 };
 
-__global__ void k_diag_x_b(const DiagB* __restrict__ D)
+template <class C>
+__global__ void __launch_bounds__(C::COLT) VK_OCC k_diag_dy_b(const DiagB* __restrict__ D, const cplx* __restrict__ tw,
+                                                              Geo g, int pl)
 {
     const DiagB& d = D[blockIdx.y];
-    diag_x_body(blockIdx.x, gridDim.x, d.psi, d.D1, d.D2, d.PR, nullptr, d.W1, d.W2, d.Q1, d.Q2, d.da, d.part);
+    col_inv_body<C>(blockIdx.x, d.K0, d.Hd, tw, g, pl, 2);
 }
 
-__global__ void k_reduce_fixed_b(const DiagB* __restrict__ D, int nb)
-{
-    const DiagB& d = D[blockIdx.x];
-    reduce_fixed_body(d.part, nb, 8, d.sums);
-}
-
-__global__ void k_spectra_b(const int* __restrict__ modes, const int* __restrict__ offs, const DiagB* __restrict__ D)
+template <class C>
+__global__ void __launch_bounds__(C::ROWT) VK_OCC k_p1d_b(const DiagB* __restrict__ D, const cplx* __restrict__ tw,
+                                                          Geo g, int pl, double scale)
 {
     const DiagB& d = D[blockIdx.y];
-    spectra_body(blockIdx.x, modes, offs, d.KW1, d.KW2, d.KQ1, d.KQ2, d.KR, d.KP, d.sa, d.spec);
+    p1_body<C, false>(blockIdx.x, gridDim.x, d.Hpsi, d.Hrho, tw, g, pl, scale, nullptr);
+}
+
+template <class C>
+__global__ void __launch_bounds__(C::COLT) VK_OCC k_p2d_b(const DiagB* __restrict__ D, const cplx* __restrict__ tw,
+                                                          Geo g)
+{
+    const DiagB& d = D[blockIdx.y];
+    p2_body<C, C::TC, 2>(blockIdx.x, gridDim.x, d.Hrho, nullptr, nullptr, d.Krho, tw, g, 2);
+}
+
+template <class C>
+__global__ void __launch_bounds__(C::ROWT) VK_DIAGOCC(C)
+k_diag_row_b(const DiagB* __restrict__ D, const cplx* __restrict__ tw, Geo g, int pl, double scale)
+{
+    const DiagB& d = D[blockIdx.y];
+    diag_row_body<C>(blockIdx.x, gridDim.x, d.Hpsi, d.Hd, d.Hrho, nullptr, d.H1, d.H2, tw, g, pl, scale, d.da, d.rsum);
+}
+
+template <class C>
+__global__ void __launch_bounds__(C::COLT) VK_DIAGOCC(C)
+k_diag_col_b(const DiagB* __restrict__ D, const cplx* __restrict__ tw, Geo g)
+{
+    const DiagB& d = D[blockIdx.y];
+    diag_col_body<C>(blockIdx.x, d.H1, d.H2, d.K0, d.Krho, tw, g, d.part);
+}
+
+__global__ void __launch_bounds__(64 * SPEC_G) k_spec_reduce_b(const DiagB* __restrict__ D)
+{
+    const DiagB& d = D[blockIdx.z];
+    spec_reduce_body(d.part, d.rsum, d.sa, d.out);
 }
 
 // ----------------------------------------------------------------------------
