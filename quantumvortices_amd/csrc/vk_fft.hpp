@@ -149,20 +149,6 @@ template <> struct Dft<16> {
     }
 };
 
-// Radix plan: largest radix dividing both S and the remaining length.
-__host__ __device__ constexpr int radix_at(int N, int S, int st)
-{
-    int n = N;
-    int r = 1;
-    for (int i = 0; i <= st; ++i) {
-        r = 1;
-        for (int R = 16; R >= 2; R >>= 1)
-            if (S % R == 0 && n % R == 0) { r = R; break; }
-        n /= r;
-    }
-    return r;
-}
-
 // LDS slot of point p in an exchange: one pad double per 16 points, so that
 // the 16-strided writes of a stage with sub-length 1 spread over the banks
 __device__ __forceinline__ int lslot(int p) { return p + (p >> 4); }
@@ -192,18 +178,74 @@ template <int NS, int R> __device__ __forceinline__ int scatter_idx(int idxD, in
     else return lslot(idxD + r * NS);
 }
 
-// Table values a stage needs per butterfly: w^1..w^3 and w^4, w^8, ... (the
-// other factors are one product of two of them)
-constexpr int tw_per(int R) { return R == 2 ? 1 : 3 + (R / 4 - 1); }
-constexpr int tw_mult(int k) { return k < 3 ? k + 1 : 4 * (k - 2); }
+// Radix plan: largest radix dividing both S and the remaining length.
+__host__ __device__ constexpr int radix_at(int N, int S, int st)
+{
+    int n = N;
+    int r = 1;
+    for (int i = 0; i <= st; ++i) {
+        r = 1;
+        for (int R = 16; R >= 2; R >>= 1)
+            if (S % R == 0 && n % R == 0) { r = R; break; }
+        n /= r;
+    }
+    return r;
+}
+
+// A stage with twiddles: X[k] = sum_r (w^r x[r]) e^{-2 pi i r k/R}, by halving
+// in time.  Level M (2, 4, .., R) joins halves e, d with o[k] = e[k] + f d[k],
+// o[k + M/2] = e[k] - f d[k], f = w^{R/M} e^{-2 pi i k/M}; the second quarter's
+// factors are -i times the first's.  Each join is six fused operations
+// (e + f d in four, the other as 2 e - it in two), 12 per point and radix-16
+// stage against 16 for twiddle products followed by an untwiddled butterfly.
+// Few-wave passes pay every operation in latency: a step at 512^2 120.4 to
+// 113.1 us, at 1024^2 181.4 to 169.2, at 2048^2 550 to 519; at 4096^2 HBM and
+// LDS bound it (2106 to 2100).  Rounding: a field after 5 to 50 steps is within
+// 7.8e-16 of one computed with longer sums, 7.5e-16 before.
+// The factors, R/2 table values: slot 0 for M = 2, 1 for M = 4, 2 + k for
+// M = 8, 4 + k for M = 16, each w_N^{(R/M) base + k N/M} with w = w_N^base.
+constexpr int tw_per(int R) { return R / 2; }
+constexpr int tw_level(int slot) { return slot == 0 ? 2 : slot == 1 ? 4 : slot < 4 ? 8 : 16; }
+template <int N, int R> constexpr int tw_mult(int slot) { return R / tw_level(slot); }
+template <int N, int R> constexpr int tw_add(int slot) { return slot < 2 ? 0 : (slot < 4 ? slot - 2 : slot - 4) * (N / tw_level(slot)); }
+
+// x: in r order; out: k order.  Level by level, f(slot) asked for at its level.
+template <int R, int M = 2, class F> __device__ __forceinline__ void dit(cplx (&x)[R], const F& f)
+{
+    // x[OFF * (M/2) + k] holds the half-size transforms of the points OFF + (2R/M) i
+    constexpr int Q = M / 4 > 0 ? M / 4 : 1;
+    constexpr int S0 = M == 2 ? 0 : M == 4 ? 1 : M == 8 ? 2 : 4;
+    cplx w[Q], o[R];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) w[q] = f(S0 + q);
+#pragma unroll
+    for (int off = 0; off < R / M; ++off)
+#pragma unroll
+        for (int k = 0; k < M / 2; ++k) {
+            const cplx e = x[off * (M / 2) + k], d = x[(off + R / M) * (M / 2) + k];
+            const cplx b = k >= Q ? mul_mi(d) : d, u = w[k % Q];
+            const cplx t = mk(__builtin_fma(-u.y, b.y, __builtin_fma(u.x, b.x, e.x)),
+                              __builtin_fma(u.y, b.x, __builtin_fma(u.x, b.y, e.y)));
+            o[off * M + k] = t;
+            o[off * M + k + M / 2] = mk(__builtin_fma(2.0, e.x, -t.x), __builtin_fma(2.0, e.y, -t.y));
+        }
+#pragma unroll
+    for (int r = 0; r < R; ++r) x[r] = o[r];
+    if constexpr (M < R) dit<R, 2 * M>(x, f);
+}
 
 // Twiddles read from the table where they are used (few registers: several
-// workgroups per CU hide the loads).
-struct TwMem {
+// workgroups per CU hide the loads).  E: a stage's values all loaded before
+// its first level, so that no level waits for its own; where the registers
+// allow it.  At 4096^2: P1 138.5 to 137.2 us, P2 70.3 to 67.8, P3 with particles
+// 150 to 146, a step with them 2229 to 2196; P3 without particles is slower so
+// (147 to 178).
+template <bool E> struct TwMem {
     const cplx* tw;
-    template <int OFF, int K> __device__ __forceinline__ cplx get(int, int k, int base) const
+    static constexpr bool EAGER = E;
+    template <int N, int R, int OFF> __device__ __forceinline__ cplx get(int, int k, int base) const
     {
-        return tw[tw_mult(k) * base];
+        return tw[tw_mult<N, R>(k) * base + tw_add<N, R>(k)];
     }
 };
 
@@ -224,7 +266,11 @@ template <int N, int S> constexpr int tw_count()
 // whose few waves leave registers idle and every load exposed.
 template <int N, int S> struct TwReg {
     cplx w[tw_count<N, S>() > 0 ? tw_count<N, S>() : 1];
-    template <int OFF, int K> __device__ __forceinline__ cplx get(int a, int k, int) const { return w[OFF + a * K + k]; }
+    static constexpr bool EAGER = false;
+    template <int, int R, int OFF> __device__ __forceinline__ cplx get(int a, int k, int) const
+    {
+        return w[OFF + a * tw_per(R) + k];
+    }
 
     template <int ST, int NS, int OFF> __device__ __forceinline__ void load_stage(const cplx* __restrict__ tw, int t)
     {
@@ -235,7 +281,7 @@ template <int N, int S> struct TwReg {
 #pragma unroll
                 for (int a = 0; a < S / R; ++a)
 #pragma unroll
-                    for (int k = 0; k < K; ++k) w[OFF + a * K + k] = tw[tw_mult(k) * (((t + T * a) % NS) * STEP)];
+                    for (int k = 0; k < K; ++k) w[OFF + a * K + k] = tw[tw_mult<N, R>(k) * (((t + T * a) % NS) * STEP) + tw_add<N, R>(k)];
                 load_stage<ST + 1, NS * R, OFF + (S / R) * K>(tw, t);
             } else {
                 load_stage<ST + 1, NS * R, OFF>(tw, t);
@@ -269,29 +315,20 @@ struct Stage {
 #pragma unroll
             for (int r = 0; r < R; ++r) x[r] = v[a + (S / R) * r];
             if constexpr (NS > 1) {
-                // w^r for r = 4a + b from table values w^1..w^3 and w^4a
-                // (one product at most per factor)
                 constexpr int STEP = N / (NS * R);
                 const int base = jm * STEP;
-                const cplx w1 = tw.template get<OFF, K>(a, 0, base);
-                if constexpr (R == 2) {
-                    x[1] = cmul(x[1], w1);
-                } else {
-                    const cplx w2 = tw.template get<OFF, K>(a, 1, base), w3 = tw.template get<OFF, K>(a, 2, base);
-                    x[1] = cmul(x[1], w1);
-                    x[2] = cmul(x[2], w2);
-                    x[3] = cmul(x[3], w3);
+                if constexpr (W::EAGER) {
+                    cplx f[K];
 #pragma unroll
-                    for (int a4 = 1; a4 < R / 4; ++a4) {
-                        const cplx wa = tw.template get<OFF, K>(a, 2 + a4, base);
-                        x[4 * a4] = cmul(x[4 * a4], wa);
-                        x[4 * a4 + 1] = cmul(x[4 * a4 + 1], cmul(wa, w1));
-                        x[4 * a4 + 2] = cmul(x[4 * a4 + 2], cmul(wa, w2));
-                        x[4 * a4 + 3] = cmul(x[4 * a4 + 3], cmul(wa, w3));
-                    }
+                    for (int k = 0; k < K; ++k) f[k] = tw.template get<N, R, OFF>(a, k, base);
+                    __builtin_amdgcn_sched_barrier(0);
+                    dit<R>(x, [&](int k) { return f[k]; });
+                } else {
+                    dit<R>(x, [&](int k) { return tw.template get<N, R, OFF>(a, k, base); });
                 }
+            } else {
+                Dft<R>::run(x);
             }
-            Dft<R>::run(x);
 #pragma unroll
             for (int r = 0; r < R; ++r) v[a + (S / R) * r] = x[r];
         }
@@ -350,7 +387,7 @@ template <int N, int S, int ST, bool SPLIT, int OFF> struct Stage<N, S, ST, N, S
 // lds: base of this transform's LDS region (Lds<N>::words doubles when
 // SPLIT, twice that otherwise).  All threads of the workgroup must call it
 // (it contains workgroup barriers).
-template <int N, int S, bool SPLIT>
+template <int N, int S, bool SPLIT, bool EAGER = false>
 __device__ __forceinline__ void fft_fwd(cplx (&v)[S], double* lds, int t, const cplx* __restrict__ tw)
 {
     // Register-only compiler barrier on the (uniform) table pointer: each
@@ -358,11 +395,11 @@ __device__ __forceinline__ void fft_fwd(cplx (&v)[S], double* lds, int t, const 
     // transform's values live across the pointwise work in between.
     const cplx* twb = tw;
     asm volatile("" : "+s"(twb));
-    Stage<N, S, 0, 1, SPLIT>::run(v, lds, SPLIT ? lds : lds + Lds<N>::words, t, TwMem{twb});
+    Stage<N, S, 0, 1, SPLIT>::run(v, lds, SPLIT ? lds : lds + Lds<N>::words, t, TwMem<EAGER>{twb});
 }
 
 // the same with twiddles in registers
-template <int N, int S, bool SPLIT>
+template <int N, int S, bool SPLIT, bool = false>
 __device__ __forceinline__ void fft_fwd(cplx (&v)[S], double* lds, int t, const TwReg<N, S>& w)
 {
     Stage<N, S, 0, 1, SPLIT>::run(v, lds, SPLIT ? lds : lds + Lds<N>::words, t, w);

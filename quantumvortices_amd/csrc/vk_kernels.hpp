@@ -276,7 +276,7 @@ __device__ __forceinline__ void p1_core(cplx (&v)[C::S], double* lg, int t, int 
                                         double scale, cplx* __restrict__ Xpsi)
 {
     constexpr int N = C::N, S = C::S, T = C::T, TC = C::TC;
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    fft_fwd<N, S, C::SPLIT, true>(v, lg, t, w_);
     if constexpr (XS) {
         cplx* xr = Xpsi + (size_t)y * N;
 #pragma unroll
@@ -287,7 +287,7 @@ __device__ __forceinline__ void p1_core(cplx (&v)[C::S], double* lg, int t, int 
         const double a = scale * v[s].x, b = scale * v[s].y;   // conj does not change |.|
         v[s] = mk(a * a + b * b, 0.0);
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    fft_fwd<N, S, C::SPLIT, true>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int pp = VK_PANEL(s);
@@ -314,7 +314,7 @@ __device__ __forceinline__ void p1_body(int blk_, int nblk_, const cplx* __restr
     }
     const auto w_ = twiddles<C>(tw, t);
 #pragma unroll
-    for (int s = 0; s < S; ++s) v[s] = panel_stored(VK_PANEL(s), NP, g, psi_pmode) ? conjc(v[s]) : czero();
+    for (int s = 0; s < S; ++s) v[s] = conjc(v[s]);   // a panel not stored loads as zero
     p1_core<C, XS>(v, lg, t, y, pidx0, c, Hrho, w_, g, scale, Xpsi);
 }
 
@@ -454,7 +454,7 @@ __device__ __forceinline__ void p2_body(int blk_, int nblk_, cplx* __restrict__ 
     cplx v[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) v[s] = Hrho[hoff<C>(p, t + T * s, c)];
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    fft_fwd<N, S, C::SPLIT, true>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int ky = t + T * s;
@@ -463,7 +463,7 @@ __device__ __forceinline__ void p2_body(int blk_, int nblk_, cplx* __restrict__ 
         else if (flags & 2) Krho[(size_t)kx * N + ky] = v[s];
         v[s] = conjc(v[s]);
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    fft_fwd<N, S, C::SPLIT, true>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) Hrho[hoff<C>(p, t + T * s, c)] = conjc(v[s]);
     if (flags & 1) {
@@ -472,7 +472,7 @@ __device__ __forceinline__ void p2_body(int blk_, int nblk_, cplx* __restrict__ 
             const int ky = t + T * s;
             v[s] = kmasked(kx, ksg(ky, N), N) ? czero() : conjc(KV[(size_t)kx * N + ky]);
         }
-        fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+        fft_fwd<N, S, C::SPLIT, true>(v, lg, t, w_);
 #pragma unroll
         for (int s = 0; s < S; ++s) HV[hoff<C>(p, t + T * s, c)] = conjc(v[s]);
     }
@@ -645,7 +645,7 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
         }
         v[s] = conjc(mk(a.x - b.y, a.y + b.x));   // a + i b, conj for the inverse
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    fft_fwd<N, S, C::SPLIT, PM == 4>(v, lg, t, w_);
     // v[s].x = rho_d (unnormalised); v[s].y = -V (unnormalised, flags & 1).
     double f[S];   // the real factor g rho_d + V
 #pragma unroll
@@ -762,7 +762,7 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
                 }
                 w[s] = conjc(a);
             }
-            fft_fwd<N, S, C::SPLIT>(w, lg, t, w_);
+            fft_fwd<N, S, C::SPLIT, PM == 4>(w, lg, t, w_);
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 const cplx e = tw[t + T * s];
@@ -775,7 +775,7 @@ __device__ __forceinline__ void p3_body(int blk_, int nblk_, const cplx* __restr
             }
         }
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    fft_fwd<N, S, C::SPLIT, PM == 4>(v, lg, t, w_);
     // branch-free buffer stores (an unstored panel gets the out-of-range
     // offset and is dropped): conditional stores made the compiler sink the
     // last butterfly into one branch per store (P3 0.191 -> 0.187 ms)
@@ -857,7 +857,7 @@ __device__ __forceinline__ void p4_body(int blk_, int nblk_, const cplx* __restr
             if constexpr (STAGE >= 3) k1v[s] = bld(r1, o);
         }
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    fft_fwd<N, S, C::SPLIT, true>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int ky = t + T * s;
@@ -884,7 +884,7 @@ __device__ __forceinline__ void p4_body(int blk_, int nblk_, const cplx* __restr
         }
         v[s] = conjc(keep ? kn : czero());
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    fft_fwd<N, S, C::SPLIT, true>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) Hpsi[hoff<C>(p, t + T * s, c)] = conjc(v[s]);
 }
