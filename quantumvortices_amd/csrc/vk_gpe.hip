@@ -115,7 +115,7 @@ struct vk_gpe {
     int sgle = 0;
     double sg_beta = 0.0, sg_nuN = 0.0, sg_ktrunc = 0.0;
     unsigned long long sg_seed = 0, sg_draw = 0;
-    cplx *Xn = nullptr, *Kn = nullptr;
+    cplx* Xn = nullptr;
     double *omega_dev = nullptr, *npart = nullptr;
     cplx *HV = nullptr, *KV = nullptr, *Krho = nullptr, *Vhat = nullptr, *EX = nullptr, *EY = nullptr;
     double* pst2 = nullptr;   // real-space path: positions and velocities after RK4 stages 1 and 3
@@ -642,35 +642,9 @@ int rk4_step(vk_gpe* h)
     });
 }
 
-// SGLE part of one ARGLE step, before the passes: the noise field of this
-// step (noise = caller's standard normals, or NULL for the generator's next
-// draw) scaled by noisesigma/sqrt(dvol) (src/gpe.f90:150-164) and
-// transformed to k-space, and the chemical potential of this step from the
-// norm of kpsi at the step's start (finiteT_adhoc_chempot, :226-266).
-constexpr int kNormBlocks = 1024;
-int sgle_prepare(vk_gpe* h, const double* noise)
-{
-    const double pi = 4.0 * std::atan(1.0);
-    const double L = 2.0 * pi, dx = L / h->N, dvol = dx * dx;
-    const double sigma = std::sqrt((1.0 / (2.0 * h->p.alpha)) * h->sg_beta);
-    if (noise) HIPCHK(hipMemcpyAsync(h->Xn, noise, f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
-    hipLaunchKernelGGL(vk::k_sgle_noise, dim3(1024), dim3(256), 0, h->stream, h->Xn, h->N, h->sg_draw, h->sg_seed,
-                       1.0 / std::sqrt(dvol), sigma, noise ? 0 : 1);
-    if (!noise) h->sg_draw++;
-    int rc = fwd2d(h, h->Xn, h->Hd, h->Kn, 0, 0);
-    if (rc) return rc;
-    hipLaunchKernelGGL(vk::k_knorm, dim3(kNormBlocks), dim3(256), 0, h->stream, (const cplx*)h->K0, f2(h), h->npart);
-    hipLaunchKernelGGL(vk::k_chempot, dim3(1), dim3(256), 0, h->stream, (const double*)h->npart, kNormBlocks,
-                       h->omega_dev, dvol / ((double)h->N * (double)h->N), h->p.dt, h->sg_nuN, L * L);
-    return 0;
-}
-
 int argle_step(vk_gpe* h, int want_res, const double* noise = nullptr)
 {
-    if (h->sgle) {
-        int rc = sgle_prepare(h, noise);
-        if (rc) return rc;
-    }
+    if (noise) HIPCHK(hipMemcpyAsync(h->Xn, noise, f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
     return dispatch(h->N, [&](auto n) {
         using C = CfgN<decltype(n)::value>;
         const double sc = scale_of(h);
@@ -690,7 +664,24 @@ int argle_step(vk_gpe* h, int want_res, const double* noise = nullptr)
         if (adv)   // i ky kpsi -> Hdy (all columns)
             colg_launch<C, GC>(h, PK_OTHER, h->NP, vk::k_col_inv<C, GC>, (const cplx*)h->K0, h->Hdy,
                                (const cplx*)h->tw, h->geo, 0, 2);
-        row_launch<C>(h, PK_P1, vk::k_p1x<C>, (const cplx*)h->Hpsi, h->Hrho, (const cplx*)h->tw, h->geo, 0, sc, h->Xs);
+        const double L = 8.0 * std::atan(1.0), dvol = (L / h->N) * (L / h->N);
+        if (h->sgle) {
+            // this step's noise (the caller's normals, or the generator's next
+            // draw; src/gpe.f90:150-164) and P1
+            const vk::NoiseArgs na{noise ? h->Xn : nullptr, h->Hd, h->sg_draw, h->sg_seed, 1.0 / std::sqrt(dvol),
+                                   std::sqrt((1.0 / (2.0 * h->p.alpha)) * h->sg_beta), h->omega_dev};
+            if (!noise) h->sg_draw++;
+            const size_t lds = (size_t)C::TR * C::ROWRS * sizeof(double);
+            auto k = vk::k_p1_noise<C>;
+            set_lds(k, lds);
+            ev_begin(h);
+            hipLaunchKernelGGL(k, dim3(2 * (C::N / C::TR)), dim3(C::ROWT), lds, h->stream, (const cplx*)h->Hpsi,
+                               h->Hrho, (const cplx*)h->tw, h->geo, sc, h->Xs, h->npart, na);
+            ev_end(h, PK_P1);
+        } else {
+            row_launch<C>(h, PK_P1, vk::k_p1x<C>, (const cplx*)h->Hpsi, h->Hrho, (const cplx*)h->tw, h->geo, 0, sc,
+                          h->Xs);
+        }
         p2_launch<C>(h, h->Hrho, h->HV, (const cplx*)h->KV, h->Krho,
                       (const cplx*)h->tw, h->geo, (parts && !rs) ? 1 : 0);
         if (adv) {
@@ -708,15 +699,20 @@ int argle_step(vk_gpe* h, int want_res, const double* noise = nullptr)
         }
         vk::ArgleArgs a{h->p.alpha, h->p.omega, h->p.dt, want_res};
         if (h->sgle) {
-            a.Kn = h->Kn;
-            a.omega_dev = h->omega_dev;
+            a.Hn = h->Hd;
+            a.nsum = h->npart;
+            a.om = h->omega_dev;
+            a.dvol = dvol;
+            a.nuN = h->sg_nuN;
+            a.L2 = L * L;
+            a.g = h->geo;
             a.sdt = std::sqrt(h->p.dt);
             a.ktrunc2 = h->sg_ktrunc > 0.0 ? h->sg_ktrunc * h->sg_ktrunc : 0.0;
         }
         // the columns per workgroup of P4 (two of four at 4096^2)
         constexpr int GA = p4_cols<C>();
         static_assert(GA == C::TC || C::NP % 8 == 0, "column groups need whole groups of 8 panels");
-        colg_launch<C, GA>(h, PK_ARG4, h->NP, vk::k_a4<C, GA>, (const cplx*)h->HN, h->Hpsi, h->K0,
+        colg_launch<C, GA>(h, PK_ARG4, h->NP, h->sgle ? vk::k_a4<C, GA, true> : vk::k_a4<C, GA>, (const cplx*)h->HN, h->Hpsi, h->K0,
                            (const cplx*)h->tw, a, h->part);
         if (want_res)
             hipLaunchKernelGGL(vk::k_reduce_fixed, dim3(1), dim3(256), 0, h->stream, (const double*)h->part,
@@ -1008,7 +1004,7 @@ void vk_gpe_destroy(vk_gpe* h)
 {
     if (!h) return;
     if (h->stream) hipStreamSynchronize(h->stream);
-    cplx* fields[] = {h->K0, h->K1, h->K2, h->Hpsi, h->Hrho, h->HN, h->tw, h->Hd, h->Xs, h->Hdy, h->Xn, h->Kn};
+    cplx* fields[] = {h->K0, h->K1, h->K2, h->Hpsi, h->Hrho, h->HN, h->tw, h->Hd, h->Xs, h->Hdy, h->Xn};
     for (auto f : fields) if (f) hipFree(f);
     for (double* f : {h->Ux, h->Uy, h->omega_dev, h->npart}) if (f) hipFree(f);
     if (h->np_cap > 0) {
@@ -1314,10 +1310,10 @@ int vk_gpe_set_sgle(vk_gpe* h, int on, double oneybeta, double nuN, double chemp
     int rc = need_x0(h);
     if (rc) return rc;
     if (!h->Xn) HIPCHK(hipMalloc(&h->Xn, f2(h) * sizeof(cplx)));
-    if (!h->Kn) HIPCHK(hipMalloc(&h->Kn, f2(h) * sizeof(cplx)));
-    if (!h->omega_dev) HIPCHK(hipMalloc(&h->omega_dev, sizeof(double)));
-    if (!h->npart) HIPCHK(hipMalloc(&h->npart, sizeof(double) * kNormBlocks));
-    HIPCHK(hipMemcpy(h->omega_dev, &chempot0, sizeof(double), hipMemcpyHostToDevice));
+    if (!h->omega_dev) HIPCHK(hipMalloc(&h->omega_dev, 2 * sizeof(double)));
+    if (!h->npart) HIPCHK(hipMalloc(&h->npart, sizeof(double) * h->N));
+    const double om[2] = {chempot0, chempot0};   // before the last step, after it
+    HIPCHK(hipMemcpy(h->omega_dev, om, sizeof(om), hipMemcpyHostToDevice));
     h->p.omega = chempot0;
     h->sgle = 1;
     h->sg_beta = oneybeta;
@@ -1334,7 +1330,7 @@ static int sgle_sync_omega(vk_gpe* h)
 {
     if (!h->sgle) return 0;
     HIPCHK(hipStreamSynchronize(h->stream));
-    HIPCHK(hipMemcpy(&h->p.omega, h->omega_dev, sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(&h->p.omega, h->omega_dev + 1, sizeof(double), hipMemcpyDeviceToHost));
     if (h->e1R) {
         const vk::EnsReal x = single_entry(h);
         HIPCHK(hipMemcpy(h->e1R, &x, sizeof(x), hipMemcpyHostToDevice));
@@ -1372,8 +1368,7 @@ int vk_sgle_noise(vk_gpe* h, unsigned long long draw, double* out_xy)
 {
     if (!h || !out_xy) return fail(VK_ERR_ARG, "sgle_noise: null argument");
     if (!h->sgle) return fail(VK_ERR_STATE, "sgle_noise: SGLE is off (vk_gpe_set_sgle)");
-    hipLaunchKernelGGL(vk::k_sgle_noise, dim3(1024), dim3(256), 0, h->stream, h->Xn, h->N, draw, h->sg_seed, 1.0, 1.0,
-                       1);
+    hipLaunchKernelGGL(vk::k_sgle_noise, dim3(1024), dim3(256), 0, h->stream, h->Xn, h->N, draw, h->sg_seed);
     HIPCHK(hipMemcpyAsync(out_xy, h->Xn, f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipGetLastError());

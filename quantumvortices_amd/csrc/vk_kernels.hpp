@@ -269,11 +269,37 @@ __global__ void k_dealias(cplx* __restrict__ K, int N)
 // Fused RK4 / ARGLE passes
 // ----------------------------------------------------------------------------
 
+// Sums over a row of nv <= 8 values per point group: thread t of the row's T
+// holds x[]; out[i] = the sum over t in a fixed tree (neighbour pairs, then
+// pairs of pairs, ...), the same in every workgroup shape.  sh: nv * T
+// doubles of LDS of this row.  Every thread of the workgroup calls it.
+template <int NV, int T>
+__device__ __forceinline__ void row_sum(const double (&x)[NV], double* sh, int t, double* __restrict__ out)
+{
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) sh[i * T + t] = x[i];
+#pragma unroll
+    for (int h = 1; h < T; h *= 2) {
+        lds_barrier();
+        if (t % (2 * h) == 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) sh[i * T + t] += sh[i * T + t + h];
+        }
+    }
+    lds_barrier();
+    if (t == 0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) out[i] = sh[i * T];
+    }
+}
+
 // P1 after its loads: v holds the conjugated Hpsi row points of this thread
-template <class C, bool XS, class W>
+// (NORM: the row's sum of |psi|^2 goes to nsum[y])
+template <class C, bool XS, bool NORM = false, class W>
 __device__ __forceinline__ void p1_core(cplx (&v)[C::S], double* lg, int t, int y, int pidx0, int c,
                                         cplx* __restrict__ Hrho, const W& w_, const Geo& g,
-                                        double scale, cplx* __restrict__ Xpsi)
+                                        double scale, cplx* __restrict__ Xpsi, double* __restrict__ nsum = nullptr)
 {
     constexpr int N = C::N, S = C::S, T = C::T, TC = C::TC;
     fft_fwd<N, S, C::SPLIT, true>(v, lg, t, w_);
@@ -287,22 +313,29 @@ __device__ __forceinline__ void p1_core(cplx (&v)[C::S], double* lg, int t, int 
         const double a = scale * v[s].x, b = scale * v[s].y;   // conj does not change |.|
         v[s] = mk(a * a + b * b, 0.0);
     }
+    double ns[1] = {0.0};
+    if constexpr (NORM) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) ns[0] += v[s].x;
+    }
     fft_fwd<N, S, C::SPLIT, true>(v, lg, t, w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int pp = VK_PANEL(s);
         if (pp < g.Pp) Hrho[hoff<C>(pp, y, c)] = v[s];
     }
+    if constexpr (NORM) row_sum<1, T>(ns, lg, t, nsum + y);
 }
 
 // P1 (row): psi row from Hpsi (inverse along x, times 1/N^2), rho = |psi|^2,
 // forward along x, keep kx >= 0 retained panels (rho is real).  The psi row
 // is stored in x-space (Xpsi[y*N + x]) for P3, which then needs no transform
 // of its own for psi; the diagnostics do without (XS false).
-template <class C, bool XS = true>
+template <class C, bool XS = true, bool NORM = false>
 __device__ __forceinline__ void p1_body(int blk_, int nblk_, const cplx* __restrict__ Hpsi, cplx* __restrict__ Hrho,
                                                 const cplx* __restrict__ tw, Geo g, int psi_pmode,
-                                                double scale, cplx* __restrict__ Xpsi)
+                                                double scale, cplx* __restrict__ Xpsi,
+                                                double* __restrict__ nsum = nullptr)
 {
     VK_ROW_SETUP(C)
     cplx v[S];
@@ -315,7 +348,7 @@ __device__ __forceinline__ void p1_body(int blk_, int nblk_, const cplx* __restr
     const auto w_ = twiddles<C>(tw, t);
 #pragma unroll
     for (int s = 0; s < S; ++s) v[s] = conjc(v[s]);   // a panel not stored loads as zero
-    p1_core<C, XS>(v, lg, t, y, pidx0, c, Hrho, w_, g, scale, Xpsi);
+    p1_core<C, XS, NORM>(v, lg, t, y, pidx0, c, Hrho, w_, g, scale, Xpsi, nsum);
 }
 
 template <class C>
@@ -902,21 +935,43 @@ struct ArgleArgs {
     double alpha, omega, dt;
     int want_res;
     // SGLE (src/gpe.f90:200-217): with Kn set, sqrt(dt) Kn (dealiased) is
-    // added to the numerator, omega is read from *omega_dev (the chemical
-    // potential of this step) and, for ktrunc2 > 0, modes with
-    // k^2 > ktrunc2 are zeroed
-    const cplx* Kn;
-    const double* omega_dev;
-    double sdt, ktrunc2;
+    // added to the numerator, omega is this step's chemical potential and,
+    // for ktrunc2 > 0, modes with k^2 > ktrunc2 are zeroed
+    const cplx* Hn;        // noise rows transformed along x, retained panels
+    const double* nsum;    // P1's row sums of |psi|^2
+    double* om;            // [0] before this step, [1] of this step
+    double sdt, ktrunc2, dvol, nuN, L2;
+    Geo g;
 };
+
+// finiteT_adhoc_chempot (src/gpe.f90:226-266): norm = sum_x |psi|^2 dvol,
+// omega - dt (nuN/L^2)(norm - L^2).  Every workgroup sums the rows in the same
+// order (N doubles from L2) instead of waiting for a launch of its own.
+template <int N, int BD> __device__ __forceinline__ double chempot_step(const ArgleArgs& a, double* lds)
+{
+    static_assert(N % BD == 0, "whole rounds of the workgroup");
+    double q[N / BD], x[1] = {0.0};
+    const double om = a.om[0];
+#pragma unroll
+    for (int i = 0; i < N / BD; ++i) q[i] = a.nsum[threadIdx.x + i * BD];
+#pragma unroll
+    for (int i = 0; i < N / BD; ++i) x[0] += q[i];
+    block_sum<1>(x, lds);
+    if (threadIdx.x == 0) lds[0] = om - a.dt * (a.nuN / a.L2) * (x[0] * a.dvol - a.L2);
+    __syncthreads();
+    const double o = lds[0];
+    __syncthreads();
+    return o;
+}
 
 // ARGLE A4 (column, all panels): forward along y -> N-hat; implicit update
 // kpsi = (kpsi + dt*(N-hat + omega*kpsi))/(1 + alpha*k^2*dt) on every mode
 // (src/gpe.f90:195-197, no dealiasing of the result); residual partial
-// sums; inverse along y of the new kpsi -> Hpsi.  G < TC: G of a panel's
+// sums; inverse along y of the new kpsi -> Hpsi.  SG: SGLE; the noise column
+// is transformed here too.  G < TC: G of a panel's
 // columns per workgroup (the host keeps NP a multiple of 8 then, so that
 // every workgroup writes its residual partials).
-template <class C, int G = C::TC>
+template <class C, int G = C::TC, bool SG = false>
 __device__ __forceinline__ void a4_body(int blk_, int nblk_, const cplx* __restrict__ HN, cplx* __restrict__ Hpsi,
                                                 cplx* __restrict__ K0, const cplx* __restrict__ tw,
                                                 ArgleArgs a, double* __restrict__ part)
@@ -934,9 +989,18 @@ __device__ __forceinline__ void a4_body(int blk_, int nblk_, const cplx* __restr
 #pragma unroll
         for (int s = 0; s < S; ++s) k0v[s] = K0[rowo + t + T * s];
     }
+    cplx nz[SG ? S : 1];
+    double omega = a.omega;
+    if constexpr (SG) {
+        const bool on = panel_stored(p, NP, a.g, 1);   // every mode of the others is masked
+#pragma unroll
+        for (int s = 0; s < S; ++s) nz[s] = on ? a.Hn[hoff<C>(p, t + T * s, c)] : czero();
+        omega = chempot_step<N, G * T>(a, lds);
+        if (blk_ == 0 && threadIdx.x == 0) a.om[1] = omega;
+        if (on) fft_fwd<N, S, C::SPLIT>(nz, lg, t, w_);
+    }
     fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
     double r[2] = {0.0, 0.0};
-    const double omega = a.omega_dev ? *a.omega_dev : a.omega;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int ky = t + T * s;
@@ -947,12 +1011,11 @@ __device__ __forceinline__ void a4_body(int blk_, int nblk_, const cplx* __restr
         const cplx t1 = cadd(v[s], rmul(omega, old));
         const double t2 = 1.0 + a.alpha * kr2 * a.dt;
         cplx num = cadd(old, rmul(a.dt, t1));
-        if (a.Kn) {
-            const cplx nt = kmasked(kxs, kys, N) ? czero() : rmul(a.sdt, a.Kn[o]);
-            num = cadd(num, nt);
-        }
+        if constexpr (SG) num = cadd(num, kmasked(kxs, kys, N) ? czero() : rmul(a.sdt, nz[s]));
         cplx nw = mk(num.x / t2, num.y / t2);
-        if (a.ktrunc2 > 0.0 && kr2 > a.ktrunc2) nw = czero();
+        if constexpr (SG) {
+            if (a.ktrunc2 > 0.0 && kr2 > a.ktrunc2) nw = czero();
+        }
         K0[o] = nw;
         if (a.want_res) {
             const double dx = nw.x - old.x, dy = nw.y - old.y;
@@ -973,12 +1036,12 @@ __device__ __forceinline__ void a4_body(int blk_, int nblk_, const cplx* __restr
     }
 }
 
-template <class C, int G = C::TC>
+template <class C, int G = C::TC, bool SG = false>
 __global__ void __launch_bounds__(G * C::T) VK_OCC k_a4(const cplx* __restrict__ HN, cplx* __restrict__ Hpsi,
                                                 cplx* __restrict__ K0, const cplx* __restrict__ tw,
                                                 ArgleArgs a, double* __restrict__ part)
 {
-    a4_body<C, G>(blockIdx.x, gridDim.x, HN, Hpsi, K0, tw, a, part);
+    a4_body<C, G, SG>(blockIdx.x, gridDim.x, HN, Hpsi, K0, tw, a, part);
 }
 
 // fixed-order reduction of nb partial records of nv doubles -> out[nv]
@@ -1010,31 +1073,6 @@ struct DiagArgs {
     int N;
     int has_v;
 };
-
-// Sums over a row of nv <= 8 values per point group: thread t of the row's T
-// holds x[]; out[i] = the sum over t in a fixed tree (neighbour pairs, then
-// pairs of pairs, ...), the same in every workgroup shape.  sh: nv * T
-// doubles of LDS of this row.  Every thread of the workgroup calls it.
-template <int NV, int T>
-__device__ __forceinline__ void row_sum(const double (&x)[NV], double* sh, int t, double* __restrict__ out)
-{
-    lds_barrier();
-#pragma unroll
-    for (int i = 0; i < NV; ++i) sh[i * T + t] = x[i];
-#pragma unroll
-    for (int h = 1; h < T; h *= 2) {
-        lds_barrier();
-        if (t % (2 * h) == 0) {
-#pragma unroll
-            for (int i = 0; i < NV; ++i) sh[i * T + t] += sh[i * T + t + h];
-        }
-    }
-    lds_barrier();
-    if (t == 0) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) out[i] = sh[i * T];
-    }
-}
 
 // Row pass of the diagnostics (src/diagnostics.f90:54-317): from the rows of
 // Hpsi, Hdy = IFFT_y(i ky kpsi), Hrhod (and HV) the x-space psi, d_x psi,
@@ -1842,7 +1880,7 @@ __host__ __device__ inline void philox4x32_10(unsigned c[4], unsigned k0, unsign
 // fractions of the 64-bit words, u1 in (0, 1], u2 in [0, 1), then the
 // Box-Muller transform.  The reference draws its pair with the polar method
 // from Fortran's RANDOM_NUMBER; only the distribution is the same.
-__host__ __device__ inline void sgle_normals(unsigned long long i, unsigned long long step, unsigned long long seed,
+__device__ __forceinline__ void sgle_normals(unsigned long long i, unsigned long long step, unsigned long long seed,
                                              double* v1, double* v2)
 {
     unsigned c[4] = {(unsigned)i, (unsigned)(i >> 32), (unsigned)step, (unsigned)(step >> 32)};
@@ -1853,55 +1891,86 @@ __host__ __device__ inline void sgle_normals(unsigned long long i, unsigned long
     const double u2 = (double)(b >> 11) * 0x1.0p-53;
     const double rr = sqrt(-2.0 * log(u1));
     double sn, cs;
-    sincos(6.283185307179586476925 * u2, &sn, &cs);
+    sincospi(2.0 * u2, &sn, &cs);
     *v1 = rr * cs;
     *v2 = rr * sn;
 }
 
-// X = noise field of draw `step`, times (1/sqrt(dvol)) then noisesigma
-// (src/gpe.f90:163), or the caller's standard normals in X scaled in place
-// (gen = 0)
-__global__ void k_sgle_noise(cplx* __restrict__ X, int N, unsigned long long step, unsigned long long seed,
-                             double invsq, double sigma, int gen)
+// X = the standard normals of noise draw `step`
+__global__ void k_sgle_noise(cplx* __restrict__ X, int N, unsigned long long step, unsigned long long seed)
 {
     const size_t n2 = (size_t)N * N;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n2; i += (size_t)gridDim.x * blockDim.x) {
         double v1, v2;
-        if (gen) sgle_normals(i, step, seed, &v1, &v2);
-        else {
-            v1 = X[i].x;
-            v2 = X[i].y;
+        sgle_normals(i, step, seed, &v1, &v2);
+        X[i] = mk(v1, v2);
+    }
+}
+
+struct NoiseArgs {
+    const cplx* X;   // the caller's standard normals, or null: draw `step` of seed
+    cplx* H;
+    unsigned long long step, seed;
+    double invsq, sigma;   // 1/sqrt(dvol), then noisesigma (src/gpe.f90:163)
+    double* om;
+};
+
+// The noise rows of one SGLE step: standard normals, scaled, transformed along
+// x, retained panels stored.
+template <class C>
+__device__ __forceinline__ void noise_row_body(int blk_, int nblk_, const cplx* __restrict__ tw, Geo g,
+                                               const NoiseArgs& a)
+{
+    VK_ROW_SETUP(C)
+    const auto w_ = twiddles<C>(tw, t);
+    if (blk_ == 0 && threadIdx.x == 0) a.om[0] = a.om[1];
+    cplx v[S];
+    if (a.X) {
+        const cplx* xr = a.X + (size_t)y * N;
+#pragma unroll
+        for (int s = 0; s < S; ++s) v[s] = rmul(a.sigma, rmul(a.invsq, xr[t + T * s]));
+    } else {
+        // the generator in a loop, its points passed on through this thread's
+        // own LDS slots (unrolled, it would be S copies of log and sincos)
+        constexpr int Q = S / 2;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll 1
+            for (int s = 0; s < Q; ++s) {
+                double v1, v2;
+                sgle_normals((size_t)y * N + t + T * (h * Q + s), a.step, a.seed, &v1, &v2);
+                const cplx z = rmul(a.sigma, rmul(a.invsq, mk(v1, v2)));
+                lg[s * T + t] = z.x;
+                lg[N / 2 + s * T + t] = z.y;
+            }
+#pragma unroll
+            for (int s = 0; s < Q; ++s) v[h * Q + s] = mk(lg[s * T + t], lg[N / 2 + s * T + t]);
         }
-        X[i] = rmul(sigma, rmul(invsq, mk(v1, v2)));
+        lds_barrier();
+    }
+    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int pp = VK_PANEL(s);
+        if (panel_stored(pp, NP, g, 1)) a.H[hoff<C>(pp, y, c)] = v[s];
     }
 }
 
-// block partial sums of |K|^2 over a k-space field
-__global__ void k_knorm(const cplx* __restrict__ K, size_t n2, double* __restrict__ part)
+// P1 of an SGLE step with its norm sums, and the noise rows, which need
+// nothing of it, as the first half of the same launch: P1's loads and the
+// generator's arithmetic then share the CUs (25 us together at 1024^2, where
+// the generator's 13, the noise rows' 11 and P1's 12 ran one after another).
+// With A4 taking the noise columns and the norm, an SGLE step is 4 launches
+// of 9 and moves no noise through k-space: 128^2 32.0 to 21.9 us, 512^2 56.0
+// to 44.8, 1024^2 88.4 to 64.8, 4096^2 1160 to 960.
+template <class C>
+__global__ void __launch_bounds__(C::ROWT) VK_OCC k_p1_noise(const cplx* __restrict__ Hpsi, cplx* __restrict__ Hrho,
+                                                     const cplx* __restrict__ tw, Geo g, double scale,
+                                                     cplx* __restrict__ Xpsi, double* __restrict__ nsum, NoiseArgs a)
 {
-    __shared__ double sh[16];
-    double acc[1] = {0.0};
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n2; i += (size_t)gridDim.x * blockDim.x) {
-        const cplx z = K[i];
-        acc[0] += z.x * z.x + z.y * z.y;
-    }
-    block_sum<1>(acc, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
-}
-
-// finiteT_adhoc_chempot (src/gpe.f90:255-264): norm = sum_x |psi|^2 dvol =
-// (dvol/N^2) sum_k |psi-hat|^2 (Parseval), omega -= dt (nuN/L^2)(norm - L^2)
-__global__ void k_chempot(const double* __restrict__ part, int nb, double* __restrict__ omega, double dvol_n2,
-                          double dt, double nuN, double L2)
-{
-    __shared__ double sh[16];
-    double acc[1] = {0.0};
-    for (int b = threadIdx.x; b < nb; b += blockDim.x) acc[0] += part[b];
-    block_sum<1>(acc, sh);
-    if (threadIdx.x == 0) {
-        const double norm = acc[0] * dvol_n2;
-        omega[0] = omega[0] - dt * (nuN / L2) * (norm - L2);
-    }
+    const int nb = gridDim.x / 2;
+    if ((int)blockIdx.x < nb) noise_row_body<C>(blockIdx.x, nb, tw, g, a);
+    else p1_body<C, true, true>(blockIdx.x - nb, nb, Hpsi, Hrho, tw, g, 0, scale, Xpsi, nsum);
 }
 
 // ----------------------------------------------------------------------------
