@@ -97,7 +97,9 @@ struct vk_gpe {
     cplx* tw = nullptr;
     // state and RK4/ARGLE work fields
     cplx *K0 = nullptr, *K1 = nullptr, *K2 = nullptr, *Hpsi = nullptr, *Hrho = nullptr, *HN = nullptr;
-    cplx* Xs = nullptr;   // x-space psi rows written by P1 and read by P3
+    // x-space field: psi rows from P1 to P3 within a step, and between steps the
+    // staging of the x-space transforms (all on the handle's stream)
+    cplx* Xs = nullptr;
     int dev = 0;        // device the handle was created on
     int ncu = 0;        // compute units of the device
     int p1pf = 0;       // RK4 P1 as the persistent prefetching kernel (4096^2)
@@ -133,7 +135,7 @@ struct vk_gpe {
     int np_cap = 0;     // particle buffers are sized for this many particles
     int rs_part = 0;   // particle potential and force evaluated in real space inside P3
     // diagnostics
-    cplx *X0 = nullptr, *Kd0 = nullptr;
+    cplx* Kd0 = nullptr;
     cplx* Hd = nullptr;
     double* hres = nullptr;   // pinned: sums and spectra of the last call
     int diag_ready = 0;
@@ -1019,7 +1021,6 @@ void vk_gpe_destroy(vk_gpe* h)
         if (h->Vx) hipFree(h->Vx);
         if (h->pst) hipFree(h->pst);
     }
-    if (h->X0) hipFree(h->X0);
     if (h->Kd0) hipFree(h->Kd0);
     if (h->hres) hipHostFree(h->hres);
     if (h->part) hipFree(h->part);
@@ -1037,9 +1038,8 @@ void vk_gpe_destroy(vk_gpe* h)
 static int sgle_sync_omega(vk_gpe* h);
 static int ensure_hdy(vk_gpe* h);
 
-static int need_x0(vk_gpe* h)
+static int need_hd(vk_gpe* h)
 {
-    if (!h->X0) HIPCHK(hipMalloc(&h->X0, f2(h) * sizeof(cplx)));
     if (!h->Hd) {
         HIPCHK(hipMalloc(&h->Hd, f2(h) * sizeof(cplx)));
         HIPCHK(hipMemset(h->Hd, 0, f2(h) * sizeof(cplx)));
@@ -1047,9 +1047,9 @@ static int need_x0(vk_gpe* h)
     return 0;
 }
 
-static int set_from_x0(vk_gpe* h, int flags)
+static int set_from_xs(vk_gpe* h, int flags)
 {
-    int rc = fwd2d(h, h->X0, h->Hd, h->K0, 0, 0);
+    int rc = fwd2d(h, h->Xs, h->Hd, h->K0, 0, 0);
     if (rc) return rc;
     h->hstate = 0;
     if (flags & VK_SYNC_DEALIAS) {
@@ -1063,12 +1063,12 @@ static int set_from_x0(vk_gpe* h, int flags)
 int vk_gpe_set_psi(vk_gpe* h, const double* psi, int flags)
 {
     if (!h || !psi) return fail(VK_ERR_ARG, "set_psi: null argument");
-    int rc = need_x0(h);
+    int rc = need_hd(h);
     if (rc) return rc;
     // stream-ordered: a device-to-device hipMemcpy does not block the host and
     // is not ordered against this non-blocking stream
-    HIPCHK(hipMemcpyAsync(h->X0, psi, f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
-    return set_from_x0(h, flags);
+    HIPCHK(hipMemcpyAsync(h->Xs, psi, f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
+    return set_from_xs(h, flags);
 }
 
 int vk_gpe_set_kpsi(vk_gpe* h, const double* kpsi)
@@ -1080,21 +1080,41 @@ int vk_gpe_set_kpsi(vk_gpe* h, const double* kpsi)
     return 0;
 }
 
+// whether a kernel of this device may write `bytes` at p as 16 byte values:
+// device memory of the current device, the whole range inside one allocation
+// (what a copy checks)
+static bool kernel_target(const void* p, size_t bytes)
+{
+    hipPointerAttribute_t a;
+    hipDeviceptr_t base = nullptr;
+    size_t n = 0;
+    int dev = -1;
+    if ((uintptr_t)p % 16 == 0 && hipGetDevice(&dev) == hipSuccess && hipPointerGetAttributes(&a, p) == hipSuccess &&
+        a.type == hipMemoryTypeDevice && a.device == dev &&
+        hipMemGetAddressRange(&base, &n, const_cast<void*>(p)) == hipSuccess)
+        return (const char*)p - (const char*)base + bytes <= n;
+    (void)hipGetLastError();
+    return false;
+}
+
+// psi goes straight into a caller's device buffer (16 us a 128..512^2 field
+// instead of 35 with a copy and a wait between); other memory through Xs
 int vk_gpe_get_psi(vk_gpe* h, double* psi, double* kpsi)
 {
     if (!h) return fail(VK_ERR_ARG, "get_psi: null handle");
     int rc;
     if (psi) {
-        if ((rc = need_x0(h))) return rc;
+        const size_t bytes = f2(h) * sizeof(cplx);
+        const bool direct = kernel_target(psi, bytes);
+        if (!direct && (rc = need_hd(h))) return rc;
         if ((rc = ensure_any(h))) return rc;
-        if ((rc = row_inv(h, h->Hpsi, h->X0, h->hstate == 2 ? 1 : 0, 0, scale_of(h)))) return rc;
-        HIPCHK(hipStreamSynchronize(h->stream));
+        cplx* x = direct ? reinterpret_cast<cplx*>(psi) : h->Xs;
+        if ((rc = row_inv(h, h->Hpsi, x, h->hstate == 2 ? 1 : 0, 0, scale_of(h)))) return rc;
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(psi, h->X0, f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
+        if (!direct) HIPCHK(hipMemcpyAsync(psi, x, bytes, hipMemcpyDefault, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
     }
     if (kpsi) {
-        HIPCHK(hipStreamSynchronize(h->stream));
         HIPCHK(hipMemcpyAsync(kpsi, h->K0, f2(h) * sizeof(cplx), hipMemcpyDefault, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
     }
@@ -1175,8 +1195,8 @@ static int particle_potential(vk_gpe* h)
 {
     const double pi = 4.0 * std::atan(1.0);
     const double L = 2.0 * pi, dx = L / h->N, c1 = 2 * pi / (2.0 * L);
-    hipLaunchKernelGGL(vk::k_pot_x, dim3(1024), dim3(256), 0, h->stream, h->X0, h->N, dx, c1, h->p.V0, h->p.d);
-    int rc = fwd2d(h, h->X0, h->Hd, h->Vhat, 0, 1);
+    hipLaunchKernelGGL(vk::k_pot_x, dim3(1024), dim3(256), 0, h->stream, h->Xs, h->N, dx, c1, h->p.V0, h->p.d);
+    int rc = fwd2d(h, h->Xs, h->Hd, h->Vhat, 0, 1);
     if (rc) return rc;
     h->have_part = 1;
     return 0;
@@ -1187,7 +1207,7 @@ int vk_gpe_particles_set(vk_gpe* h, const double* pos, const double* vel, const 
     if (!h) return fail(VK_ERR_ARG, "particles_set: null handle");
     const int np = h->p.np;
     if (np <= 0) return fail(VK_ERR_STATE, "particles_set: handle created with np = 0");
-    int rc = need_x0(h);
+    int rc = need_hd(h);
     if (rc) return rc;
     // steps queued by vk_gpe_rk4_steps_async read and write the particle
     // state (the side-stream updates are joined into h->stream at the end of
@@ -1307,7 +1327,7 @@ int vk_gpe_set_sgle(vk_gpe* h, int on, double oneybeta, double nuN, double chemp
         h->sgle = 0;
         return 0;
     }
-    int rc = need_x0(h);
+    int rc = need_hd(h);
     if (rc) return rc;
     if (!h->Xn) HIPCHK(hipMalloc(&h->Xn, f2(h) * sizeof(cplx)));
     if (!h->omega_dev) HIPCHK(hipMalloc(&h->omega_dev, 2 * sizeof(double)));
@@ -1394,7 +1414,7 @@ int vk_gpe_set_obstacles(vk_gpe* h, int np, const double* pos, double V0, double
         return fail(VK_ERR_ARG, "set_obstacles: np must be in [0, np of the params the handle was created with]");
     if (np > 0 && (!pos || !(d > 0.0) || !std::isfinite(V0)))
         return fail(VK_ERR_ARG, "set_obstacles: positions, d > 0 and a finite V0 are required");
-    int rc = need_x0(h);
+    int rc = need_hd(h);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(h->stream));
     h->p.np = np;
@@ -1428,23 +1448,23 @@ int vk_gpe_particles_get(vk_gpe* h, double* pos, double* vel, double* frc)
 int vk_fft2d(vk_gpe* h, int dir, const double* in, double* out)
 {
     if (!h || !in || !out || (dir != -1 && dir != 1)) return fail(VK_ERR_ARG, "fft2d: bad arguments");
-    int rc = need_x0(h);
+    int rc = need_hd(h);
     if (rc) return rc;
     if (!h->Kd0) HIPCHK(hipMalloc(&h->Kd0, f2(h) * sizeof(cplx)));
     const size_t fb = f2(h) * sizeof(cplx);
     if (dir < 0) {
-        HIPCHK(hipMemcpy(h->X0, in, fb, hipMemcpyHostToDevice));
-        if ((rc = fwd2d(h, h->X0, h->Hd, h->Kd0, 0, 0))) return rc;
+        HIPCHK(hipMemcpyAsync(h->Xs, in, fb, hipMemcpyHostToDevice, h->stream));
+        if ((rc = fwd2d(h, h->Xs, h->Hd, h->Kd0, 0, 0))) return rc;
         HIPCHK(hipStreamSynchronize(h->stream));
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpy(out, h->Kd0, fb, hipMemcpyDeviceToHost));
     } else {
         HIPCHK(hipMemcpy(h->Kd0, in, fb, hipMemcpyHostToDevice));
         if ((rc = col_inv(h, h->Kd0, h->Hd, 0, 0))) return rc;
-        if ((rc = row_inv(h, h->Hd, h->X0, 0, 0, scale_of(h)))) return rc;
+        if ((rc = row_inv(h, h->Hd, h->Xs, 0, 0, scale_of(h)))) return rc;
         HIPCHK(hipStreamSynchronize(h->stream));
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpy(out, h->X0, fb, hipMemcpyDeviceToHost));
+        HIPCHK(hipMemcpy(out, h->Xs, fb, hipMemcpyDeviceToHost));
     }
     return 0;
 }
@@ -1492,7 +1512,7 @@ int vk_ic_vortices_host(int N, int nv, const double* xs, const double* ys, const
 int vk_gpe_set_ic_vortices(vk_gpe* h, int nv, const double* xs, const double* ys, const int* qs, int nimg, int flags)
 {
     if (!h || nv < 0 || (nv > 0 && (!xs || !ys || !qs))) return fail(VK_ERR_ARG, "set_ic_vortices: bad arguments");
-    int rc = need_x0(h);
+    int rc = need_hd(h);
     if (rc) return rc;
     double *dx = nullptr, *dy = nullptr;
     int* dq = nullptr;
@@ -1505,14 +1525,14 @@ int vk_gpe_set_ic_vortices(vk_gpe* h, int nv, const double* xs, const double* ys
         HIPCHK(hipMemcpy(dy, ys, sizeof(double) * nv, hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(dq, qs, sizeof(int) * nv, hipMemcpyHostToDevice));
     }
-    hipLaunchKernelGGL(vk::k_ic, dim3(2048), dim3(256), 0, h->stream, h->X0, h->N, nv, (const double*)dx,
+    hipLaunchKernelGGL(vk::k_ic, dim3(2048), dim3(256), 0, h->stream, h->Xs, h->N, nv, (const double*)dx,
                        (const double*)dy, (const int*)dq, h->p.xi, nimg);
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipGetLastError());
     hipFree(dx);
     hipFree(dy);
     hipFree(dq);
-    return set_from_x0(h, flags);
+    return set_from_xs(h, flags);
 }
 
 void* vk_gpe_stream(vk_gpe* h) { return h ? (void*)h->stream : nullptr; }
