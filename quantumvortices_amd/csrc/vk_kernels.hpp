@@ -1085,7 +1085,10 @@ struct DiagArgs {
 // (this pairing lets each direction's pair go before the next one's gradient
 // is formed; w_x with w_y would hold 64 registers more and spill 240).
 // Six transforms per row.  4096^2: 0.8 GB against the 5.4 GB of separate
-// transforms and a pointwise pass over x-space arrays (1.5 ms).
+// transforms and a pointwise pass over x-space arrays (1.5 ms).  0.42 ms, bound
+// by the transforms (0.05 ms each at full occupancy): with the directions
+// unrolled and index arithmetic shared by the transforms 96 registers spilled,
+// 0.56 ms.
 template <class C>
 __device__ __forceinline__ void diag_row_body(int blk_, int nblk_, const cplx* __restrict__ Hpsi,
                                               const cplx* __restrict__ Hdy, const cplx* __restrict__ Hrhod,
@@ -1124,7 +1127,7 @@ __device__ __forceinline__ void diag_row_body(int blk_, int nblk_, const cplx* _
         }
     };
     load(rH, false);
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    fft_fwd<N, S, C::SPLIT>(v, lg, again(t), w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) ps[s] = rmul(scale, conjc(v[s]));
     // P_G rho + i V from the kx >= 0 halves
@@ -1142,7 +1145,7 @@ __device__ __forceinline__ void diag_row_body(int blk_, int nblk_, const cplx* _
         }
         v[s] = conjc(mk(z.x - zv.y, z.y + zv.x));
     }
-    fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+    fft_fwd<N, S, C::SPLIT>(v, lg, again(t), w_);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const double pr = scale * v[s].x, ap2 = ps[s].x * ps[s].x + ps[s].y * ps[s].y;
@@ -1151,10 +1154,9 @@ __device__ __forceinline__ void diag_row_body(int blk_, int nblk_, const cplx* _
         if (a.has_v) acc[5] += (-scale * v[s].y) * pr;
         acc[6] += ap2;
     }
-#pragma unroll
-    for (int dir = 0; dir < 2; ++dir) {
+    auto direction = [&](int dir) {
         load(dir == 0 ? rH : rD, dir == 0);
-        fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+        fft_fwd<N, S, C::SPLIT>(v, lg, again(t), w_);
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             const cplx d = rmul(scale, conjc(v[s]));
@@ -1168,7 +1170,7 @@ __device__ __forceinline__ void diag_row_body(int blk_, int nblk_, const cplx* _
             // one point's square root and division at a time
             if constexpr (!is_lat<C>::value) __builtin_amdgcn_sched_barrier(0);
         }
-        fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+        fft_fwd<N, S, C::SPLIT>(v, lg, again(t), w_);
         const brsrc ro = mkbuf(dir == 0 ? H1 : H2, N);
         const int p0 = again(pidx0);
 #pragma unroll
@@ -1176,6 +1178,13 @@ __device__ __forceinline__ void diag_row_body(int blk_, int nblk_, const cplx* _
             const int pp = p0 + (T / TC) * s;
             bst(ro, boff(hoff<C>(pp, y, c), panel_stored(pp, NP, g, 1)), v[s]);
         }
+    };
+    if constexpr (is_lat<C>::value) {
+        direction(0);
+        direction(1);
+    } else {
+#pragma unroll 1
+        for (int dir = 0; dir < 2; ++dir) direction(dir);   // rolled, nothing spills
     }
     row_sum<7, T>(acc, lg, t, rsum + 8 * (size_t)y);
 }
@@ -1205,8 +1214,8 @@ __device__ __forceinline__ int shell_end(int m, int kx)
 // share the first five.  The shells of a column are runs of ky, so each
 // shell's sum is one thread's, in order of |ky|; part[kx][6][spec_shells],
 // entries m >= kx, summed over the columns by spec_reduce_body.
-// 4096^2: 0.6 GB in order, against a gather of 16-byte values by shell lists
-// (0.42 ms) after eight transforms.
+// 4096^2: 0.6 GB in order, 0.28 ms, against a gather of 16-byte values by shell
+// lists (0.42 ms) after eight transforms.
 template <class C, int G = C::TC>
 __device__ __forceinline__ void diag_col_body(int b, cplx* __restrict__ H1, const cplx* __restrict__ H2,
                                               const cplx* __restrict__ K0, const cplx* __restrict__ Krho,
@@ -1233,6 +1242,10 @@ __device__ __forceinline__ void diag_col_body(int b, cplx* __restrict__ H1, cons
                 pk[q * MS + m] = x;
             }
     };
+    auto again = [&](int q) {   // index arithmetic formed anew per transform
+        if constexpr (!is_lat<C>::value) asm volatile("" : "+v"(q));
+        return q;
+    };
     cplx v[S], um[S];
     // the transforms of the two real fields packed in H: v, um
     auto pair = [&](const cplx* H) {
@@ -1242,9 +1255,9 @@ __device__ __forceinline__ void diag_col_body(int b, cplx* __restrict__ H1, cons
             v[s] = bld(rb, boff(hoff<C>(p, t + T * s, c), live));
             um[s] = bld(rb, boff(hoff<C>(km / TC, t + T * s, km % TC), live));
         }
-        fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
+        fft_fwd<N, S, C::SPLIT>(v, lg, again(t), w_);
         lds_barrier();
-        fft_fwd<N, S, C::SPLIT>(um, lg, t, w_);
+        fft_fwd<N, S, C::SPLIT>(um, lg, again(t), w_);
         lds_barrier();
         // um at -ky
 #pragma unroll
@@ -1267,18 +1280,30 @@ __device__ __forceinline__ void diag_col_body(int b, cplx* __restrict__ H1, cons
     auto sq = [](cplx z) { return z.x * z.x + z.y * z.y; };
     double e[3][S];
     // w_x, q_x: w_x waits in its column of H1, this workgroup's alone
-    pair(H1);
-#pragma unroll
-    for (int s = 0; s < S; ++s) e[2][s] = mult * sq(um[s]);
     const brsrc r1 = mkbuf(H1, N);
 #pragma unroll
-    for (int s = 0; s < S; ++s) bst(r1, boff(hoff<C>(p, t + T * s, c), live), v[s]);
-    lds_barrier();
-    pair(H2);
+    for (int s = 0; s < S; ++s) e[2][s] = 0.0;
+    auto direction = [&](int dir) {
+        pair(dir == 0 ? H1 : H2);
+#pragma unroll
+        for (int s = 0; s < S; ++s) e[2][s] += mult * sq(um[s]);
+        if (dir == 0) {
+#pragma unroll
+            for (int s = 0; s < S; ++s) bst(r1, boff(hoff<C>(p, t + T * s, c), live), v[s]);
+            lds_barrier();
+        }
+    };
+    if constexpr (is_lat<C>::value) {
+        direction(0);
+        direction(1);
+    } else {
+#pragma unroll 1
+        for (int dir = 0; dir < 2; ++dir) direction(dir);
+    }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const bool use = live && !kmasked(kx, ksg(t + T * s, N), N);
-        e[2][s] = use ? e[2][s] + mult * sq(um[s]) : 0.0;
+        if (!use) e[2][s] = 0.0;
         um[s] = bld(r1, boff(hoff<C>(p, t + T * s, c), live));
     }
     bin(e[2], 3);
@@ -1364,8 +1389,10 @@ __global__ void __launch_bounds__(C::ROWT) k_p1d(const cplx* __restrict__ Hpsi, 
     p1_body<C, false>(blockIdx.x, gridDim.x, Hpsi, Hrho, tw, g, psi_pmode, scale, nullptr);
 }
 
-// two waves per SIMD (<= 256 VGPRs); the LAT shapes one
-#define VK_DIAGOCC(C) __attribute__((amdgpu_waves_per_eu(is_lat<C>::value ? 1 : 2)))
+// waves per SIMD: two (<= 256 VGPRs) with 16 points per thread, with 8 what
+// whole workgroups fill (T/256 waves per SIMD each); the LAT shapes one
+#define VK_DIAGOCC(C) \
+    __attribute__((amdgpu_waves_per_eu(is_lat<C>::value ? 1 : C::S == 16 ? 2 : C::T == 512 ? 4 : 3)))
 
 template <class C>
 __global__ void __launch_bounds__(C::ROWT) VK_DIAGOCC(C)
