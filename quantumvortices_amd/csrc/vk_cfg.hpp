@@ -89,6 +89,18 @@ template <> struct CfgS<1024> : CfgT<1024, 16, 4, 1, false> { static constexpr i
 template <class C, class = void> struct is_lat { static constexpr bool value = false; };
 template <class C> struct is_lat<C, decltype((void)C::LAT)> { static constexpr bool value = C::LAT; };
 
+// Shapes of the diagnostics' spectra pass, a long serial chain per column (four
+// transforms, six shell sums) over a third of the columns: from 256^2 on 8
+// points per thread, twice the threads per column of Cfg<N>, in its layout.
+// L: a single field's, up to 1024^2 as the LAT shapes, one wave or two per
+// workgroup; else the ensemble's.
+// 1024^2: 30 us against 37 with 16 points (diagnostics 113 to 107, 512^2 90 to 80,
+// 256^2 76 to 67); 4096^2 282 against 315.  128 members of 512^2 1.91 to 1.81 ms.
+template <int N, bool L> struct CfgD : CfgT<N, 8, Cfg<N>::TC, 1, (N >= 2048)> {
+    static constexpr bool LAT = L && N <= 1024;
+    static constexpr int G = LAT ? (N >= 512 ? 1 : 512 / N) : (N >= 2048 ? 1 : 2048 / N);
+};
+
 // twiddles of this thread: in registers for the LAT shapes, else the table
 template <class C> __device__ __forceinline__ auto twiddles(const cplx* __restrict__ tw, int t)
 {

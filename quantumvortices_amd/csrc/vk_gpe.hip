@@ -754,13 +754,6 @@ vk::DiagArgs diag_args(const vk_gpe* h, int has_v)
     return vk::DiagArgs{h->p.alpha, h->p.omega, h->p.g, (double)1e-30f, h->N, has_v};
 }
 
-// columns per workgroup of the spectra pass: workgroups of 256 threads
-template <class C> constexpr int diag_cols()
-{
-    if constexpr (vk::is_lat<C>::value) return C::G;
-    else return C::T >= 256 ? 1 : 256 / C::T;
-}
-
 // the diagnostics' device work on h->stream: the energy sums and the six
 // spectra to out (8 + 6 (nshell + 1) doubles the device can write), particle
 // diagnostics in the particle state
@@ -784,11 +777,8 @@ int diag_launch(vk_gpe* h, double* out)
         p2_launch<C>(h, h->Hrho, h->HV, (const cplx*)h->KV, h->Krho, tw, h->geo, parts ? 3 : 2);
         row_launch<C1>(h, PK_OTHER, vk::k_diag_row<C1>, (const cplx*)h->Hpsi, (const cplx*)h->Hd, (const cplx*)h->Hrho,
                        (const cplx*)h->HV, H1, H2, tw, h->geo, pl, sc, diag_args(h, parts), diag_rsum(h));
-        // from 2048^2 on the spectra pass holds 8 points per thread, twice the
-        // threads (four waves per SIMD at 4096^2): 0.282 ms against 0.315 with 16
-        // points and two waves; the row pass with 8 points 0.55 against 0.42
-        using CC = std::conditional_t<(C::N >= 2048), vk::CfgT<C::N, 8, C::TC, 1, true>, C>;
-        constexpr int G = diag_cols<CC>();
+        using CC = std::conditional_t<(C::N >= 256), vk::CfgD<C::N, true>, C>;
+        constexpr int G = CC::G;
         colg_launch<CC, G>(h, PK_OTHER, h->geo.Pp, vk::k_diag_col<CC, G>, H1, (const cplx*)H2,
                           (const cplx*)h->K0, (const cplx*)h->Krho, tw, h->geo, diag_part(h));
         return 0;
@@ -2011,6 +2001,13 @@ int col_inv_var(vk_gpe* h, int var)
 // stream has passed the copy.
 size_t ens_diag_tab_bytes(size_t n) { return n * sizeof(vk::DiagB); }
 
+// columns per workgroup of the ensemble's spectra pass
+template <class C, class CC> constexpr int diag_cols()
+{
+    if constexpr (C::N >= 256) return CC::G;
+    else return C::TC;
+}
+
 template <class C>
 int ens_diag_group(const std::vector<vk_gpe*>& hs, int pl, hipStream_t st, void* tab, void* htab,
                    const std::vector<double*>& out)
@@ -2033,13 +2030,17 @@ int ens_diag_group(const std::vector<vk_gpe*>& hs, int pl, hipStream_t st, void*
     set_lds(vk::k_diag_row_b<C>, rl);
     set_lds(vk::k_diag_dy_b<C>, cl);
     set_lds(vk::k_p2d_b<C>, cl);
-    set_lds(vk::k_diag_col_b<C>, cl);
+    using CC = std::conditional_t<(C::N >= 256), vk::CfgD<C::N, false>, C>;
+    constexpr int GC = diag_cols<C, CC>(), GS = C::TC / GC;
+    const size_t ccl = (size_t)GC * CC::COLRS * sizeof(double);
+    set_lds(vk::k_diag_col_b<CC, GC>, ccl);
     const dim3 rg(C::N / C::TR, n), rb(C::ROWT), cb(C::COLT);
     hipLaunchKernelGGL(vk::k_diag_dy_b<C>, dim3(pl == 1 ? g.Pp + g.Pn : C::NP, n), cb, cl, st, dd, tw, g, pl);
     hipLaunchKernelGGL(vk::k_p1d_b<C>, rg, rb, rl, st, dd, tw, g, pl, sc);
     hipLaunchKernelGGL(vk::k_p2d_b<C>, dim3(g.Pp, n), cb, cl, st, dd, tw, g);
     hipLaunchKernelGGL(vk::k_diag_row_b<C>, rg, rb, rl, st, dd, tw, g, pl, sc);
-    hipLaunchKernelGGL(vk::k_diag_col_b<C>, dim3(g.Pp, n), cb, cl, st, dd, tw, g);
+    hipLaunchKernelGGL((vk::k_diag_col_b<CC, GC>), dim3(GS == 1 ? g.Pp : (g.Pp + 7) / 8 * 8 * GS, n), dim3(GC * CC::T),
+                       ccl, st, dd, tw, g);
     hipLaunchKernelGGL(vk::k_spec_reduce_b, dim3(h0->nshell / 64 + 1, 7, n), dim3(64 * vk::SPEC_G), 0, st, dd);
     return 0;
 }

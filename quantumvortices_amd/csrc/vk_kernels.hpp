@@ -1478,12 +1478,12 @@ k_diag_row_b(const DiagB* __restrict__ D, const cplx* __restrict__ tw, Geo g, in
     diag_row_body<C>(blockIdx.x, gridDim.x, d.Hpsi, d.Hd, d.Hrho, nullptr, d.H1, d.H2, tw, g, pl, scale, d.da, d.rsum);
 }
 
-template <class C>
-__global__ void __launch_bounds__(C::COLT) VK_DIAGOCC(C)
+template <class C, int G>
+__global__ void __launch_bounds__(G * C::T) VK_DIAGOCC(C)
 k_diag_col_b(const DiagB* __restrict__ D, const cplx* __restrict__ tw, Geo g)
 {
     const DiagB& d = D[blockIdx.y];
-    diag_col_body<C>(blockIdx.x, d.H1, d.H2, d.K0, d.Krho, tw, g, d.part);
+    diag_col_body<C, G>(blockIdx.x, d.H1, d.H2, d.K0, d.Krho, tw, g, d.part);
 }
 
 __global__ void __launch_bounds__(64 * SPEC_G) k_spec_reduce_b(const DiagB* __restrict__ D)
