@@ -921,13 +921,15 @@ int vk_gpe_create(vk_gpe** out, const vk_gpe_params* p)
         h->p1pf = p1_prefetch_ok(h);
         const char* t1 = std::getenv("VK_P1_TR1");
         const char* t3 = std::getenv("VK_P3_TR1");
-        // Measured defaults: one row per workgroup in P1 and P3 at 2048^2
-        // and 4096^2 (both with 4-column panels: 64-byte row pieces); 13%
-        // faster per step than four rows at 2048^2, 3% than two at 4096^2.
+        // Measured defaults (4-column panels: 64-byte row pieces), ms per step
+        // with 32 particles / without: at 2048^2 one row per workgroup in P1
+        // and P3, 0.552 / 0.507 (four rows in P3 0.580 / 0.527, in both 0.636 /
+        // 0.590); at 4096^2 one row in P1 and two in P3, 2.056 / 2.013 (one in
+        // both 2.092 / 2.050, two in both 2.111 / 2.068).
         // VK_P1_TR1 / VK_P3_TR1 = 0 or 1 override; vk_gpe_autotune_rows
         // times every pair on the device at hand.
         h->tr1_p1 = t1 ? t1[0] == '1' : (N == 4096 || N == 2048);
-        h->tr1_p3 = t3 ? t3[0] == '1' : (N == 4096 || N == 2048);
+        h->tr1_p3 = t3 ? t3[0] == '1' : N == 2048;
     }
     if (hipMalloc(&h->Xs, fb) != hipSuccess) return cleanup(fail(VK_ERR_HIP, "hipMalloc failed (psi rows)"));
     if (hipMalloc(&h->tw, sizeof(cplx) * N) != hipSuccess) return cleanup(fail(VK_ERR_HIP, "hipMalloc tw"));
