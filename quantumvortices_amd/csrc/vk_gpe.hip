@@ -281,6 +281,18 @@ void colg_launch(vk_gpe* h, int kind, int npan, Kern k, A... args)
     ev_end(h, kind);
 }
 
+// P4 after the workgroups of the particles' update
+template <class C, int G, class Kern>
+void p4_part_launch(vk_gpe* h, Kern k, const vk::RKArgs& a, const vk::PStage& q)
+{
+    constexpr int GS = C::TC / G;
+    const size_t lds = (size_t)G * C::COLRS * sizeof(double);
+    set_lds(k, lds);
+    const int npan = h->geo.Pp + h->geo.Pn, grid = GS == 1 ? npan : (npan + 7) / 8 * 8 * GS;
+    hipLaunchKernelGGL(k, dim3((h->p.np + 7) / 8 * 8 + grid), dim3(G * C::T), lds, h->stream, (const cplx*)h->HN,
+                       h->Hpsi, h->K0, h->K1, h->K2, (const cplx*)h->tw, h->geo, a, q);
+}
+
 // the flags (last argument, 0..3) select a compile-time instantiation
 template <class C>
 void p2_launch(vk_gpe* h, cplx* Hrho, cplx* HV, const cplx* KV, cplx* Krho, const cplx* tw, Geo g, int flags)
@@ -545,7 +557,15 @@ int particle_forces(vk_gpe* h, const cplx* Krho, int nrows, int half, int stage)
 // Particle stage update from the real-space block partials written by P3; the
 // next P3 needs its window tables.  From 2048^2 on it runs on a side stream
 // while P4, P1, P2 proceed (0.1 ms of passes hide it); below, the two event
-// waits would cost more than the update itself (6 us).
+// waits would cost more than the update itself (6 us), and it goes with P4
+// (vk::k_p4_part) where P4's workgroups are whole waves.
+vk::PStage pstage_args(vk_gpe* h, int nblk, int nw, int stage)
+{
+    double *cur = stage % 2 ? h->pst : h->pst2, *nxt = stage % 2 ? h->pst2 : h->pst;
+    return vk::PStage{h->fpart, h->phit, cur, nxt, h->pst, part_args(h, 0, 0, stage, nblk, nw), wtab(h)};
+}
+
+template <int NT>
 int particle_step_rs(vk_gpe* h, int nblk, int nw, int stage)
 {
     const bool side = !h->timing && h->pstream && h->N >= 2048;
@@ -555,10 +575,7 @@ int particle_step_rs(vk_gpe* h, int nblk, int nw, int stage)
         hipStreamWaitEvent(h->pstream, h->ev_p3, 0);
     }
     ev_begin(h);
-    double *cur = stage % 2 ? h->pst : h->pst2, *nxt = stage % 2 ? h->pst2 : h->pst;
-    hipLaunchKernelGGL(vk::k_pstage, dim3(h->p.np), dim3(256), 0, st, (const double*)h->fpart,
-                       (const unsigned char*)h->phit, (const double*)cur, nxt, h->pst,
-                       part_args(h, 0, 0, stage, nblk, nw), wtab(h));
+    hipLaunchKernelGGL(vk::k_pstage<NT>, dim3(h->p.np), dim3(NT), 0, st, pstage_args(h, nblk, nw, stage));
     ev_end(h, PK_PART);
     if (side) {
         hipEventRecord(h->ev_ps, h->pstream);
@@ -623,16 +640,28 @@ int rk4_step(vk_gpe* h)
                 row_launch_x<C>(h, PK_P3, p3_extra(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV,
                                 (const cplx*)h->Xs, h->HN, (const cplx*)h->tw, h->geo, 1, h->p.g * sc, sc, 1.0, pa);
             }
-            if (rs) {
-                if (VAR && h->tr1_p3) particle_step_rs(h, C::N, (C1::ROWT + 63) / 64, stage);
-                else particle_step_rs(h, C::N / C::TR, (C::ROWT + 63) / 64, stage);
+            constexpr int G4 = p4_cols<C>();
+            // up to 1024^2 the particles' update goes with P4 (timed passes: alone)
+            constexpr bool WITH_P4 = !VAR && G4 * C::T >= 64;
+            constexpr int PT = WITH_P4 ? G4 * C::T : 256;
+            const bool with_p4 = WITH_P4 && rs && !h->timing;
+            if (rs && !with_p4) {
+                if (VAR && h->tr1_p3) particle_step_rs<PT>(h, C::N, (C1::ROWT + 63) / 64, stage);
+                else particle_step_rs<PT>(h, C::N / C::TR, (C::ROWT + 63) / 64, stage);
             }
             a.stage = stage;
             a.wacc = (stage == 1 || stage == 4) ? dt * oney6 : dt * oney6 * 2.0;
             a.cstep = stage == 3 ? dt : dt * 0.5;
             a.r1 = (dt * oney6) / (dt * 0.5);
             a.r3 = (dt * oney6 * 2.0) / dt;
-            constexpr int G4 = p4_cols<C>();
+            if constexpr (WITH_P4) {
+                if (with_p4) {
+                    auto kp = stage == 1 ? vk::k_p4_part<C, 1, G4> : stage == 2 ? vk::k_p4_part<C, 2, G4>
+                                         : stage == 3 ? vk::k_p4_part<C, 3, G4> : vk::k_p4_part<C, 4, G4>;
+                    p4_part_launch<C, G4>(h, kp, a, pstage_args(h, C::N / C::TR, (C::ROWT + 63) / 64, stage));
+                    continue;
+                }
+            }
             auto k4 = stage == 1 ? vk::k_p4<C, 1, G4> : stage == 2 ? vk::k_p4<C, 2, G4>
                                                       : stage == 3 ? vk::k_p4<C, 3, G4> : vk::k_p4<C, 4, G4>;
             colg_launch<C, G4>(h, PK_P4, h->geo.Pp + h->geo.Pn, k4, (const cplx*)h->HN, h->Hpsi, h->K0, h->K1,

@@ -1808,13 +1808,27 @@ __global__ void __launch_bounds__(PSTEP_T) k_pstep(const double* __restrict__ fp
 // `nxt` (pos(2np) vel(2np) each; four stages end where they began).
 // Separate force, update and table kernels took 12 us of a 512^2 stage; this
 // one 6.
-__global__ void __launch_bounds__(256) k_pstage(const double* __restrict__ ppart, const unsigned char* __restrict__ phit,
-                                                const double* __restrict__ cur, double* __restrict__ nxt,
-                                                double* __restrict__ st, PartArgs a, WTab w)
+struct PStage {
+    const double* ppart;
+    const unsigned char* phit;
+    const double* cur;
+    double *nxt, *st;
+    PartArgs a;
+    WTab w;
+};
+
+template <int NT>
+__device__ __forceinline__ void pstage_body(int p, const PStage& q)
 {
-    __shared__ double sh[4 * 4];
+    static_assert(NT >= 64, "whole waves");
+    __shared__ double sh[4 * NT / 64];
     __shared__ double pnew[2];
-    const int np = a.np, p = blockIdx.x, tid = threadIdx.x;
+    const double *ppart = q.ppart, *cur = q.cur;
+    const unsigned char* phit = q.phit;
+    double *nxt = q.nxt, *st = q.st;
+    const PartArgs& a = q.a;
+    const WTab& w = q.w;
+    const int np = a.np, tid = threadIdx.x;
     const double *pos = cur, *vel = cur + 2 * np;
     double* fext = st + 4 * np;
     double* tpos = st + 6 * np;
@@ -1842,7 +1856,7 @@ __global__ void __launch_bounds__(256) k_pstage(const double* __restrict__ ppart
             acc[3] += -a.rf * sin(y) / den;
         }
     }
-    for (int b = tid; b < a.nblk; b += 256) {
+    for (int b = tid; b < a.nblk; b += NT) {
         if (!phit[(size_t)b * np + p]) continue;
         for (int v = 0; v < a.nw; ++v) {
             acc[0] += ppart[(((size_t)b * a.nw + v) * np + p) * 2];
@@ -1876,7 +1890,29 @@ __global__ void __launch_bounds__(256) k_pstage(const double* __restrict__ ppart
         }
     }
     __syncthreads();
-    window_table(w, p, tid / 128, pnew[tid / 128], a.N, tid % 128, 128);
+    constexpr int H = NT / 2;
+    window_table(w, p, tid / H, pnew[tid / H], a.N, tid % H, H);
+}
+
+template <int NT> __global__ void __launch_bounds__(NT) k_pstage(PStage q) { pstage_body<NT>(blockIdx.x, q); }
+
+// P4 with the particles' update, which it does not touch, as the first
+// workgroups of its launch (a multiple of eight, so that P4's keep their XCDs).
+// us per step with a launch of its own for the update, then so: 128^2 with 8
+// particles 119 and 105, 512^2 162 and 141, 1024^2 221 and 195, with 64 268 and
+// 239.
+template <class C, int STAGE, int G>
+__global__ void __launch_bounds__(G * C::T) VK_OCC k_p4_part(const cplx* __restrict__ HN, cplx* __restrict__ Hpsi,
+                                                     cplx* __restrict__ K0, cplx* __restrict__ K1,
+                                                     cplx* __restrict__ K2, const cplx* __restrict__ tw, Geo g,
+                                                     RKArgs a, PStage q)
+{
+    const int n = (q.a.np + 7) / 8 * 8;
+    if ((int)blockIdx.x < n) {
+        if ((int)blockIdx.x < q.a.np) pstage_body<G * C::T>(blockIdx.x, q);
+        return;
+    }
+    p4_body<C, STAGE, G>(blockIdx.x - n, gridDim.x - n, HN, Hpsi, K0, K1, K2, tw, g, a);
 }
 
 // ----------------------------------------------------------------------------
