@@ -94,7 +94,9 @@ __global__ void __launch_bounds__(G * C::T) k_sts_time(const cplx* __restrict__ 
 // one shell x 64 frequencies; wave j sums modes off[sh]+j, +BW, ... in list
 // order and the BW partial sums are added in wave order (a fixed order:
 // the result does not depend on scheduling).
-constexpr int BW = 4;
+// Eight waves: 512^2 x 256 39 us against 47 with four, 256^2 x 512 19 and 21.5,
+// 128^2 x 64 7.8 and 10; 128^2 x 2048 18 either way (at HBM's rate).
+constexpr int BW = 8;
 __global__ void __launch_bounds__(64 * BW) k_sts_bin(const double* __restrict__ P, const int* __restrict__ off,
                                                    int nsh, int Nt, double* __restrict__ spec)
 {
