@@ -1507,8 +1507,10 @@ int vk_fno_get_params(vk_fno* f, float* p)
 int vk_fno_get_grad(vk_fno* f, float* gout)
 {
     if (!f || !gout) return vk_set_error(VK_ERR_ARG, "fno_get_grad: null");
+    // on f->st: a plain copy into device memory neither blocks the host nor is
+    // ordered against this non-blocking stream, and the next step rewrites g
+    FCHK(hipMemcpyAsync(gout, f->g, f->np * 4, hipMemcpyDefault, f->st));
     FCHK(hipStreamSynchronize(f->st));
-    FCHK(hipMemcpy(gout, f->g, f->np * 4, hipMemcpyDefault));
     return 0;
 }
 
