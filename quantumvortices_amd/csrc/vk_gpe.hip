@@ -1130,6 +1130,9 @@ int vk_gpe_get_psi(vk_gpe* h, double* psi, double* kpsi)
     int rc;
     if (psi) {
         const size_t bytes = f2(h) * sizeof(cplx);
+        // an error of the steps queued so far: kernel_target's query leaves and
+        // clears one of its own for host memory
+        HIPCHK(hipGetLastError());
         const bool direct = kernel_target(psi, bytes);
         if (!direct && (rc = need_hd(h))) return rc;
         if ((rc = ensure_any(h))) return rc;
