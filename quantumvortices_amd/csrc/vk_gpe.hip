@@ -9,6 +9,7 @@
 // kpsi is dealiased, so only |kx| <= N/3 columns are stored and moved;
 // rho, rho_d and V are real, so only their kx >= 0 halves are moved.
 #include "vk_ens.hpp"
+#include "vk_target.hpp"
 #include "vikshobha.h"
 
 #include <cmath>
@@ -1105,19 +1106,15 @@ int vk_gpe_set_kpsi(vk_gpe* h, const double* kpsi)
     return 0;
 }
 
-// whether a kernel of this device may write `bytes` at p as 16 byte values:
-// device memory of the current device, the whole range inside one allocation
-// (what a copy checks)
-static bool kernel_target(const void* p, size_t bytes)
+// whether a kernel on the handle's stream may write `bytes` at p
+static bool kernel_target(const vk_gpe* h, const void* p, size_t bytes)
 {
     hipPointerAttribute_t a;
     hipDeviceptr_t base = nullptr;
     size_t n = 0;
-    int dev = -1;
-    if ((uintptr_t)p % 16 == 0 && hipGetDevice(&dev) == hipSuccess && hipPointerGetAttributes(&a, p) == hipSuccess &&
-        a.type == hipMemoryTypeDevice && a.device == dev &&
+    if (hipPointerGetAttributes(&a, p) == hipSuccess && a.type == hipMemoryTypeDevice &&
         hipMemGetAddressRange(&base, &n, const_cast<void*>(p)) == hipSuccess)
-        return (const char*)p - (const char*)base + bytes <= n;
+        return vk::kernel_writable((uintptr_t)p, bytes, vk::Target{true, a.device, (uintptr_t)base, n}, h->dev);
     (void)hipGetLastError();
     return false;
 }
@@ -1133,7 +1130,7 @@ int vk_gpe_get_psi(vk_gpe* h, double* psi, double* kpsi)
         // an error of the steps queued so far: kernel_target's query leaves and
         // clears one of its own for host memory
         HIPCHK(hipGetLastError());
-        const bool direct = kernel_target(psi, bytes);
+        const bool direct = kernel_target(h, psi, bytes);
         if (!direct && (rc = need_hd(h))) return rc;
         if ((rc = ensure_any(h))) return rc;
         cplx* x = direct ? reinterpret_cast<cplx*>(psi) : h->Xs;
