@@ -128,7 +128,7 @@ struct vk_gpe {
     int4* pwin = nullptr;            // real-space path: windows and factor tables of the positions,
     double2 *ptx = nullptr, *pty = nullptr;
     double* Vx = nullptr;            // and the potential on the grid for ARGLE
-    int tab_valid = 0, vx_valid = 0; // they belong to the current positions
+    int vx_valid = 0;   // Vx belongs to the current positions
     int hstate = 0;   // 0: Hpsi stale, 1: Hpsi = IFFT_y K0 on all panels, 2: K0 dealiased, Hpsi on retained panels,
                       // 3: K0 dealiased, Hpsi on the retained panels of the single-field shape svar (layout CfgE<N, svar>)
     int kv_valid = 0;
@@ -498,11 +498,14 @@ vk::WTab wtab(const vk_gpe* h)
     return vk::WTab{h->p.V0, h->p.d, real_space_window(h->p.d), h->pwin, h->ptx, h->pty};
 }
 
-// windows and tables of the current positions
-void particle_tables(vk_gpe* h)
+// The particles have been set: windows and tables of their positions now, not
+// in the next step, so that they follow the positions for every later step,
+// also one that was recorded before (steps move them along themselves)
+void particles_moved(vk_gpe* h)
 {
-    hipLaunchKernelGGL(vk::k_wtab, dim3(h->p.np, 2), dim3(128), 0, h->stream, (const double*)h->pst, h->N, wtab(h));
-    h->tab_valid = 1;
+    h->kv_valid = h->vx_valid = 0;
+    if (h->rs_part)
+        hipLaunchKernelGGL(vk::k_wtab, dim3(h->p.np, 2), dim3(128), 0, h->stream, (const double*)h->pst, h->N, wtab(h));
 }
 
 // ARGLE never moves the particles: their potential on the grid, once per set
@@ -511,7 +514,6 @@ int particle_field(vk_gpe* h)
 {
     if (h->vx_valid) return 0;
     if (!h->Vx) HIPCHK(hipMalloc(&h->Vx, f2(h) * sizeof(double)));
-    if (!h->tab_valid) particle_tables(h);
     hipLaunchKernelGGL(vk::k_potfield, dim3(std::min((int)(f2(h) / 256), 4096)), dim3(256), 0, h->stream,
                        (const int4*)h->pwin, (const double2*)h->ptx, (const double2*)h->pty, h->p.np, h->N, h->Vx);
     h->vx_valid = 1;
@@ -609,7 +611,6 @@ int rk4_step(vk_gpe* h)
         const int parts = h->have_part && h->p.np > 0;
         const int rs = parts && h->rs_part;
         const int Kp = C::TC * h->geo.Pp;
-        if (rs && !h->tab_valid) particle_tables(h);
         h->vx_valid = 0;
         const vk::P3Part pa = p3part(h);
         vk::RKArgs a{};
@@ -1242,7 +1243,7 @@ int vk_gpe_particles_set(vk_gpe* h, const double* pos, const double* vel, const 
     if (fext) HIPCHK(hipMemcpyAsync(h->pst + 4 * np, fext, sizeof(double) * 2 * np, hipMemcpyDefault, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
     if (!h->have_part && (rc = particle_potential(h))) return rc;
-    h->kv_valid = h->tab_valid = h->vx_valid = 0;
+    particles_moved(h);
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipGetLastError());
     return 0;
@@ -1447,12 +1448,12 @@ int vk_gpe_set_obstacles(vk_gpe* h, int np, const double* pos, double V0, double
     h->p.d = d;
     h->rs_part = use_real_space(h->p);
     h->have_part = 0;
-    h->kv_valid = h->tab_valid = h->vx_valid = 0;
     if (np == 0) return 0;
     std::vector<double> st(30 * (size_t)np + 8, 0.0);
     std::copy(pos, pos + 2 * np, st.begin());
     HIPCHK(hipMemcpyAsync(h->pst, st.data(), sizeof(double) * st.size(), hipMemcpyHostToDevice, h->stream));
     if ((rc = particle_potential(h))) return rc;
+    particles_moved(h);
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipGetLastError());
     return 0;
@@ -1682,7 +1683,8 @@ int vk_gpe_autotune_rows(vk_gpe* h, int nsteps, int* choice, double* ms_out)
     release();
     if (rc) return rc;
     h->hstate = 2;
-    h->kv_valid = h->tab_valid = h->vx_valid = 0;
+    h->kv_valid = h->vx_valid = 0;
+    if (h->have_part && h->p.np > 0) particles_moved(h);
     if (choice) { choice[0] = b1; choice[1] = b3; }
     return 0;
 }
