@@ -166,6 +166,17 @@ namespace {
 
 size_t f2(const vk_gpe* h) { return (size_t)h->N * h->N; }
 
+// A field made on first use, zero: cleared by a kernel on the stream of the
+// kernels that follow, which is non-blocking (a clear on the default stream
+// could land after them)
+int make_field(vk_gpe* h, cplx** p, hipStream_t st)
+{
+    if (*p) return 0;
+    HIPCHK(hipMalloc(p, f2(h) * sizeof(cplx)));
+    hipLaunchKernelGGL(vk::k_zero, dim3(1024), dim3(256), 0, st, *p, f2(h));
+    return 0;
+}
+
 template <int N> using CfgN = vk::CfgS<N>;
 // The same panel layout with one row per row-pass workgroup (256 threads)
 // instead of TR rows: more, smaller workgroups per CU at the cost of half
@@ -756,13 +767,11 @@ int argle_step(vk_gpe* h, int want_res, const double* noise = nullptr)
 
 // ---- diagnostics ---------------------------------------------------------------
 
-int diag_setup(vk_gpe* h)
+int diag_setup(vk_gpe* h, hipStream_t st)
 {
     if (h->diag_ready) return 0;
-    if (!h->Hd) {
-        HIPCHK(hipMalloc(&h->Hd, f2(h) * sizeof(cplx)));
-        HIPCHK(hipMemset(h->Hd, 0, f2(h) * sizeof(cplx)));
-    }
+    int rc = make_field(h, &h->Hd, st);
+    if (rc) return rc;
     h->diag_ready = 1;
     return 0;
 }
@@ -790,7 +799,7 @@ vk::DiagArgs diag_args(const vk_gpe* h, int has_v)
 // diagnostics in the particle state
 int diag_launch(vk_gpe* h, double* out)
 {
-    int rc = diag_setup(h);
+    int rc = diag_setup(h, h->stream);
     if (rc) return rc;
     if ((rc = ensure_any(h))) return rc;
     const double sc = scale_of(h);
@@ -1065,14 +1074,7 @@ void vk_gpe_destroy(vk_gpe* h)
 static int sgle_sync_omega(vk_gpe* h);
 static int ensure_hdy(vk_gpe* h);
 
-static int need_hd(vk_gpe* h)
-{
-    if (!h->Hd) {
-        HIPCHK(hipMalloc(&h->Hd, f2(h) * sizeof(cplx)));
-        HIPCHK(hipMemset(h->Hd, 0, f2(h) * sizeof(cplx)));
-    }
-    return 0;
-}
+static int need_hd(vk_gpe* h) { return make_field(h, &h->Hd, h->stream); }
 
 static int set_from_xs(vk_gpe* h, int flags)
 {
@@ -1273,14 +1275,7 @@ int vk_gpe_set_advection(vk_gpe* h, int taylor_green, double vnx, double vny)
     return 0;
 }
 
-static int ensure_hdy(vk_gpe* h)
-{
-    if (!h->Hdy) {
-        HIPCHK(hipMalloc(&h->Hdy, f2(h) * sizeof(cplx)));
-        HIPCHK(hipMemset(h->Hdy, 0, f2(h) * sizeof(cplx)));
-    }
-    return 0;
-}
+static int ensure_hdy(vk_gpe* h) { return make_field(h, &h->Hdy, h->stream); }
 
 static int ensure_field_bufs(vk_gpe* h)
 {
@@ -2171,7 +2166,7 @@ int ens_check_barrier(vk_ens* e)
     int err = 0;
     HIPCHK(hipMemcpy(&err, e->derr, sizeof(int), hipMemcpyDeviceToHost));
     if (!err) return 0;
-    HIPCHK(hipMemset(e->derr, 0, sizeof(int)));
+    hipLaunchKernelGGL(vk::k_zero_u32, dim3(1), dim3(64), 0, e->stream, reinterpret_cast<unsigned*>(e->derr), 1);
     return fail(VK_ERR_STATE, "ensemble mode 3: a grid barrier timed out (workgroups not co-resident); state invalid");
 }
 
@@ -2368,7 +2363,7 @@ int vk_ens_diagnostics_all(vk_ens* e, double* scal, double* spec)
         e->nstage = need;
     }
     for (auto h : e->h) {
-        int rc = diag_setup(h);
+        int rc = diag_setup(h, e->stream);
         if (rc) return rc;
     }
     // groups of one size and one Hpsi state, batched launches on the
@@ -2570,13 +2565,13 @@ int vk_ens_autotune_shapes(vk_ens* e, int nsteps, int* vars_out, double* ms_out)
     for (auto h : e->h) {
         cplx* p = nullptr;
         HIPCHK(hipMalloc(&p, f2(h) * sizeof(cplx)));
-        HIPCHK(hipMemcpy(p, h->K0, f2(h) * sizeof(cplx), hipMemcpyDeviceToDevice));
+        HIPCHK(hipMemcpyAsync(p, h->K0, f2(h) * sizeof(cplx), hipMemcpyDeviceToDevice, e->stream));
         save.push_back(p);
     }
     auto restore = [&]() -> int {
         for (size_t i = 0; i < e->h.size(); ++i) {
             vk_gpe* h = e->h[i];
-            HIPCHK(hipMemcpy(h->K0, save[i], f2(h) * sizeof(cplx), hipMemcpyDeviceToDevice));
+            HIPCHK(hipMemcpyAsync(h->K0, save[i], f2(h) * sizeof(cplx), hipMemcpyDeviceToDevice, e->stream));
             h->hstate = 0;
         }
         e->synced = 0;

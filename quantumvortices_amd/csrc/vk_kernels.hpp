@@ -255,6 +255,12 @@ __global__ void __launch_bounds__(C::ROWT) VK_OCC k_row_inv(const cplx* __restri
     row_inv_body<C>(blockIdx.x, gridDim.x, H, X, tw, g, pload, op, scale);
 }
 
+// zero a field
+__global__ void k_zero(cplx* __restrict__ K, size_t n)
+{
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) K[i] = czero();
+}
+
 // zero the dealiased modes of a k-space field (all N^2 entries)
 __global__ void k_dealias(cplx* __restrict__ K, int N)
 {

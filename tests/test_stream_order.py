@@ -1,7 +1,8 @@
-"""Copies into memory that the caller names, read off the HIP sources: the
-library's streams are non-blocking, and a plain hipMemcpy whose destination
-turns out to be device memory neither waits nor is ordered against them, so the
-data of the call may arrive after a later call has rewritten its source."""
+"""Copies and clears of device memory, read off the HIP sources: the library's
+streams are non-blocking, and a plain hipMemcpy between device buffers (or into
+memory that the caller names, which may be one) or a plain hipMemset neither
+waits nor is ordered against them, so its data may arrive after later kernels
+have run."""
 import glob
 import os
 import re
@@ -27,4 +28,27 @@ def calls(name, text):
 @pytest.mark.parametrize("path", SOURCES, ids=os.path.basename)
 def test_copies_to_callers_are_on_a_stream(path):
     bad = [a for a in calls("hipMemcpy", open(path).read()) if "hipMemcpyDefault" in a]
+    assert not bad, bad
+
+
+@pytest.mark.parametrize("path", SOURCES, ids=os.path.basename)
+def test_device_copies_are_on_a_stream(path):
+    bad = [a for a in calls("hipMemcpy", open(path).read()) if "hipMemcpyDeviceToDevice" in a]
+    assert not bad, bad
+
+
+# where a device-wide wait or a blocking upload on the default stream follows
+# before anything else can run
+CREATES = {"vk_gpe_create", "vk_ens_create", "fno_alloc", "vk_pattern_bandwidth"}
+
+
+@pytest.mark.parametrize("path", SOURCES, ids=os.path.basename)
+def test_clears_are_on_a_stream(path):
+    inside, bad = "", []
+    for line in open(path):
+        m = re.match(r"^[a-z][\w:<>*& \"]*?\b(\w+)\(.*", line)
+        if m and not line.rstrip().endswith(";"):
+            inside = m.group(1)
+        if re.search(r"\bhipMemset(D\d+)?\(", line.split("//")[0]) and inside not in CREATES:
+            bad.append((inside, line.strip()))
     assert not bad, bad
