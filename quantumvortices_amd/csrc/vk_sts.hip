@@ -59,7 +59,9 @@ __global__ void k_sts_gather(const cplx* __restrict__ K, const int* __restrict__
 // One workgroup: TC modes, each transformed along time (Nt = C::N points,
 // contiguous per mode).  P[m][w] = stsnorm |sum_n h_n X[m][n] e^{-2 pi i n w/Nt}|^2
 // with the window h from a table.  Blocks past the last mode return before
-// the transform's barriers (whole workgroups only).
+// the transform's barriers (whole workgroups only).  128^2 x 2048 snapshots:
+// 281 MB moved in 57 us, 4.9 TB/s, a large copy's rate, so the transform takes
+// the form that adds least to it.
 template <class C, int G>
 __global__ void __launch_bounds__(G * C::T) k_sts_time(const cplx* __restrict__ X, int nm, double* __restrict__ P,
                                                       const cplx* __restrict__ tw, const double* __restrict__ hann,
@@ -82,7 +84,7 @@ __global__ void __launch_bounds__(G * C::T) k_sts_time(const cplx* __restrict__ 
         const cplx x = live ? xr[n] : vk::mk(0.0, 0.0);
         v[s] = vk::mk(h * x.x, h * x.y);
     }
-    vk::fft_fwd<Nt, S, C::SPLIT>(v, lg, t, tw);
+    vk::fft_fwd_products<Nt, S, C::SPLIT>(v, lg, t, tw);
     if (live) {
         double* pr = P + (size_t)m * Nt;
 #pragma unroll
@@ -95,7 +97,9 @@ __global__ void __launch_bounds__(G * C::T) k_sts_time(const cplx* __restrict__ 
 // order and the BW partial sums are added in wave order (a fixed order:
 // the result does not depend on scheduling).
 // Eight waves: 512^2 x 256 39 us against 47 with four, 256^2 x 512 19 and 21.5,
-// 128^2 x 64 7.8 and 10; 128^2 x 2048 18 either way (at HBM's rate).
+// 128^2 x 64 7.8 and 10; 128^2 x 2048 18 either way launched over and over (at
+// HBM's rate), 15.5 and 16.4 right behind the time transforms, whose output is
+// then partly still in the last-level cache.
 constexpr int BW = 8;
 __global__ void __launch_bounds__(64 * BW) k_sts_bin(const double* __restrict__ P, const int* __restrict__ off,
                                                    int nsh, int Nt, double* __restrict__ spec)
