@@ -195,13 +195,20 @@ __host__ __device__ constexpr int radix_at(int N, int S, int st)
 // A stage with twiddles: X[k] = sum_r (w^r x[r]) e^{-2 pi i r k/R}, by halving
 // in time.  Level M (2, 4, .., R) joins halves e, d with o[k] = e[k] + f d[k],
 // o[k + M/2] = e[k] - f d[k], f = w^{R/M} e^{-2 pi i k/M}; the second quarter's
-// factors are -i times the first's.  Each join is six fused operations
-// (e + f d in four, the other as 2 e - it in two), 12 per point and radix-16
-// stage against 16 for twiddle products followed by an untwiddled butterfly.
-// Few-wave passes pay every operation in latency: a step at 512^2 120.4 to
-// 113.1 us, at 1024^2 181.4 to 169.2, at 2048^2 550 to 519; at 4096^2 HBM and
-// LDS bound it (2106 to 2100).  Rounding: a field after 5 to 50 steps is within
-// 7.8e-16 of one computed with longer sums, 7.5e-16 before.
+// factors are -i times the first's.  A join is six fused operations (e + f d in
+// four, the other as 2 e - it in two), but eight for k = 0 (both in four): there
+// a field's mean meets itself, and 2 e - (e + f d) would turn the rounding of the
+// large sum into the error of the small difference beside it.  14 operations per
+// point and radix-16 stage, against 16 for twiddle products followed by an
+// untwiddled butterfly (TwProd).  Few-wave passes pay every operation in latency:
+// a step (its share of a psi read included) with products and then so at 512^2
+// 131 and 117 us, at 1024^2 202 and 175 (115 and 171 with six operations for k = 0
+// too).  From 2048^2 on the passes keep the products: HBM bounds them, and the
+// joins' k = 0 needs registers that P3 and P4 do not have (4096^2 2.03 ms a step,
+// with joins 2.33, or 2.05 with six operations; 2048^2 552, 668 and 523 us).
+// Rounding, 1024 points against 80-bit sums: white input 2.1e-16 of its norm
+// (products 2.2, six operations throughout 2.2); near-constant input, the other
+// bins' error over the mean's bin 1.7e-16 (1.7 and 2.2).
 // The factors, R/2 table values: slot 0 for M = 2, 1 for M = 4, 2 + k for
 // M = 8, 4 + k for M = 16, each w_N^{(R/M) base + k N/M} with w = w_N^base.
 constexpr int tw_per(int R) { return R / 2; }
@@ -227,7 +234,11 @@ template <int R, int M = 2, class F> __device__ __forceinline__ void dit(cplx (&
             const cplx t = mk(__builtin_fma(-u.y, b.y, __builtin_fma(u.x, b.x, e.x)),
                               __builtin_fma(u.y, b.x, __builtin_fma(u.x, b.y, e.y)));
             o[off * M + k] = t;
-            o[off * M + k + M / 2] = mk(__builtin_fma(2.0, e.x, -t.x), __builtin_fma(2.0, e.y, -t.y));
+            if (k == 0)
+                o[off * M + M / 2] = mk(__builtin_fma(u.y, b.y, __builtin_fma(-u.x, b.x, e.x)),
+                                        __builtin_fma(-u.y, b.x, __builtin_fma(-u.x, b.y, e.y)));
+            else
+                o[off * M + k + M / 2] = mk(__builtin_fma(2.0, e.x, -t.x), __builtin_fma(2.0, e.y, -t.y));
         }
 #pragma unroll
     for (int r = 0; r < R; ++r) x[r] = o[r];
@@ -237,9 +248,7 @@ template <int R, int M = 2, class F> __device__ __forceinline__ void dit(cplx (&
 // Twiddles read from the table where they are used (few registers: several
 // workgroups per CU hide the loads).  E: a stage's values all loaded before
 // its first level, so that no level waits for its own; where the registers
-// allow it.  At 4096^2: P1 138.5 to 137.2 us, P2 70.3 to 67.8, P3 with particles
-// 150 to 146, a step with them 2229 to 2196; P3 without particles is slower so
-// (147 to 178).
+// allow it (five steps of 384 ensemble members 29.3 to 28.9 ms).
 template <bool E> struct TwMem {
     const cplx* tw;
     static constexpr bool EAGER = E, PRODUCTS = false;
@@ -249,11 +258,11 @@ template <bool E> struct TwMem {
     }
 };
 
-// Twiddle products followed by an untwiddled butterfly, for a transform that
-// memory bounds and that runs once (the spectra's over time): w^r for r = 4a + b
-// from table values w^1..w^3 and w^4a (one product at most per factor), 16
-// operations per point and radix-16 stage.  2048 snapshots of 128^2 54.7 us,
-// with joins 55.2 to 55.4; 256 of 512^2 111.8 against 115.6.
+// Twiddle products followed by an untwiddled butterfly, for transforms that
+// memory bounds (the 2D passes from 2048^2 on, the spectra's over time): w^r for
+// r = 4a + b from table values w^1..w^3 and w^4a (one product at most per
+// factor).  Spectra of 2048 snapshots of 128^2 54.7 us, with joins 55.2 to 55.4;
+// of 256 snapshots of 512^2 111.8 against 115.6.
 struct TwProd {
     const cplx* tw;
     static constexpr bool EAGER = false, PRODUCTS = true;
@@ -428,10 +437,11 @@ __device__ __forceinline__ void fft_fwd(cplx (&v)[S], double* lds, int t, const 
     const cplx* twb = tw;
     asm volatile("" : "+s"(twb));
     // Likewise the index arithmetic, where registers bind: P4 at 4096^2 spilled 16
-    // registers with it shared by its two transforms, 178 us against 165; at
-    // 2048^2 54 against 50.  Smaller ones have registers to keep it.
+    // registers with it shared by its two transforms, 178 us.  Smaller ones have
+    // registers to keep it.
     if constexpr (N >= 2048) asm volatile("" : "+v"(t));
-    Stage<N, S, 0, 1, SPLIT>::run(v, lds, SPLIT ? lds : lds + Lds<N>::words, t, TwMem<EAGER>{twb});
+    using W = std::conditional_t<(N >= 2048), TwProd, TwMem<EAGER>>;
+    Stage<N, S, 0, 1, SPLIT>::run(v, lds, SPLIT ? lds : lds + Lds<N>::words, t, W{twb});
 }
 
 // the same with twiddle products; no opaque index from 2048 points on either

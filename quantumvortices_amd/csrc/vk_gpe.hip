@@ -963,9 +963,9 @@ int vk_gpe_create(vk_gpe** out, const vk_gpe_params* p)
         const char* t3 = std::getenv("VK_P3_TR1");
         // Measured defaults (4-column panels: 64-byte row pieces), ms per step
         // with 32 particles / without: at 2048^2 one row per workgroup in P1
-        // and P3, 0.552 / 0.507 (four rows in P3 0.580 / 0.527, in both 0.636 /
-        // 0.590); at 4096^2 one row in P1 and two in P3, 2.056 / 2.013 (one in
-        // both 2.092 / 2.050, two in both 2.111 / 2.068).
+        // and P3, 0.574 / 0.530 (four rows in P3 0.586 / 0.541, in both 0.637 /
+        // 0.595); at 4096^2 one row in P1 and two in P3, 2.027 / 2.006 (one in
+        // both 2.091 / 2.035, two in both 2.078 / 2.049).
         // VK_P1_TR1 / VK_P3_TR1 = 0 or 1 override; vk_gpe_autotune_rows
         // times every pair on the device at hand.
         h->tr1_p1 = t1 ? t1[0] == '1' : (N == 4096 || N == 2048);
