@@ -168,11 +168,10 @@ __device__ __forceinline__ int ksg(int i, int N) { return i < N / 2 ? i : i - N;
 // 1/9 of an integer, so the REAL comparison equals 9*ksqr >= N^2.
 __device__ __forceinline__ bool kmasked(int kx, int ky, int N) { return 9 * (kx * kx + ky * ky) >= N * N; }
 
-// panel pmode: 0 all, 1 retained both signs, 2 retained kx >= 0 only
+// panel pmode: 0 all, 1 retained (both signs of kx)
 __device__ __forceinline__ bool panel_stored(int p, int NP, const Geo& g, int pmode)
 {
     if (pmode == 0) return true;
-    if (pmode == 2) return p < g.Pp;
     return p < g.Pp || p >= NP - g.Pn;
 }
 __device__ __forceinline__ int panel_of_block(int b, int NP, const Geo& g, int pmode)

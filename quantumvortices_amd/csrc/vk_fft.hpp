@@ -201,11 +201,11 @@ __host__ __device__ constexpr int radix_at(int N, int S, int st)
 // large sum into the error of the small difference beside it.  14 operations per
 // point and radix-16 stage, against 16 for twiddle products followed by an
 // untwiddled butterfly (TwProd).  Few-wave passes pay every operation in latency:
-// a step (its share of a psi read included) with products and then so at 512^2
-// 131 and 117 us, at 1024^2 202 and 175 (115 and 171 with six operations for k = 0
-// too).  From 2048^2 on the passes keep the products: HBM bounds them, and the
-// joins' k = 0 needs registers that P3 and P4 do not have (4096^2 2.03 ms a step,
-// with joins 2.33, or 2.05 with six operations; 2048^2 552, 668 and 523 us).
+// a step with products 120 us at 512^2 and 181 at 1024^2, with six operations for
+// every join 113 and 169, 2% more with eight for k = 0.  From 2048^2 on the passes
+// keep the products: HBM bounds them, and the joins' k = 0 needs registers that P3
+// and P4 do not have (4096^2 2.01 ms a step, with joins 2.33, or 2.05 with six
+// operations; 2048^2 517, 668 and 523 us).
 // Rounding, 1024 points against 80-bit sums: white input 2.1e-16 of its norm
 // (products 2.2, six operations throughout 2.2); near-constant input, the other
 // bins' error over the mean's bin 1.7e-16 (1.7 and 2.2).

@@ -359,23 +359,20 @@ void p1p_launch(vk_gpe* h, double sc)
 
 int ncols(const vk_gpe* h, int pmode)
 {
-    if (pmode == 0) return h->NP;
-    if (pmode == 2) return h->geo.Pp;
-    return h->geo.Pp + h->geo.Pn;
+    return pmode == 0 ? h->NP : h->geo.Pp + h->geo.Pn;
 }
 
 double scale_of(const vk_gpe* h) { return 1.0 / ((double)h->N * (double)h->N); }
 
 // ---- generic 2D transforms ------------------------------------------------
 
-int fwd2d(vk_gpe* h, const cplx* X, cplx* Hs, cplx* K, int op_row, int op_col)
+int fwd2d(vk_gpe* h, const cplx* X, cplx* Hs, cplx* K, int op_col)
 {
     return dispatch(h->N, [&](auto n) {
         using C = CfgN<decltype(n)::value>;
-        row_launch<C>(h, PK_OTHER, vk::k_row_fwd<C>, X, Hs, (const cplx*)h->tw, h->geo, 0, op_row);
+        row_launch<C>(h, PK_OTHER, vk::k_row_fwd<C>, X, Hs, (const cplx*)h->tw);
         constexpr int G = p4_cols<C>();
-        colg_launch<C, G>(h, PK_OTHER, h->NP, vk::k_col_fwd<C, G>, (const cplx*)Hs, K, (const cplx*)h->tw, h->geo, 0,
-                          op_col);
+        colg_launch<C, G>(h, PK_OTHER, h->NP, vk::k_col_fwd<C, G>, (const cplx*)Hs, K, (const cplx*)h->tw, op_col);
         return 0;
     });
 }
@@ -391,11 +388,11 @@ int col_inv(vk_gpe* h, const cplx* K, cplx* Hs, int pmode, int op)
     });
 }
 
-int row_inv(vk_gpe* h, const cplx* Hs, cplx* X, int pload, int op, double scale)
+int row_inv(vk_gpe* h, const cplx* Hs, cplx* X, int pload, double scale)
 {
     return dispatch(h->N, [&](auto n) {
         using C = CfgN<decltype(n)::value>;
-        row_launch<C>(h, PK_OTHER, vk::k_row_inv<C>, Hs, X, (const cplx*)h->tw, h->geo, pload, op, scale);
+        row_launch<C>(h, PK_OTHER, vk::k_row_inv<C>, Hs, X, (const cplx*)h->tw, h->geo, pload, scale);
         return 0;
     });
 }
@@ -550,7 +547,7 @@ int particle_kv(vk_gpe* h, int nrows)
     hipLaunchKernelGGL(vk::k_ptab, dim3((np * h->N + 255) / 256), dim3(256), 0, h->stream, (const double*)h->pst,
                        h->EX, h->EY, np, h->N);
     hipLaunchKernelGGL(vk::k_kv, dim3(nrows), dim3(256), (size_t)np * sizeof(cplx), h->stream,
-                       (const cplx*)h->Vhat, (const cplx*)h->EX, (const cplx*)h->EY, h->KV, np, h->N, nrows);
+                       (const cplx*)h->Vhat, (const cplx*)h->EX, (const cplx*)h->EY, h->KV, np, h->N);
     ev_end(h, PK_PART);
     return 0;
 }
@@ -963,9 +960,9 @@ int vk_gpe_create(vk_gpe** out, const vk_gpe_params* p)
         const char* t3 = std::getenv("VK_P3_TR1");
         // Measured defaults (4-column panels: 64-byte row pieces), ms per step
         // with 32 particles / without: at 2048^2 one row per workgroup in P1
-        // and P3, 0.574 / 0.530 (four rows in P3 0.586 / 0.541, in both 0.637 /
-        // 0.595); at 4096^2 one row in P1 and two in P3, 2.027 / 2.006 (one in
-        // both 2.091 / 2.035, two in both 2.078 / 2.049).
+        // and P3, 0.551 / 0.513 (four rows in P3 0.575 / 0.533, in both 0.637 /
+        // 0.588); at 4096^2 one row in P1 and two in P3, 2.019 / 1.997 (one in
+        // both 2.087 / 2.038, two in both 2.064 / 2.026).
         // VK_P1_TR1 / VK_P3_TR1 = 0 or 1 override; vk_gpe_autotune_rows
         // times every pair on the device at hand.
         h->tr1_p1 = t1 ? t1[0] == '1' : (N == 4096 || N == 2048);
@@ -1078,7 +1075,7 @@ static int need_hd(vk_gpe* h) { return make_field(h, &h->Hd, h->stream); }
 
 static int set_from_xs(vk_gpe* h, int flags)
 {
-    int rc = fwd2d(h, h->Xs, h->Hd, h->K0, 0, 0);
+    int rc = fwd2d(h, h->Xs, h->Hd, h->K0, 0);
     if (rc) return rc;
     h->hstate = 0;
     if (flags & VK_SYNC_DEALIAS) {
@@ -1137,7 +1134,7 @@ int vk_gpe_get_psi(vk_gpe* h, double* psi, double* kpsi)
         if (!direct && (rc = need_hd(h))) return rc;
         if ((rc = ensure_any(h))) return rc;
         cplx* x = direct ? reinterpret_cast<cplx*>(psi) : h->Xs;
-        if ((rc = row_inv(h, h->Hpsi, x, h->hstate == 2 ? 1 : 0, 0, scale_of(h)))) return rc;
+        if ((rc = row_inv(h, h->Hpsi, x, h->hstate == 2 ? 1 : 0, scale_of(h)))) return rc;
         HIPCHK(hipGetLastError());
         if (!direct) HIPCHK(hipMemcpyAsync(psi, x, bytes, hipMemcpyDefault, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
@@ -1224,7 +1221,7 @@ static int particle_potential(vk_gpe* h)
     const double pi = 4.0 * std::atan(1.0);
     const double L = 2.0 * pi, dx = L / h->N, c1 = 2 * pi / (2.0 * L);
     hipLaunchKernelGGL(vk::k_pot_x, dim3(1024), dim3(256), 0, h->stream, h->Xs, h->N, dx, c1, h->p.V0, h->p.d);
-    int rc = fwd2d(h, h->Xs, h->Hd, h->Vhat, 0, 1);
+    int rc = fwd2d(h, h->Xs, h->Hd, h->Vhat, 1);
     if (rc) return rc;
     h->have_part = 1;
     return 0;
@@ -1475,14 +1472,14 @@ int vk_fft2d(vk_gpe* h, int dir, const double* in, double* out)
     const size_t fb = f2(h) * sizeof(cplx);
     if (dir < 0) {
         HIPCHK(hipMemcpyAsync(h->Xs, in, fb, hipMemcpyHostToDevice, h->stream));
-        if ((rc = fwd2d(h, h->Xs, h->Hd, h->Kd0, 0, 0))) return rc;
+        if ((rc = fwd2d(h, h->Xs, h->Hd, h->Kd0, 0))) return rc;
         HIPCHK(hipStreamSynchronize(h->stream));
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpy(out, h->Kd0, fb, hipMemcpyDeviceToHost));
     } else {
         HIPCHK(hipMemcpy(h->Kd0, in, fb, hipMemcpyHostToDevice));
         if ((rc = col_inv(h, h->Kd0, h->Hd, 0, 0))) return rc;
-        if ((rc = row_inv(h, h->Hd, h->Xs, 0, 0, scale_of(h)))) return rc;
+        if ((rc = row_inv(h, h->Hd, h->Xs, 0, scale_of(h)))) return rc;
         HIPCHK(hipStreamSynchronize(h->stream));
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpy(out, h->Xs, fb, hipMemcpyDeviceToHost));
@@ -1513,8 +1510,8 @@ int vk_fft2d_noalloc(vk_gpe* h, int dir, const double* in, double* out)
     const cplx* ci = reinterpret_cast<const cplx*>(in);
     cplx* co = reinterpret_cast<cplx*>(out);
     int rc;
-    if (dir < 0) rc = fwd2d(h, ci, H, co, 0, 0);
-    else if (!(rc = col_inv(h, ci, H, 0, 0))) rc = row_inv(h, H, co, 0, 0, scale_of(h));
+    if (dir < 0) rc = fwd2d(h, ci, H, co, 0);
+    else if (!(rc = col_inv(h, ci, H, 0, 0))) rc = row_inv(h, H, co, 0, scale_of(h));
     if (rc) return rc;
     HIPCHK(hipGetLastError());
     return 0;
@@ -1590,7 +1587,7 @@ int vk_gpe_pass_times(vk_gpe* h, int nsteps, double* ms_out, int nkinds)
 int vk_gpe_set_row_variants(vk_gpe* h, int p1, int p3)
 {
     if (!h || p1 < 0 || p1 > 2 || p3 < 0 || p3 > 1) return fail(VK_ERR_ARG, "set_row_variants: bad arguments");
-    if (h->N < 2048) return fail(VK_ERR_UNSUPPORTED, "set_row_variants: the row-pass variants exist for the psi-row path only");
+    if (h->N < 2048) return fail(VK_ERR_UNSUPPORTED, "set_row_variants: the row-pass variants exist for N >= 2048 only");
     if (p1 == 2 && !p1_prefetch_fits(h))
         return fail(VK_ERR_UNSUPPORTED, "set_row_variants: the prefetching P1 does not fit this size or device");
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -1611,7 +1608,7 @@ int vk_gpe_get_row_variants(vk_gpe* h, int* p1, int* p3)
 int vk_gpe_autotune_rows(vk_gpe* h, int nsteps, int* choice, double* ms_out)
 {
     if (!h || nsteps <= 0) return fail(VK_ERR_ARG, "autotune_rows: bad arguments");
-    if (h->N < 2048) return fail(VK_ERR_UNSUPPORTED, "autotune_rows: the row-pass variants exist for the psi-row path only");
+    if (h->N < 2048) return fail(VK_ERR_UNSUPPORTED, "autotune_rows: the row-pass variants exist for N >= 2048 only");
     int rc = ensure_rk4(h);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(h->stream));

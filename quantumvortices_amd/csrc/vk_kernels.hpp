@@ -112,44 +112,35 @@ __device__ __forceinline__ cplx czero() { return mk(0.0, 0.0); }
 // Generic transform passes (set/get, diagnostics, conformance hook)
 // ----------------------------------------------------------------------------
 
-// x-space rows -> FFT along x -> H.  op 1: transform |X|^2 instead of X.
+// x-space rows -> FFT along x -> H, all panels.
 template <class C>
 __device__ __forceinline__ void row_fwd_body(int blk_, int nblk_, const cplx* __restrict__ X, cplx* __restrict__ H,
-                                             const cplx* __restrict__ tw, Geo g, int pstore, int op)
+                                             const cplx* __restrict__ tw)
 {
     VK_ROW_SETUP(C)
     const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
     const cplx* xr = X + (size_t)y * N;
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-        cplx a = xr[t + T * s];
-        v[s] = op == 1 ? mk(a.x * a.x + a.y * a.y, 0.0) : a;
-    }
+    for (int s = 0; s < S; ++s) v[s] = xr[t + T * s];
     fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-        const int pp = VK_PANEL(s);
-        if (panel_stored(pp, NP, g, pstore)) H[hoff<C>(pp, y, c)] = v[s];
-    }
+    for (int s = 0; s < S; ++s) H[hoff<C>(VK_PANEL(s), y, c)] = v[s];
 }
 
 template <class C>
 __global__ void __launch_bounds__(C::ROWT) VK_OCC k_row_fwd(const cplx* __restrict__ X, cplx* __restrict__ H,
-                                                     const cplx* __restrict__ tw, Geo g, int pstore, int op)
+                                                     const cplx* __restrict__ tw)
 {
-    row_fwd_body<C>(blockIdx.x, gridDim.x, X, H, tw, g, pstore, op);
+    row_fwd_body<C>(blockIdx.x, gridDim.x, X, H, tw);
 }
 
-// H column -> FFT along y -> K.  op 1: dealias.
-// panels a column pass over pmode covers (0 all, 1 retained, 2 kx >= 0)
-#define VK_NPAN(C, g, pmode) ((pmode) == 0 ? C::NP : ((pmode) == 2 ? (g).Pp : (g).Pp + (g).Pn))
-
+// H column -> FFT along y -> K, all panels.  op 1: dealias.
 template <class C, int G = C::TC>
 __device__ __forceinline__ void col_fwd_body(int b, const cplx* __restrict__ H, cplx* __restrict__ K,
-                                             const cplx* __restrict__ tw, Geo g, int pmode, int op)
+                                             const cplx* __restrict__ tw, int op)
 {
-    VK_COL_SETUP_G(C, G, b, panel_of_block(pb_, C::NP, g, pmode), VK_NPAN(C, g, pmode))
+    VK_COL_SETUP_G(C, G, b, pb_, C::NP)
     const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
 #pragma unroll
@@ -168,13 +159,16 @@ __device__ __forceinline__ void col_fwd_body(int b, const cplx* __restrict__ H, 
 
 template <class C, int G = C::TC>
 __global__ void __launch_bounds__(G * C::T) VK_OCC k_col_fwd(const cplx* __restrict__ H, cplx* __restrict__ K,
-                                                     const cplx* __restrict__ tw, Geo g, int pmode, int op)
+                                                     const cplx* __restrict__ tw, int op)
 {
-    col_fwd_body<C, G>(blockIdx.x, H, K, tw, g, pmode, op);
+    col_fwd_body<C, G>(blockIdx.x, H, K, tw, op);
 }
 
+// panels a column pass over pmode covers (0 all, 1 retained)
+#define VK_NPAN(C, g, pmode) ((pmode) == 0 ? C::NP : (g).Pp + (g).Pn)
+
 // K row -> op -> unnormalised inverse FFT along y -> H.
-// op 0: as is; 1: dealias; 2: times i*ky.
+// op 0: as is; 2: times i*ky.
 template <class C, int G = C::TC>
 __device__ __forceinline__ void col_inv_body(int b, const cplx* __restrict__ K, cplx* __restrict__ H,
                                              const cplx* __restrict__ tw, Geo g, int pmode, int op)
@@ -182,16 +176,15 @@ __device__ __forceinline__ void col_inv_body(int b, const cplx* __restrict__ K, 
     VK_COL_SETUP_G(C, G, b, panel_of_block(pb_, C::NP, g, pmode), VK_NPAN(C, g, pmode))
     const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
-    const int kxs = ksg(kx, N);
     const cplx* kr = K + (size_t)kx * N;
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-        const int ky = t + T * s;
-        const int kys = ksg(ky, N);
-        cplx a = kr[ky];
-        if (op == 1 && kmasked(kxs, kys, N)) a = czero();
-        if (op == 2) a = mk(-(double)kys * a.y, (double)kys * a.x);
-        v[s] = conjc(a);
+    for (int s = 0; s < S; ++s) v[s] = conjc(kr[t + T * s]);
+    if (op == 2) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const double kys = ksg(t + T * s, N);
+            v[s] = mk(kys * v[s].y, -kys * v[s].x);
+        }
     }
     fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
 #pragma unroll
@@ -205,42 +198,23 @@ __global__ void __launch_bounds__(G * C::T) VK_OCC k_col_inv(const cplx* __restr
     col_inv_body<C, G>(blockIdx.x, K, H, tw, g, pmode, op);
 }
 
-// H row -> op -> unnormalised inverse FFT along x -> times scale -> X.
-// pload 2: kx >= 0 panels stored, negative kx from Hermitian symmetry.
-// op 1: times i*kx before the transform.
+// H row (panels of mode pload) -> unnormalised inverse FFT along x -> times
+// scale -> X.
 template <class C>
 __device__ __forceinline__ void row_inv_body(int blk_, int nblk_, const cplx* __restrict__ H, cplx* __restrict__ X,
-                                             const cplx* __restrict__ tw, Geo g, int pload, int op, double scale)
+                                             const cplx* __restrict__ tw, Geo g, int pload, double scale)
 {
     VK_ROW_SETUP(C)
     const auto w_ = twiddles<C>(tw, t);
     cplx v[S];
-    const int Kp = TC * g.Pp;
     const brsrc rH = mkbuf(H, N);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-        const int kxi = t + T * s;
-        unsigned o;
-        if (pload == 2) {
-            const int km = kxi >= Kp ? N - kxi : kxi;
-            o = boff(hoff<C>(km / TC, y, km % TC), kxi < Kp || kxi > N - Kp);
-        } else {
-            const int pp = VK_PANEL(s);
-            o = boff(hoff<C>(pp, y, c), panel_stored(pp, NP, g, pload));
-        }
-        v[s] = bld(rH, o);
+        const int pp = VK_PANEL(s);
+        v[s] = bld(rH, boff(hoff<C>(pp, y, c), panel_stored(pp, NP, g, pload)));
     }
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-        const int kxi = t + T * s;
-        cplx a = v[s];
-        if (pload == 2 && kxi > N - Kp) a = conjc(a);
-        if (op == 1) {
-            const double kk = (double)ksg(kxi, N);
-            a = mk(-kk * a.y, kk * a.x);
-        }
-        v[s] = conjc(a);
-    }
+    for (int s = 0; s < S; ++s) v[s] = conjc(v[s]);
     fft_fwd<N, S, C::SPLIT>(v, lg, t, w_);
     cplx* xr = X + (size_t)y * N;
 #pragma unroll
@@ -249,10 +223,9 @@ __device__ __forceinline__ void row_inv_body(int blk_, int nblk_, const cplx* __
 
 template <class C>
 __global__ void __launch_bounds__(C::ROWT) VK_OCC k_row_inv(const cplx* __restrict__ H, cplx* __restrict__ X,
-                                                     const cplx* __restrict__ tw, Geo g, int pload, int op,
-                                                     double scale)
+                                                     const cplx* __restrict__ tw, Geo g, int pload, double scale)
 {
-    row_inv_body<C>(blockIdx.x, gridDim.x, H, X, tw, g, pload, op, scale);
+    row_inv_body<C>(blockIdx.x, gridDim.x, H, X, tw, g, pload, scale);
 }
 
 // zero a field
@@ -1597,7 +1570,7 @@ __global__ void k_ptab(const double* __restrict__ pos, cplx* __restrict__ EX, cp
 // KV(kx,ky) = Vhat(kx,ky) * sum_p EX_p(kx) EY_p(ky) on the unmasked modes of
 // rows kx in [0, nrows) (nrows = N: all rows)   (:334-349, separable)
 __global__ void k_kv(const cplx* __restrict__ Vhat, const cplx* __restrict__ EX, const cplx* __restrict__ EY,
-                     cplx* __restrict__ KV, int np, int N, int rows_pos)
+                     cplx* __restrict__ KV, int np, int N)
 {
     extern __shared__ double dsh[];
     cplx* ex = reinterpret_cast<cplx*>(dsh);
@@ -1605,7 +1578,6 @@ __global__ void k_kv(const cplx* __restrict__ Vhat, const cplx* __restrict__ EX,
     for (int pp = threadIdx.x; pp < np; pp += blockDim.x) ex[pp] = EX[(size_t)pp * N + kx];
     __syncthreads();
     const int kxs = ksg(kx, N);
-    (void)rows_pos;
     for (int ky = threadIdx.x; ky < N; ky += blockDim.x) {
         const int kys = ksg(ky, N);
         if (kmasked(kxs, kys, N)) continue;
