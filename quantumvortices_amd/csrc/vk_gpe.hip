@@ -112,9 +112,9 @@ struct vk_gpe {
     // caller-supplied advection velocity (replaces the Taylor-Green field)
     double *Ux = nullptr, *Uy = nullptr;
     int adv_field = 0;
-    // SGLE (GPE_SGLE): noise field (x-space, then k-space), the chemical
-    // potential on the device, norm partials, the draw counter of the
-    // generator
+    // SGLE (GPE_SGLE): the caller's normals (or the generator's, on request), the
+    // chemical potential before and after a step on the device, the row sums of
+    // |psi|^2, the draw counter of the generator
     int sgle = 0;
     double sg_beta = 0.0, sg_nuN = 0.0, sg_ktrunc = 0.0;
     unsigned long long sg_seed = 0, sg_draw = 0;
@@ -1240,7 +1240,6 @@ int vk_gpe_particles_set(vk_gpe* h, const double* pos, const double* vel, const 
     if (pos) HIPCHK(hipMemcpyAsync(h->pst, pos, sizeof(double) * 2 * np, hipMemcpyDefault, h->stream));
     if (vel) HIPCHK(hipMemcpyAsync(h->pst + 2 * np, vel, sizeof(double) * 2 * np, hipMemcpyDefault, h->stream));
     if (fext) HIPCHK(hipMemcpyAsync(h->pst + 4 * np, fext, sizeof(double) * 2 * np, hipMemcpyDefault, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
     if (!h->have_part && (rc = particle_potential(h))) return rc;
     particles_moved(h);
     HIPCHK(hipStreamSynchronize(h->stream));
