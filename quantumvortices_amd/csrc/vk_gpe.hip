@@ -691,7 +691,12 @@ int argle_step(vk_gpe* h, int want_res, const double* noise = nullptr)
         const double sc = scale_of(h);
         const int parts = h->have_part && h->p.np > 0;
         const int rs = parts && h->rs_part;
-        if (rs) {
+        // the obstacles' potential: from the grid up to 1024^2; from 2048^2 on from
+        // the windows, as RK4 (with 8 obstacles 4096^2 745 us a step from the grid,
+        // whose 134 MB P3 would read, and 702 so)
+        constexpr bool GRID = C::N < 2048;
+        constexpr int PMR = GRID ? 8 : 4;
+        if (GRID && rs) {
             int rc = particle_field(h);
             if (rc) return rc;
         }
@@ -730,11 +735,11 @@ int argle_step(vk_gpe* h, int want_res, const double* noise = nullptr)
                                  h->adv_field ? (const double*)h->Ux : nullptr,
                                  h->adv_field ? (const double*)h->Uy : nullptr};
             row_launch_x<C>(h, PK_P3, p3_extra(h),
-                            !parts ? vk::k_p3a<C, 0> : (rs ? vk::k_p3a<C, 8> : vk::k_p3a<C, 1>), (const cplx*)h->Hrho,
+                            !parts ? vk::k_p3a<C, 0> : (rs ? vk::k_p3a<C, PMR> : vk::k_p3a<C, 1>), (const cplx*)h->Hrho,
                             (const cplx*)h->HV, (const cplx*)h->Hpsi, (const cplx*)h->Xs, (const cplx*)h->Hdy, h->HN,
                             (const cplx*)h->tw, h->geo, -h->p.g * sc, -sc, -1.0, pa, aa);
         } else {
-            auto k3 = !parts ? vk::k_p3x<C, 0> : (rs ? vk::k_p3x<C, 8> : vk::k_p3x<C, 1>);
+            auto k3 = !parts ? vk::k_p3x<C, 0> : (rs ? vk::k_p3x<C, PMR> : vk::k_p3x<C, 1>);
             row_launch_x<C>(h, PK_P3, p3_extra(h), k3, (const cplx*)h->Hrho, (const cplx*)h->HV, (const cplx*)h->Xs,
                             h->HN, (const cplx*)h->tw, h->geo, 0, -h->p.g * sc, -sc, -1.0, pa);
         }
