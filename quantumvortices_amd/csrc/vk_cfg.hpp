@@ -50,13 +50,12 @@ template <> struct Cfg<2048> : CfgT<2048, 16, 4, 4, true> {};
 #ifndef VK4096_S
 #define VK4096_S 16
 #endif
-// 4-column panels: the row passes gather 64-byte row pieces with one row
-// per workgroup (P1 0.152 -> 0.139 ms, P3 0.186 -> 0.163 ms) and the column
-// passes take two of a panel's columns per workgroup (P4 0.151 -> 0.170
-// ms).  Per step, against 2-column panels on the same device: 2-3% faster
-// without particles, within 1% with them (+0.9% and -0.4% on two
-// devices).  The fields are bitwise the same: the layout moves data, the
-// arithmetic is unchanged.
+// 4-column panels: the row passes gather 64-byte row pieces (P1 with one row
+// per workgroup 134 us, P3 with two 138) and the column passes take two of a
+// panel's columns per workgroup (P4 162).  Against 2-column panels, when P1, P3
+// and P4 took 139, 163 and 170 us so and 152, 186 and 151 with them, a step was
+// 2-3% faster without particles and within 1% with them.  The fields are bitwise
+// the same: the layout moves data, the arithmetic is unchanged.
 #ifndef VK4096_TC
 #define VK4096_TC 4
 #endif

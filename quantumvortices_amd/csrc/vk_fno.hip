@@ -59,9 +59,10 @@ __host__ __device__ inline uint16_t f2bf(float f)
 
 // Phi(x) = (1 + erf(x/sqrt 2))/2 as exp2(t P(t))/2, t = |x|: log2 erfc(t/sqrt 2)
 // divided by t is smooth, so one polynomial (degree 9, weighted minimax fit
-// on [0, 6]) and one exp2 serve every x without a branch.  Absolute error
-// of Phi 3.5e-8 (half an FP32 ulp of 1 is 3e-8), relative error 5e-6 in the tail
-// to |x| = 5; P's leading coefficient is negative, so |x| -> inf gives 0 or 1.
+// on [0, 6]) and one exp2 serve every x without a branch.  In FP32, absolute
+// error of Phi 3.5e-8 for x < 0 and 6.5e-8 for x > 0, where the rounding of 1 - e
+// (half an FP32 ulp of 1, 3e-8) adds; relative error 5.6e-6 in the tail to x = -5.
+// P's leading coefficient is negative, so |x| -> inf gives 0 or 1.
 __device__ __forceinline__ float phi_cdf(float x)
 {
     const float t = fabsf(x);
@@ -76,7 +77,7 @@ __device__ __forceinline__ float phi_cdf(float x)
     p = fmaf(p, t, -0.45921661787979434f);
     p = fmaf(p, t, -1.1511046520970696f);
     const float e = 0.5f * __builtin_amdgcn_exp2f(p * t);
-    return x >= 0.f ? 1.0f - e : (x < 0.f ? e : 0.5f + x);   // x = 0 and NaN take the last form
+    return x >= 0.f ? 1.0f - e : (x < 0.f ? e : 0.5f + x);   // NaN takes the last form
 }
 __device__ __forceinline__ float gelu(float x) { return x * phi_cdf(x); }
 // gelu(x) and its derivative Phi(x) + x phi(x)

@@ -552,7 +552,7 @@ __device__ __forceinline__ void block_sum(double (&x)[NV], double* sh)
 // tabulated over the window by k_wtab whenever the positions change.  P3 with
 // the sines and exponentials in its point loop took 17.5 us at 512^2 with 8
 // particles (229 VGPRs and 162 us at 4096^2 with 32); from the tables 10.9 us
-// (128 VGPRs, 137 us: the time without particles).
+// (at most 128 VGPRs, 138 us at 4096^2 with 32 and without any).
 struct P3Part {
     const int4* win;     // per particle: first column and count of its window, first row and count
     const double2* tx;   // [particle][k < N]: ex, -ex X dX/dx / d^2, ex = exp(-X^2 / (2 d^2))
@@ -913,7 +913,7 @@ __global__ void __launch_bounds__(G * C::T) VK_P4OCC(C) k_p4(const cplx* __restr
 struct ArgleArgs {
     double alpha, omega, dt;
     int want_res;
-    // SGLE (src/gpe.f90:200-217): with Kn set, sqrt(dt) Kn (dealiased) is
+    // SGLE (src/gpe.f90:200-217): sqrt(dt) times the transform of Hn (dealiased) is
     // added to the numerator, omega is this step's chemical potential and,
     // for ktrunc2 > 0, modes with k^2 > ktrunc2 are zeroed
     const cplx* Hn;        // noise rows transformed along x, retained panels
